@@ -484,7 +484,7 @@ __global__ void k_synchrotron(const double* Ne, const double* Th, const double* 
   const long p = (long)blockIdx.x * blockDim.x + threadIdx.x;
   if (p >= n) return;
   double jj, aa;
-  synchrotron<double>(Ne[p], Th[p], B[p], pitch[p], nu[p], invariant != 0, rescale, jj, aa);
+  synchrotron(Ne[p], Th[p], B[p], pitch[p], nu[p], invariant != 0, rescale, jj, aa);
   j[p] = jj;
   al[p] = aa;
 }

@@ -160,10 +160,10 @@ __global__ void __launch_bounds__(256) k_sample_scalars(SnapView sv, const doubl
   double q[8];
 #pragma unroll
   for (int k = 0; k < 8; ++k) q[k] = S[8 * p + k];
-  double P[8], sc[5];
+  double P[8];
   trilinear<double>(sv, q[1], q[2], q[3], P);
-  fluid_scalars<double>(P, q[1], q[2], q[3], q[4], q[5], q[6], q[7], a, fbc, sc);
-  sc[2] = ::acos(sc[2]);  // pitch angle from its cosine
+  const Fluid64 F = fluid64(P, q[1], q[2], q[3], q[4], q[5], q[6], q[7], a, fbc);
+  const double sc[5] = {P[0], P[1], ::acos(F.cosp), F.kdotu, F.W == 0.0 ? 0.0 : F.sW * F.iu0};
 #pragma unroll
   for (int c = 0; c < 5; ++c) out[c * n + p] = sc[c];
 }
