@@ -5,7 +5,8 @@
 // `steps` times; the shader clock (s_memtime) and the 100 MHz real-time
 // counter around the loop give cycles and nanoseconds per repetition.  The
 // pieces are the stages of mk_render's per-ray work in each precision:
-//   0 / 1  RK4 step, FP64 / mixed (rk4_step<double> / rk4_step_mixed)
+//   0 / 1  RK4 step, FP64 / mixed (rk4_step64 with the next step's position
+//          terms, which hold the radius / rk4_step_mixed)
 //   2 / 3  geodesic step: RK4 + radius + step rule, FP64 / mixed (the
 //          geodesic wave's arithmetic per round, geodesics.py:249-261, 317-336)
 //   4 / 5  trilinear interpolation of the 8 primitives from 8 corner records
@@ -46,24 +47,30 @@ __global__ void __launch_bounds__(64) k_step_cycles(int variant, int steps, doub
   const double rEH = 1.0 + __builtin_sqrt(1.0 - a * a);
   for (int k = 0; k < 200; ++k) {
     double nw[8];
-    rk4_step<double>(s, -(radius_cal(s[1], s[2], s[3], a) - rEH) / 40.0, a, nw);
+    const KsHead h0 = ks_head(s[1], s[2], s[3], a);
+    rk4_step64(s, h0, -(h0.r - rEH) / 40.0, a, nw);
     for (int q = 0; q < 8; ++q) s[q] = nw[q];
   }
   double acc = 0.0;
   unsigned long long c0 = 0, c1 = 0, w0 = 0, w1 = 0;
   if (variant <= 3) {
     double dt = -0.02;
+    KsHead h = ks_head(s[1], s[2], s[3], a);
     pin(s[1]);
     c0 = __builtin_readcyclecounter();
     w0 = __builtin_amdgcn_s_memrealtime();
     for (int k = 0; k < steps; ++k) {
       double nw[8];
-      if (variant == 0 || variant == 2) rk4_step<double>(s, dt, a, nw);
-      else rk4_step_mixed(s, dt, (float)a, nw);
+      if (variant == 0 || variant == 2) {
+        rk4_step64(s, h, dt, a, nw);
+        h = ks_head(nw[1], nw[2], nw[3], a);
+      } else {
+        rk4_step_mixed(s, dt, (float)a, nw);
+      }
       if (variant >= 2) {
         double rn, dtn;
         if (variant == 2) {
-          rn = radius_cal(nw[1], nw[2], nw[3], a);
+          rn = h.r;
           dtn = step_rule(rn, rEH, 40.0, 1e-4);
         } else {
           rn = radius_f32(nw[1], nw[2], nw[3], a);

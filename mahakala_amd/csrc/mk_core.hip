@@ -85,7 +85,7 @@ __global__ void k_rhs(const double* s, long n, double a, double* out) {
   if (p >= n) return;
   const double* q = s + 8 * p;
   double acc[4];
-  ks_accel<double>(q[1], q[2], q[3], q[4], q[5], q[6], q[7], a, acc);
+  ks_accel64(ks_head(q[1], q[2], q[3], a), q[1], q[2], q[3], q[4], q[5], q[6], q[7], a, acc);
 #pragma unroll
   for (int k = 0; k < 4; ++k) { out[8 * p + k] = q[4 + k]; out[8 * p + 4 + k] = acc[k]; }
 }
@@ -96,7 +96,7 @@ __global__ void k_rk4(const double* s, const double* dt, long n, double a, doubl
   double st[8], nw[8];
 #pragma unroll
   for (int k = 0; k < 8; ++k) st[k] = s[8 * p + k];
-  rk4_step<double>(st, dt[p], a, nw);
+  rk4_step64(st, ks_head(st[1], st[2], st[3], a), dt[p], a, nw);
 #pragma unroll
   for (int k = 0; k < 8; ++k) out[8 * p + k] = nw[k];
 }
@@ -125,14 +125,16 @@ __device__ __forceinline__ void walk_ray(const double s0[8], int N, double div, 
   for (int k = 0; k < 8; ++k) s[k] = s0[k];
   double r = radius_cal(s[1], s[2], s[3], a);
   double dt = step_rule(r, rEH, div, tol);
+  KsHead h = ks_head(s[1], s[2], s[3], a), hn = h;
   double best = -__builtin_inf(), r_prev = __builtin_nan(""), r_at = __builtin_nan("");
   int besti = -1, K = N;
   for (int n = 0; n < N; ++n) {
     bool frozen = (dt == 0.0);
     double rn = 0.0, dtn = 0.0;
     if (!frozen) {
-      rk4_step<double>(s, dt, a, nw);
-      rn = radius_cal(nw[1], nw[2], nw[3], a);
+      rk4_step64(s, h, dt, a, nw);
+      hn = ks_head(nw[1], nw[2], nw[3], a);
+      rn = hn.r;
       dtn = step_rule(rn, rEH, div, tol);
       frozen = (dtn == 0.0);
     }
@@ -145,6 +147,7 @@ __device__ __forceinline__ void walk_ray(const double s0[8], int N, double div, 
     for (int k = 0; k < 8; ++k) s[k] = nw[k];
     dt = dtn;
     r = rn;
+    h = hn;
   }
   o.K = K;
 #pragma unroll
@@ -185,6 +188,7 @@ __global__ void __launch_bounds__(256) k_integrate_history(const double* s0, lon
 #pragma unroll
   for (int k = 0; k < 8; ++k) s[k] = s0[8 * p + k];
   double dt = step_rule(radius_cal(s[1], s[2], s[3], a), rEH, div, tol);
+  KsHead h = ks_head(s[1], s[2], s[3], a), hn = h;
   bool frozen = false;
   for (long row = 0; row < T; ++row) {
     double edt = 0.0, dtn = 0.0;
@@ -192,8 +196,9 @@ __global__ void __launch_bounds__(256) k_integrate_history(const double* s0, lon
       if (dt == 0.0) {
         frozen = true;
       } else {
-        rk4_step<double>(s, dt, a, nw);
-        dtn = step_rule(radius_cal(nw[1], nw[2], nw[3], a), rEH, div, tol);
+        rk4_step64(s, h, dt, a, nw);
+        hn = ks_head(nw[1], nw[2], nw[3], a);
+        dtn = step_rule(hn.r, rEH, div, tol);
         if (dtn == 0.0) frozen = true;
         else edt = dt;
       }
@@ -206,6 +211,7 @@ __global__ void __launch_bounds__(256) k_integrate_history(const double* s0, lon
 #pragma unroll
       for (int k = 0; k < 8; ++k) s[k] = nw[k];
       dt = dtn;
+      h = hn;
     }
   }
 }

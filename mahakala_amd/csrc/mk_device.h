@@ -223,9 +223,31 @@ __device__ __forceinline__ void ks_accel(T x, T y, T z, T v0, T v1, T v2, T v3, 
   acc[3] = c3 - l3 * flc;
 }
 
-// Position terms of the metric in FP64: den = r^4 + a^2 z^2 = 2 r^2 Q with Q =
-// sqrt(k^2 + a^2 z^2), k = (x^2 + y^2 + z^2 - a^2)/2 (r^2 solves r^4 - 2 k r^2 -
-// a^2 z^2 = 0), so f = r/Q and the reciprocal of den is not needed.
+// --------------------------------------------- FP64 right-hand side and step
+// The FP64 chains (plain images, bisections, the integrator) are bound by the
+// issue of this code: one wave64 FP64 instruction per 4 cycles, one RK4 step
+// after the other.  It therefore takes the acceleration of ks_accel in a
+// shorter form, equal to it in exact arithmetic:
+//   den = r^4 + a^2 z^2 = 2 r^2 Q, with Q = sqrt(k^2 + a^2 z^2) and
+//     k = (x^2 + y^2 + z^2 - a^2)/2 (r^2 solves r^4 - 2 k r^2 - a^2 z^2 = 0),
+//     so f = r/Q, 2 r^2/den = 1/Q, kappa = (3/2r - f)/Q, zeta = a^2 l3/Q^2,
+//     and the reciprocal of den is gone;
+//   l is geodesic in flat space (l.grad l = 0) and of unit length, l.grad r =
+//     1 and z/r is constant along it, so l^b c_b = L^2/2 l.grad f =
+//     L^2/2 (1/Q - f^2): no contraction with c;
+//   c_b - l_b f (l.c) collects l_b (P + f l.c) = l_b a^t, and with d_i and
+//     A_i written in x_i and l_i, and l_i in x and y, the first two
+//     components are X x + Y y - 2 s a f L v2 and X y - Y x + 2 s a f L v1
+//     with shared X and Y; the dot products with v need only x v1 + y v2 and
+//     y v1 - x v2.
+// The radius of the step rule is the r of the next step's first stage, so the
+// state carries that stage's position terms (KsHead) from step to step and no
+// separate radius is evaluated.
+// Vector instructions per accepted step of k_bisect_band (step, radius and
+// step rule): 596 before, 448 now.  Bisection of 64 angles 3.06 -> 2.46 ms, of
+// 4096 angles 7.44 -> 6.00 ms, final states and histories of a 64^2 grid 3.66
+// -> 2.96 ms, plain FP64 512^2 image 6.21 -> 5.32 ms; the same radii and step
+// counts.
 struct KsHead {
   double rr, iQ, r, ir, s;  // r^2, 1/Q, r, 1/r, 1/(r^2 + a^2)
 };
@@ -243,7 +265,72 @@ __device__ __forceinline__ KsHead ks_head(double x, double y, double z, double a
   return h;
 }
 
-// RK4 over the 8-vector state, all in T (geodesics.py:317-336).  The stage
+__device__ __forceinline__ void ks_accel64(const KsHead& h, double x, double y, double z, double v0, double v1,
+                                           double v2, double v3, double a, double acc[4]) {
+  const double aa = a * a;
+  const double rs = h.r * h.s, as = a * h.s;
+  const double f = h.r * h.iQ, l3 = z * h.ir;
+  const double g = h.rr * h.iQ, fra = f * (h.rr + aa);  // d(r^2) = (x g, y g, l3 fra)
+  const double hr = 0.5 * h.ir, hi = hr * h.ir;         // A3 = -l3 hi
+  const double aQ = aa * (h.iQ * h.iQ);                 // zeta = l3 aQ
+  const double xv = x * v1 + y * v2, jv = y * v1 - x * v2, zv = l3 * v3;
+  const double lv = rs * xv + as * jv;                  // l1 v1 + l2 v2
+  const double L = v0 + lv + zv;
+  const double dv = g * xv + fra * zv;
+  const double Av = h.s * (hr * xv - lv) - hi * zv;
+  const double Wv = dv * Av + rs * (v1 * v1 + v2 * v2) + h.ir * (v3 * v3);
+  const double kap = h.iQ * (1.5 * h.ir - f);
+  const double fL = f * L, hL2 = 0.5 * L * L;
+  const double P = L * (kap * dv - aQ * zv) + f * Wv;
+  const double a0 = P + hL2 * (f * (h.iQ - f * f));
+  const double mu = hL2 * kap + fL * Av, nu = fL * dv;
+  const double nus = nu * h.s;
+  const double Y = nus - a0;
+  const double X = mu * g - nus * hr + Y * rs;
+  const double Ya = Y * as, w = 2.0 * as * fL;
+  acc[0] = a0;
+  acc[1] = X * x + Ya * y - w * v2;
+  acc[2] = X * y - Ya * x + w * v1;
+  acc[3] = l3 * (nu * hi - a0 + mu * fra - hL2 * aQ);
+}
+
+// RK4 step of the FP64 paths; h0: the position terms at s.  The stage
+// velocities are v + (h/2) a1, v + (h/2) a2 and v + h a3, so the position's
+// slope sum v1 + 2 v2 + 2 v3 + v4 is 6 v + h (a1 + a2 + a3) and only the
+// accelerations are summed.
+__device__ __forceinline__ void rk4_step64(const double s[8], const KsHead& h0, double dt, double a, double out[8]) {
+  const double hh = 0.5 * dt, h6 = dt * (1.0 / 6.0);
+  double a1[4], a2[4], a3[4], a4[4], x[4], v[4], u[4];
+  ks_accel64(h0, s[1], s[2], s[3], s[4], s[5], s[6], s[7], a, a1);
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    x[i] = s[i] + hh * s[4 + i];
+    v[i] = s[4 + i] + hh * a1[i];
+  }
+  ks_accel64(ks_head(x[1], x[2], x[3], a), x[1], x[2], x[3], v[0], v[1], v[2], v[3], a, a2);
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    x[i] = s[i] + hh * v[i];
+    u[i] = s[4 + i] + hh * a2[i];
+  }
+  ks_accel64(ks_head(x[1], x[2], x[3], a), x[1], x[2], x[3], u[0], u[1], u[2], u[3], a, a3);
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    x[i] = s[i] + dt * u[i];
+    v[i] = s[4 + i] + dt * a3[i];
+  }
+  ks_accel64(ks_head(x[1], x[2], x[3], a), x[1], x[2], x[3], v[0], v[1], v[2], v[3], a, a4);
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const double b = a2[i] + a3[i], c = a1[i] + b;
+    out[i] = s[i] + dt * (s[4 + i] + h6 * c);
+    out[4 + i] = s[4 + i] + h6 * (c + b + a4[i]);
+  }
+}
+
+// RK4 over the 8-vector state, all in T (geodesics.py:317-336): the FP64 steps
+// of the mixed-precision zone, whose neighbouring FP32 steps would turn a last
+// bit of the state into an FP32 ulp, so they keep ks_accel's roundings.  The stage
 // slopes stay unscaled: t = s + (h/2) F is one FMA, and h/6 scales the slope
 // sum F1 + 2 F2 + 2 F3 + F4 once, which saves the 32 products k = h F of the
 // scaled form (the roundings differ from it at the ulp level).

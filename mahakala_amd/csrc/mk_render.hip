@@ -49,6 +49,8 @@ __device__ __forceinline__ void trace_ray(const SnapView& sv, const double* meta
   nullify(sx, sv4, rp.a, s);
   double r = radius_cal(s[1], s[2], s[3], rp.a);
   double dt = step_rule(r, rp.rEH, rp.div, rp.tol);
+  KsHead h{}, hn{};  // FP64: the position terms at s and at the candidate
+  if constexpr (!MIXED) h = ks_head(s[1], s[2], s[3], rp.a);
   double I = 0.0, trans = 1.0, drdl = 1e300;
   int nacc = 0;
   bool pend = false;
@@ -96,12 +98,12 @@ __device__ __forceinline__ void trace_ray(const SnapView& sv, const double* meta
       // a sample of the wave is inside the domain: the next RK4 step and
       // that sample's emission are independent, and one straight block lets
       // a wave that is alone on its SIMD interleave the two
-      if constexpr (!MIXED) rk4_step<double>(s, dt, rp.a, nw);
+      if constexpr (!MIXED) rk4_step64(s, h, dt, rp.a, nw);
       else rk4_step_mixed(s, dt, (float)rp.a, nw);
       consume_flat();
     } else {
       if constexpr (!MIXED) {
-        rk4_step<double>(s, dt, rp.a, nw);
+        rk4_step64(s, h, dt, rp.a, nw);
       } else {
         const bool fp64 = zone && __any((r < rp.fp64_r) || (r < rp.ring_r && __builtin_fabs(drdl) < rp.ring_drdl));
         if (fp64) rk4_step<double>(s, dt, rp.a, nw);
@@ -112,7 +114,8 @@ __device__ __forceinline__ void trace_ray(const SnapView& sv, const double* meta
     pend = false;
     double rn, dtn;
     if constexpr (!MIXED) {
-      rn = radius_cal(nw[1], nw[2], nw[3], rp.a);
+      hn = ks_head(nw[1], nw[2], nw[3], rp.a);
+      rn = hn.r;
       dtn = step_rule(rn, rp.rEH, rp.div, rp.tol);
     } else {
       rn = radius_f32(nw[1], nw[2], nw[3], rp.a);
@@ -138,6 +141,7 @@ __device__ __forceinline__ void trace_ray(const SnapView& sv, const double* meta
     for (int q = 0; q < 8; ++q) s[q] = nw[q];
     dt = dtn;
     r = rn;
+    h = hn;
   }
   if (pend) consume();
   I_out = I;
@@ -307,6 +311,7 @@ __global__ void __launch_bounds__(128 * kPairTiles) k_render_pair(SnapView sv, R
   const long p = (long)pi * rp.res + pj;
   if (geo) {
     double s[8], r = 0.0, dt = 0.0, drdl = 1e300;
+    KsHead h{}, hn{};  // FP64: the position terms at s and at the candidate
     int k = 0, nacc = 0;
     bool alive = false;
     if (valid) {
@@ -315,6 +320,7 @@ __global__ void __launch_bounds__(128 * kPairTiles) k_render_pair(SnapView sv, R
       nullify(sx, sv4, rp.a, s);
       r = radius_cal(s[1], s[2], s[3], rp.a);
       dt = step_rule(r, rp.rEH, rp.div, rp.tol);
+      if constexpr (!MIXED) h = ks_head(s[1], s[2], s[3], rp.a);
       alive = true;
     }
     const bool zone = MIXED && (rp.fp64_r > 0.0 || rp.ring_r > 0.0);
@@ -333,7 +339,7 @@ __global__ void __launch_bounds__(128 * kPairTiles) k_render_pair(SnapView sv, R
         } else {
           double nw[8];
           if constexpr (!MIXED) {
-            rk4_step<double>(s, dt, rp.a, nw);
+            rk4_step64(s, h, dt, rp.a, nw);
           } else {
             const bool fp64 = zone && __any((r < rp.fp64_r) || (r < rp.ring_r && __builtin_fabs(drdl) < rp.ring_drdl));
             if (fp64) rk4_step<double>(s, dt, rp.a, nw);
@@ -341,7 +347,8 @@ __global__ void __launch_bounds__(128 * kPairTiles) k_render_pair(SnapView sv, R
           }
           double rn, dtn;
           if constexpr (!MIXED) {
-            rn = radius_cal(nw[1], nw[2], nw[3], rp.a);
+            hn = ks_head(nw[1], nw[2], nw[3], rp.a);
+            rn = hn.r;
             dtn = step_rule(rn, rp.rEH, rp.div, rp.tol);
           } else {
             rn = radius_f32(nw[1], nw[2], nw[3], rp.a);
@@ -362,6 +369,7 @@ __global__ void __launch_bounds__(128 * kPairTiles) k_render_pair(SnapView sv, R
             for (int c = 0; c < 8; ++c) s[c] = nw[c];
             dt = dtn;
             r = rn;
+            h = hn;
             if (++k >= rp.N) alive = false;
           }
         }
@@ -575,6 +583,7 @@ __global__ void __launch_bounds__(192 * kPairTiles) k_render_tri(SnapView sv, Re
   const long p = (long)pi * rp.res + pj;
   if (stage == 0) {  // geodesic
     double s[8], r = 0.0, dt = 0.0, drdl = 1e300;
+    KsHead h{}, hn{};  // FP64: the position terms at s and at the candidate
     int k = 0, nacc = 0;
     bool alive = false;
     if (valid) {
@@ -583,6 +592,7 @@ __global__ void __launch_bounds__(192 * kPairTiles) k_render_tri(SnapView sv, Re
       nullify(sx, sv4, rp.a, s);
       r = radius_cal(s[1], s[2], s[3], rp.a);
       dt = step_rule(r, rp.rEH, rp.div, rp.tol);
+      if constexpr (!MIXED) h = ks_head(s[1], s[2], s[3], rp.a);
       alive = true;
     }
     const bool zone = ZONE != 0 && MIXED && (rp.fp64_r > 0.0 || rp.ring_r > 0.0);
@@ -614,7 +624,7 @@ __global__ void __launch_bounds__(192 * kPairTiles) k_render_tri(SnapView sv, Re
       double* nw = MIXED ? s : nw_;
       if (alive) {
         if constexpr (!MIXED) {
-          rk4_step<double>(s, dt, rp.a, nw);
+          rk4_step64(s, h, dt, rp.a, nw);
         } else {
           bool fp64;
           if constexpr (ZONE == 2) fp64 = zone && ((r < rp.fp64_r) || (r < rp.ring_r && __builtin_fabs(drdl) < rp.ring_drdl));
@@ -645,7 +655,8 @@ __global__ void __launch_bounds__(192 * kPairTiles) k_render_tri(SnapView sv, Re
       if (alive) {
         double rn, dtn;
         if constexpr (!MIXED) {
-          rn = radius_cal(nw[1], nw[2], nw[3], rp.a);
+          hn = ks_head(nw[1], nw[2], nw[3], rp.a);
+          rn = hn.r;
           dtn = step_rule(rn, rp.rEH, rp.div, rp.tol);
         } else {
           rn = radius_f32(nw[1], nw[2], nw[3], rp.a);
@@ -668,6 +679,7 @@ __global__ void __launch_bounds__(192 * kPairTiles) k_render_tri(SnapView sv, Re
           }
           dt = dtn;
           r = rn;
+          h = hn;
           if (++k >= rp.N) alive = false;
         }
       }

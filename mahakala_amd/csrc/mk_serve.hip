@@ -108,6 +108,7 @@ __device__ __forceinline__ void pop_tile(const ServeArgs& A, int& rid, int& tile
 struct Lane {
   double s[8], dt, r, f10, f11, best, r_prev, r_at;
   int k, n, besti;
+  KsHead h;             // FP64 steps: the position terms at s
   int cmb;              // block of the ray's last sample (-1: none), and its record:
   double crec[kMeta];   // the snapshot tables are in global memory here, not in LDS
 };
@@ -119,6 +120,7 @@ __device__ __forceinline__ void shadow_begin(const ReqDev& q, int item, Lane& L)
   nullify(sx, sv4, q.a, L.s);
   L.r = radius_cal(L.s[1], L.s[2], L.s[3], q.a);
   L.dt = step_rule(L.r, q.rEH, 40.0, 1e-2);
+  L.h = ks_head(L.s[1], L.s[2], L.s[3], q.a);
   L.k = 0;
   L.best = -__builtin_inf();
   L.besti = -1;
@@ -147,6 +149,7 @@ __device__ __forceinline__ bool item_begin(const ReqDev& q, int item, Lane& L) {
     nullify(sx, sv4, q.a, L.s);
     L.r = radius_cal(L.s[1], L.s[2], L.s[3], q.a);
     L.dt = step_rule(L.r, q.rEH, q.div, q.tol);
+    L.h = ks_head(L.s[1], L.s[2], L.s[3], q.a);
     L.f10 = 0.0;  // I
     L.f11 = 1.0;  // transmission
     L.k = 0;
@@ -195,11 +198,12 @@ template <bool MIXED, bool IN_PLACE = false>
 __device__ __forceinline__ bool image_pass(const ReqDev& q, bool go, Lane& L, Pending& p, bool& pend) {
   bool fin = false, adv = false;
   double nw[8];
+  KsHead hn{};
   if (go) {
     if (L.k >= q.N || L.dt == 0.0) {
       fin = true;
     } else {
-      if constexpr (!MIXED) rk4_step<double>(L.s, L.dt, q.a, nw);
+      if constexpr (!MIXED) rk4_step64(L.s, L.h, L.dt, q.a, nw);
       else rk4_step_mixed(L.s, L.dt, (float)q.a, nw);
       adv = true;
     }
@@ -211,7 +215,8 @@ __device__ __forceinline__ bool image_pass(const ReqDev& q, bool go, Lane& L, Pe
   if (adv) {
     double rn, dtn;
     if constexpr (!MIXED) {
-      rn = radius_cal(nw[1], nw[2], nw[3], q.a);
+      hn = ks_head(nw[1], nw[2], nw[3], q.a);
+      rn = hn.r;
       dtn = step_rule(rn, q.rEH, q.div, q.tol);
     } else {
       rn = radius_f32(nw[1], nw[2], nw[3], q.a);
@@ -238,6 +243,7 @@ __device__ __forceinline__ bool image_pass(const ReqDev& q, bool go, Lane& L, Pe
       for (int c = 0; c < 8; ++c) L.s[c] = nw[c];
       L.dt = dtn;
       L.r = rn;
+      if constexpr (!MIXED) L.h = hn;
       ++L.k;
       fin = L.k >= q.N;  // no sample is pending then
     }
@@ -252,9 +258,11 @@ __device__ __forceinline__ bool shadow_step(const ReqDev& q, int item, Lane& L) 
   const double r_here = L.r;
   bool frozen = (L.dt == 0.0);
   double nw[8], rn = 0.0, dtn = 0.0;
+  KsHead hn{};
   if (!frozen) {
-    rk4_step<double>(L.s, L.dt, q.a, nw);
-    rn = radius_cal(nw[1], nw[2], nw[3], q.a);
+    rk4_step64(L.s, L.h, L.dt, q.a, nw);
+    hn = ks_head(nw[1], nw[2], nw[3], q.a);
+    rn = hn.r;
     dtn = step_rule(rn, q.rEH, 40.0, 1e-2);
     frozen = (dtn == 0.0);
   }
@@ -274,6 +282,7 @@ __device__ __forceinline__ bool shadow_step(const ReqDev& q, int item, Lane& L) 
       for (int c = 0; c < 8; ++c) L.s[c] = nw[c];
       L.dt = dtn;
       L.r = rn;
+      L.h = hn;
       ++L.k;
     }
   }
@@ -318,6 +327,7 @@ __global__ void __launch_bounds__(256, 2) k_serve(const ReqDev* __restrict__ req
     L.k = A.i[l];
     L.n = A.i[L_ + l];
     L.besti = A.i[2 * L_ + l];
+    L.h = ks_head(L.s[1], L.s[2], L.s[3], req[rid].a);  // the same bits as before the launch boundary
   }
   int budget = A.M, steps = 0;
   while (budget > 0) {
