@@ -204,10 +204,9 @@ typedef struct mk_render_params {
 } mk_render_params;
 
 /* mk_render_params.flags: kernel form.  By default the library runs a launch
- * of up to 3 8x8 tiles per SIMD in the triple form -- a geodesic wave, a
- * gather wave (block lookup, cell loads, interpolation) and an emission wave
- * per tile, with the snapshot's block tables in LDS where they fit and in
- * global memory otherwise -- and a larger one in the classic form (one wave
+ * of up to 15.5 8x8 tiles per CU (11 in FP64) in the triple form -- a geodesic
+ * wave, two gather waves (block lookup, cell loads, interpolation) and an
+ * emission wave per tile -- and a larger one in the classic form (one wave
  * per tile).  The paired form (a geodesic wave and a transfer wave per tile)
  * runs only when forced and its tables fit in LDS (else the classic form).
  * The bits force one form; all give the same image, bit for bit. */

@@ -429,11 +429,13 @@ __device__ __forceinline__ double radius_f32(double x, double y, double z, doubl
   return (double)__builtin_amdgcn_sqrtf(0.5f * (w + __builtin_amdgcn_sqrtf(w * w + 4.0f * aa * (zf * zf))));
 }
 
-// step rule with the division by div replaced by a product with 1/div
-__device__ __forceinline__ double step_rule_fast(double r, double rEH, double inv_div, double div, double tol) {
+// step rule with the division by div replaced by a product with 1/div; lim:
+// the reference's 1500, or less for a ray whose later steps cannot matter
+__device__ __forceinline__ double step_rule_fast(double r, double rEH, double inv_div, double div, double tol,
+                                                 double lim = 1500.0) {
   const double dt = -(r - rEH) * inv_div;
   const double m = __builtin_fabs(dt) * div;
-  if (dt != dt || m < tol || m > 1500.0) return 0.0;
+  if (dt != dt || m < tol || m > lim) return 0.0;
   return dt;
 }
 
@@ -443,14 +445,14 @@ __device__ __forceinline__ double step_rule_fast(double r, double rEH, double in
 // is exact in one FMA and q + residual y rounds to num/div (Markstein's
 // theorem; no overflow or underflow here).  A zero num gives +0 where the
 // division gives -0, and both are frozen below.
-__device__ __forceinline__ double step_rule(double r, double rEH, double div, double tol) {
+__device__ __forceinline__ double step_rule(double r, double rEH, double div, double tol, double lim = 1500.0) {
 #pragma clang fp contract(off)
   const double num = -(r - rEH);
   const double y = 1.0 / div;
   const double q = num * y;
   const double dt = __builtin_fma(__builtin_fma(-q, div, num), y, q);
   const double m = __builtin_fabs(dt) * div;
-  if (dt != dt || m < tol || m > 1500.0) return 0.0;
+  if (dt != dt || m < tol || m > lim) return 0.0;
   return dt;
 }
 

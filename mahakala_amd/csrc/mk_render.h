@@ -12,10 +12,13 @@ struct RenderDev {
   long ntiles;
   ImageParams ip;
   double fp64_r, ring_r, ring_drdl;
+  double r_dom, r_out;  // set_domain_radii
   int spin_limit;     // polls before a bounded wait gives up (paired and triple forms)
   const int* order;   // tiles in the order they are handed out (nullptr: row-major)
   int* next_tile;     // classic form: tiles taken from this counter by each wave (nullptr: one tile per wave)
 };
+
+void set_domain_radii(const SnapView& sv, bool whole_rays, double* r_dom, double* r_out);
 
 int fill_render_dev(const mk_render_params* p, RenderDev* rp);
 

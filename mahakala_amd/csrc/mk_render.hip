@@ -438,31 +438,39 @@ __global__ void __launch_bounds__(128 * kPairTiles) k_render_pair(SnapView sv, R
 }
 
 // ------------------------------------------------------------- triple form
-// Three waves per tile on one SIMD -- geodesic, gather (lookup, cell loads,
+// Three stages per tile -- geodesic, gather (lookup, cell loads,
 // interpolation) and emission (fluid scalars, j and alpha, transfer) --
-// chained by two LDS rings with the counters of the paired form: three
-// independent instruction streams fill the SIMD better than two.  Ring A
-// carries (state, dt) from the geodesic wave, ring B the eight interpolated
-// primitives and the state in the emission's precision (FP32 values are what
-// the FP32 emission would round them to) and dt in FP64 (0: nothing to add).
-// Ring depths: ring A (geodesic -> gather) holds 3 rounds in mixed, 2 in
-// FP64 (LDS), ring B (gather -> emission) DB_ rounds (3 in mixed where LDS
-// allows, else 2).
-template <bool MIXED, int DB_>
+// chained by two LDS rings with the counters of the paired form.  One tile is
+// one workgroup of four waves: a geodesic wave, two gather waves that take the
+// rounds in turn, and an emission wave.  A lone gather wave's round (ring
+// read, lookup, cell loads, interpolation: one latency after the other) takes
+// about 3300 cycles, a geodesic step 2200, so one gather wave set the pace.
+// The hardware puts a workgroup's four waves on the CU's four SIMDs and
+// rotates the order from workgroup to workgroup, so with four workgroups per
+// CU every SIMD holds one wave of each kind.  The block tables stay in global
+// memory (each gather wave keeps its rays' last block record in registers):
+// with 51 KB of them in LDS only two workgroups fit a CU, and where both fit
+// the times are equal.
+// 256^2, a = 0.9, i = 60 deg (a = 0.5, i = 30 deg): with four tiles and one
+// gather wave each per workgroup, tables in LDS, plain FP64 3.99 (2.08) ms,
+// mixed 3.38 (1.72) ms; with this split 3.48 (2.02) and 3.22 (1.57) ms; with
+// rays ending outside the domain and nothing handed over on their way in 3.14
+// (1.73) and 3.03 (1.46) ms.  160^2 at a = 0.9: plain 3.93 -> 2.70 ms, mixed 3.18 -> 2.65 ms.
+// Ring A carries (state, dt) from the geodesic wave, ring B the eight
+// interpolated primitives and the state in the emission's precision (FP32
+// values are what the FP32 emission would round them to) and dt in FP64 (0:
+// nothing to add).
+template <bool MIXED>
 struct TriRings {
   using T = typename std::conditional<MIXED, float, double>::type;
-  static constexpr int kDepthA = MIXED ? 3 : 2, kDepthB = DB_;
-  static constexpr int kCompB = 15;                                                  // P[8], s[1..7]
-  static constexpr size_t kA = (size_t)kPairTiles * kDepthA * kPairComp * 64;        // doubles
-  static constexpr size_t kBd = (size_t)kPairTiles * kDepthB * 64;                   // doubles (dt)
-  static constexpr size_t kBt = (size_t)kPairTiles * kDepthB * kCompB * 64;          // elements of T
-  static constexpr size_t kLdsExtra = (kA + kBd) * sizeof(double) + kBt * sizeof(T) + kPairTiles * 8 * sizeof(int);
+  static constexpr int kDepthA = 4, kDepthB = MIXED ? 4 : 2;  // rounds (35 KB: four workgroups fit 160 KB)
+  static constexpr int kCompB = 15;                           // P[8], s[1..7]
+  double a[kDepthA][kPairComp][64];
+  double bd[kDepthB][64];  // dt
+  T bt[kDepthB][kCompB][64];
+  int producedA, doneA, consumedB;
+  int consumedA[2], producedB[2], doneB[2];  // per gather wave
 };
-
-template <bool MIXED, int DB_>
-constexpr size_t tri_lds_extra() {
-  return TriRings<MIXED, DB_>::kLdsExtra;
-}
 
 // Polls *cnt until it reaches target: the value read, or -1 after `limit`
 // polls.
@@ -496,236 +504,171 @@ __device__ __forceinline__ int wait_round(int* produced, int* done, int t, int* 
   return -1;
 }
 
-// LDS: the block tables are staged in LDS; otherwise (a snapshot whose tables
-// exceed the LDS budget) they are read from global memory, and the gather
-// wave keeps each ray's last block record in registers.  ZONE (mixed): 0 the
-// zone code is compiled out; 1 the geodesic wave takes FP64 steps while any
-// of its rays is in the zone (rp.fp64_r, rp.ring_r), as the other forms do;
-// 2 only for launches without a zone, where that test never fires: the zone
-// code in the loop layout that measured fastest for launches of several
-// workgroup waves (builds 0 and 1 were 5-9 % slower there, same results).
-// Build 2's test is per ray, not per tile, so it must never see a zone:
-// launch_tri refuses one (MK_ERR_ARG).
-template <bool MIXED, bool LDS, int DB_, int ZONE>
-__global__ void __launch_bounds__(192 * kPairTiles) k_render_tri(SnapView sv, RenderDev rp, double* __restrict__ img,
-                                                                  int32_t* __restrict__ steps, int tab_doubles,
-                                                                  int nres) {
+// ZONE (mixed): the geodesic wave takes FP64 steps while any of its rays is in
+// the zone (rp.fp64_r, rp.ring_r), as the other forms do; without it the zone
+// code is compiled out.
+template <bool MIXED, bool ZONE>
+__global__ void __launch_bounds__(256, 4) k_render_tri(SnapView sv, RenderDev rp, double* __restrict__ img,
+                                                       int32_t* __restrict__ steps) {
   using T = typename std::conditional<MIXED, float, double>::type;
-  using R = TriRings<MIXED, DB_>;
-  constexpr int DA = R::kDepthA, DB = R::kDepthB, CB = R::kCompB;
-  extern __shared__ double lds[];
-  double* ringA_all = lds + tab_doubles;
-  double* ringBd_all = ringA_all + R::kA;
-  T* ringBt_all = reinterpret_cast<T*>(ringBd_all + R::kBd);
-  // per tile: producedA, consumedA, doneA, producedB, consumedB, doneB, pad, pad
-  int* ctr = reinterpret_cast<int*>(ringBt_all + R::kBt);
-  if (threadIdx.x < 8 * kPairTiles) {
-    const int f = threadIdx.x & 7;
-    ctr[threadIdx.x] = (f == 2 || f == 5) ? -1 : 0;
-  }
-  const double* meta;
-  const int* grid;
-  stage_tables<LDS>(sv, lds, meta, grid);  // with LDS: ends with a workgroup barrier
-  if constexpr (!LDS) __syncthreads();    // the counters are set
-  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-  // Wave w runs on SIMD w % 4 (the hardware's placement).  The three waves of
-  // tile k sit on SIMDs k, k + 1 and k + 2: every SIMD holds one wave of each
-  // stage, and a tile that outlives the others of its workgroup has its
-  // stages on three SIMDs instead of sharing one.
-  const int stage = wave / kPairTiles;
-  const int tl = (wave + (kPairTiles - 1) * stage) % kPairTiles;
-  double* ringA = ringA_all + (size_t)tl * DA * kPairComp * 64 + lane;
-  double* ringBd = ringBd_all + (size_t)tl * DB * 64 + lane;
-  T* ringBt = ringBt_all + (size_t)tl * DB * CB * 64 + lane;
-  int* c = ctr + 8 * tl;
-  const unsigned nwg = gridDim.x, wg = blockIdx.x, per = nwg / 8;
-  // with a tile order, workgroups take ranks in index (start) order
-  const unsigned lwg = (!rp.order && nwg % 8 == 0) ? (wg % 8) * per + wg / 8 : wg;
-  // Workgroups lwg < n (n = nres) are strided: their four tiles come from four
-  // quarters of ranks [0, 4n) of the order (four bands of the image without
-  // one), taken in snake order (ranks w, 2n - 1 - w, 2n + w, 4n - 1 - w), so
-  // the longest tiles share their CU with the shortest.  The host sets n to
-  // the whole grid when every workgroup is resident at once, to the resident
-  // count when a tile order spreads over at most two waves of workgroups (the
-  // first wave then holds one long tile per CU, and the second, the shortest
-  // tiles, starts as CUs free), else 0.  Workgroups from n on take the rest of
-  // the ranks in order, four adjacent ones each.
-  const unsigned n = (unsigned)nres;
-  const bool first = lwg < n;
-  long tile = first ? ((tl & 1) ? (long)(tl + 1) * n - 1 - lwg : (long)tl * n + lwg)
-                    : 4L * n + (long)(lwg - n) * kPairTiles + tl;
-  // Strided with a tile order: the three waves of the tile from the first
-  // quarter (the longest tiles) issue at a raised priority, so where the waves
-  // of a SIMD compete it goes first; the other tiles have slack until it
-  // ends, and the waits of every wave sleep, so they still run.  FP64 uses one
-  // level per quarter (1-3 % faster there than one raised level; in mixed
-  // 1 % slower).
-  // s_setprio is a scalar instruction: it takes effect whatever the exec
-  // mask, so the condition is made uniform (an SGPR and a scalar branch).
-  if (first && rp.order) {
-    const int q = __builtin_amdgcn_readfirstlane(tl);
-    if constexpr (MIXED) {
-      if (q == 0) __builtin_amdgcn_s_setprio(1);
-    } else {  // FP64: one level per quarter
-      if (q == 0) __builtin_amdgcn_s_setprio(3);
-      else if (q == 1) __builtin_amdgcn_s_setprio(2);
-      else if (q == 2) __builtin_amdgcn_s_setprio(1);
+  using R = TriRings<MIXED>;
+  constexpr int DA = R::kDepthA, DB = R::kDepthB;
+  __shared__ R ring;
+  if (threadIdx.x == 0) {
+    ring.producedA = ring.consumedB = 0;
+    ring.doneA = -1;
+    for (int g = 0; g < 2; ++g) {
+      ring.consumedA[g] = ring.producedB[g] = 0;
+      ring.doneB[g] = -1;
     }
   }
-  if (rp.order && tile < rp.ntiles) tile = rp.order[tile];
-  int pi = 0, pj = 0;
-  bool valid = tile < rp.ntiles;
-  if (valid) {
-    pi = (int)(tile / rp.tiles_x) * 8 + (lane >> 3);
-    pj = (int)(tile % rp.tiles_x) * 8 + (lane & 7);
-    valid = pi < rp.res && pj < rp.res;
-  }
+  __syncthreads();
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  // workgroups start in index order: with a tile order the longest tiles go
+  // first; without one each of the 8 XCDs takes a contiguous band of tiles
+  const unsigned nwg = gridDim.x, wg = blockIdx.x;
+  long tile = (!rp.order && nwg % 8 == 0) ? (wg % 8) * (nwg / 8) + wg / 8 : wg;
+  if (rp.order) tile = rp.order[tile];
+  const int pi = (int)(tile / rp.tiles_x) * 8 + (lane >> 3), pj = (int)(tile % rp.tiles_x) * 8 + (lane & 7);
+  const bool valid = pi < rp.res && pj < rp.res;
   const long p = (long)pi * rp.res + pj;
-  if (stage == 0) {  // geodesic
+  if (wave == 0) {  // geodesic
+    // A lane is alive while its dt is not 0; dead lanes step along with dt = 0
+    // and are ignored, so the loop has no branches per lane.  All live lanes
+    // have taken the same number of steps, k.
     double s[8], r = 0.0, dt = 0.0, drdl = 1e300;
     KsHead h{}, hn{};  // FP64: the position terms at s and at the candidate
     int k = 0, nacc = 0;
-    bool alive = false;
+#pragma unroll
+    for (int q = 0; q < 8; ++q) s[q] = 0.0;
     if (valid) {
       double sx[4], sv4[4];
       camera_ray(grid_coord(rp.lo, rp.step, pi), grid_coord(rp.lo, rp.step, pj), rp.ci, rp.si, rp.dist, sx, sv4);
       nullify(sx, sv4, rp.a, s);
       r = radius_cal(s[1], s[2], s[3], rp.a);
       dt = step_rule(r, rp.rEH, rp.div, rp.tol);
-      if constexpr (!MIXED) h = ks_head(s[1], s[2], s[3], rp.a);
-      alive = true;
     }
-    const bool zone = ZONE != 0 && MIXED && (rp.fp64_r > 0.0 || rp.ring_r > 0.0);
+    if constexpr (!MIXED) h = ks_head(s[1], s[2], s[3], rp.a);
+    double lim = 1500.0;  // largest |r - r_EH| of a live ray
+    // one RK4 step of every live lane into nw (mixed may step in place: the
+    // step functions write their output only after reading the state)
+    auto step = [&](double nw[8]) {
+      if constexpr (!MIXED) {
+        rk4_step64(s, h, dt, rp.a, nw);
+      } else {
+        const bool fp64 = ZONE && __any(dt != 0.0 && ((r < rp.fp64_r) || (r < rp.ring_r && __builtin_fabs(drdl) < rp.ring_drdl)));
+        if (fp64) rk4_step<double>(s, dt, rp.a, nw);
+        else rk4_step_mixed(s, dt, (float)rp.a, nw);
+      }
+    };
+    // radius and step of the candidate; 0 ends the ray
+    auto rule = [&](const double nw[8], double& rn) {
+      double dtn;
+      if constexpr (!MIXED) {
+        hn = ks_head(nw[1], nw[2], nw[3], rp.a);
+        rn = hn.r;
+        dtn = step_rule(rn, rp.rEH, rp.div, rp.tol, lim);
+      } else {
+        rn = radius_f32(nw[1], nw[2], nw[3], rp.a);
+        dtn = step_rule_fast(rn, rp.rEH, rp.inv_div, rp.div, rp.tol, lim);
+      }
+      return dt != 0.0 ? dtn : 0.0;
+    };
+    // The way in: no ray of the tile is inside the sphere around the domain,
+    // so the steps are taken without handing anything over.  The step that
+    // first takes a ray inside is left to the loop below.
+    double nw_[8];
+    while (k < rp.N && __any(dt != 0.0)) {
+      double rn;
+      step(nw_);
+      const double dtn = rule(nw_, rn);
+      if (__any(dtn != 0.0 && rn <= rp.r_dom)) break;
+      nacc += dtn != 0.0;
+      if (ZONE) drdl = (rn - r) / dt;
+#pragma unroll
+      for (int q = 0; q < 8; ++q) s[q] = nw_[q];
+      dt = dtn;
+      r = rn;
+      h = hn;
+      ++k;
+    }
+    // A ray inside the sphere of radius r_out ends when it leaves it again.
+    if (r < rp.r_out) lim = __builtin_fmin(1500.0, rp.r_out - rp.rEH);
     bool ok = true;
-    int t = 0, freed = 0;  // freed: ring A rounds the gather wave has read (last value seen)
-    while (__any(alive)) {
-      // Slot t % DA is free once the gather wave has read round t - DA.  FP64
-      // and the zone-free mixed build load that count here without waiting
-      // and check it after the RK4 step: a wait at the loop head would also
-      // wait on this wave's slot writes of the round before (-2 to -4 % in
-      // FP64, -1 % in one-wave mixed launches; the mixed zone build, which
-      // also runs launches of several workgroup waves, measured slower).
-      int polled = 0;
-      if constexpr (!MIXED || ZONE == 0) {
-        polled = __hip_atomic_load(c + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
-      } else if (t - DA + 1 > freed) {
-        freed = wait_value(c + 1, t - DA + 1, rp.spin_limit);
-        if (freed < 0) {
-          ok = false;
-          break;
-        }
-      }
-      double* out = ringA + (size_t)(t % DA) * kPairComp * 64;
-      if (alive && (k >= rp.N || dt == 0.0)) alive = false;
-      // mixed steps the state in place (the step functions write their output
-      // only after reading the state; a ray that stops is not used again):
-      // -1.3 %; in FP64 the copy is faster
-      double nw_[8];
-      double* nw = MIXED ? s : nw_;
-      if (alive) {
-        if constexpr (!MIXED) {
-          rk4_step64(s, h, dt, rp.a, nw);
-        } else {
-          bool fp64;
-          if constexpr (ZONE == 2) fp64 = zone && ((r < rp.fp64_r) || (r < rp.ring_r && __builtin_fabs(drdl) < rp.ring_drdl));
-          else fp64 = zone && __any((r < rp.fp64_r) || (r < rp.ring_r && __builtin_fabs(drdl) < rp.ring_drdl));
-          if (fp64) rk4_step<double>(s, dt, rp.a, nw);
-          else rk4_step_mixed(s, dt, (float)rp.a, nw);
-        }
-      }
+    int t = 0;  // the next round
+    for (; k < rp.N && __any(dt != 0.0); ++k, ++t) {
+      // Slot t % DA is free once round t - DA has been read.  That count is
+      // loaded here without waiting and checked after the RK4 step: a wait at
+      // the loop head would also wait on this wave's slot writes of the round
+      // before (-2 to -4 % in FP64, -1 % in mixed).
+      int* readA = &ring.consumedA[t & 1];
+      const int polled = __hip_atomic_load(readA, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+      double* out = &ring.a[t % DA][0][lane];
+      double* nw = MIXED ? s : nw_;  // mixed in place: -1.3 %; in FP64 the copy is faster
+      step(nw);
       // release the previous round here: its slot writes were issued a whole
       // RK4 step ago, so the release fence does not wait on them
-      if (t > 0) publish(c + 0, t);
-      if constexpr (!MIXED || ZONE == 0) {
-        const int seen = __builtin_amdgcn_readfirstlane(polled);
-        if (t - DA + 1 > freed) {
-          if (seen >= t - DA + 1) {
-            freed = seen;
-            __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
-          } else {
-            freed = wait_value(c + 1, t - DA + 1, rp.spin_limit);
-            if (freed < 0) {
-              ok = false;
-              break;
-            }
-          }
-        }
+      if (t > 0) publish(&ring.producedA, t);
+      if (__builtin_amdgcn_readfirstlane(polled) > t - DA) {
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
+      } else if (wait_value(readA, t - DA + 1, rp.spin_limit) < 0) {
+        ok = false;
+        break;
       }
-      bool wrote = false;
-      if (alive) {
-        double rn, dtn;
-        if constexpr (!MIXED) {
-          hn = ks_head(nw[1], nw[2], nw[3], rp.a);
-          rn = hn.r;
-          dtn = step_rule(rn, rp.rEH, rp.div, rp.tol);
-        } else {
-          rn = radius_f32(nw[1], nw[2], nw[3], rp.a);
-          dtn = step_rule_fast(rn, rp.rEH, rp.inv_div, rp.div, rp.tol);
-        }
-        if (dtn == 0.0) {
-          alive = false;
-        } else {
-          ++nacc;
-          if (k + 1 < rp.N) {  // row N is never emitted
+      double rn;
+      const double dtn = rule(nw, rn);
+      nacc += dtn != 0.0;
 #pragma unroll
-            for (int q = 0; q < 8; ++q) out[q * 64] = nw[q];
-            out[8 * 64] = dt;
-            wrote = true;
-          }
-          if (zone) drdl = (rn - r) / dt;
-          if constexpr (!MIXED) {
+      for (int q = 0; q < 8; ++q) out[q * 64] = nw[q];
+      out[8 * 64] = dtn != 0.0 && k + 1 < rp.N ? dt : 0.0;  // row N is never emitted
+      if (ZONE) drdl = (rn - r) / dt;
+      if constexpr (!MIXED) {
 #pragma unroll
-            for (int q = 0; q < 8; ++q) s[q] = nw[q];
-          }
-          dt = dtn;
-          r = rn;
-          h = hn;
-          if (++k >= rp.N) alive = false;
-        }
+        for (int q = 0; q < 8; ++q) s[q] = nw[q];
       }
-      if (!wrote) out[8 * 64] = 0.0;
-      ++t;
+      dt = dtn;
+      r = rn;
+      h = hn;
     }
-    if (ok) publish(c + 0, t);
-    publish(c + 2, ok ? t : -2);
+    if (ok) publish(&ring.producedA, t);
+    publish(&ring.doneA, ok ? t : -2);
     if (valid && steps) steps[p] = ok ? nacc : -1;
     return;
   }
-  if (stage == 1) {  // gather: lookup, cell loads, interpolation
+  if (wave <= 2) {  // gather: lookup, cell loads, interpolation of every other round
+    const int g = wave - 1;
     bool ok = true;
-    int t = 0, avail = 0, freed = 0;  // rounds of ring A published, of ring B read (last values seen)
-    int cmb = -1;                     // global tables: block of the ray's last sample and its record
+    int avail = 0, freed = 0;  // rounds of ring A published, of ring B read (last values seen)
+    int cmb = -1;              // block of the ray's last sample and its record
     double crec[kMeta];
-    for (;; ++t) {
+    int t = g;
+    for (;; t += 2) {
       if (t >= avail) {
-        const int st = wait_round(c + 0, c + 2, t, &avail, rp.spin_limit);
+        const int st = wait_round(&ring.producedA, &ring.doneA, t, &avail, rp.spin_limit);
         if (st <= 0) {
           ok = st == 0;
           break;
         }
       }
       if (t - DB + 1 > freed) {
-        freed = wait_value(c + 4, t - DB + 1, rp.spin_limit);
+        freed = wait_value(&ring.consumedB, t - DB + 1, rp.spin_limit);
         if (freed < 0) {
           ok = false;
           break;
         }
       }
-      const double* in = ringA + (size_t)(t % DA) * kPairComp * 64;
+      const double* in = &ring.a[t % DA][0][lane];
       double pdt = in[8 * 64];
       double ps[8];
 #pragma unroll
       for (int q = 0; q < 8; ++q) ps[q] = in[q * 64];
-      publish(c + 1, t + 1);  // ring A slot is in registers
-      T* ob = ringBt + (size_t)(t % DB) * CB * 64;
-      double* obd = ringBd + (size_t)(t % DB) * 64;
+      publish(&ring.consumedA[g], t + 1);  // ring A slot is in registers
+      T* ob = &ring.bt[t % DB][0][lane];
       T P[8];
 #pragma unroll
       for (int q = 0; q < 8; ++q) P[q] = T(0);
       if (pdt != 0.0) {
-        Stencil stc;
-        if constexpr (LDS) stc = locate(sv, meta, grid, ps[1], ps[2], ps[3]);
-        else stc = locate_cached(sv, meta, grid, ps[1], ps[2], ps[3], cmb, crec);
+        const Stencil stc = locate_cached(sv, sv.meta, sv.grid, ps[1], ps[2], ps[3], cmb, crec);
         if (stc.mb >= 0) {
           Corners cr;
           fetch(sv, stc, cr);
@@ -737,26 +680,24 @@ __global__ void __launch_bounds__(192 * kPairTiles) k_render_tri(SnapView sv, Re
       for (int q = 0; q < 8; ++q) ob[q * 64] = P[q];
 #pragma unroll
       for (int q = 1; q < 8; ++q) ob[(7 + q) * 64] = (T)ps[q];
-      obd[0] = pdt;
-      publish(c + 3, t + 1);
+      ring.bd[t % DB][lane] = pdt;
+      publish(&ring.producedB[g], t + 1);
     }
-    publish(c + 5, ok ? t : -2);
+    publish(&ring.doneB[g], ok ? t : -2);
     return;
   }
   // emission and transfer, in step order
   double I = 0.0, trans = 1.0;
   bool ok = true;
-  int avail = 0;  // rounds of ring B published (last value seen)
   for (int t = 0;; ++t) {
-    if (t >= avail) {
-      const int st = wait_round(c + 3, c + 5, t, &avail, rp.spin_limit);
-      if (st <= 0) {
-        ok = st == 0;
-        break;
-      }
+    int avail = 0;
+    const int st = wait_round(&ring.producedB[t & 1], &ring.doneB[t & 1], t, &avail, rp.spin_limit);
+    if (st <= 0) {
+      ok = st == 0;
+      break;
     }
-    const T* ib = ringBt + (size_t)(t % DB) * CB * 64;
-    const double pdt = ringBd[(size_t)(t % DB) * 64];
+    const T* ib = &ring.bt[t % DB][0][lane];
+    const double pdt = ring.bd[t % DB][lane];
     T P[8];
     double ps[8];
 #pragma unroll
@@ -764,7 +705,7 @@ __global__ void __launch_bounds__(192 * kPairTiles) k_render_tri(SnapView sv, Re
     ps[0] = 0.0;
 #pragma unroll
     for (int q = 1; q < 8; ++q) ps[q] = (double)ib[(7 + q) * 64];
-    publish(c + 4, t + 1);  // ring B slot is in registers
+    publish(&ring.consumedB, t + 1);  // ring B slot is in registers
     if (pdt != 0.0) {
       T j, al;
       emission_from_prims<T>(rp.ip, P, ps, rp.a, j, al);
@@ -923,6 +864,23 @@ size_t table_bytes(const SnapView& sv) {
   return (size_t)sv.nmb * kMeta * sizeof(double) + (size_t)sv.gx * sv.gy * sv.gz * sizeof(int);
 }
 
+// r_dom: no point of the domain has a larger Kerr-Schild radius (r^2 <= x^2 +
+// y^2 + z^2; the corner's distance with a margin for the radius in FP32).
+// r_out: a ray that moves outward beyond it, outside the domain, never returns
+// (a null geodesic has no outer turning point beyond the photon orbits, r <= 4 M),
+// so every later step would add exactly nothing and the ray may end: an escaping
+// ray takes about 120 of its 530 steps out there.  Infinite when the caller asks
+// for step counts, which cover the whole ray.
+void set_domain_radii(const SnapView& sv, bool whole_rays, double* r_dom, double* r_out) {
+  double s = 0.0;
+  for (int d = 0; d < 3; ++d) {
+    const double m = std::max(std::fabs(sv.dom_lo[d]), std::fabs(sv.dom_hi[d]));
+    s += m * m;
+  }
+  *r_dom = 1.001 * std::sqrt(s);
+  *r_out = whole_rays ? HUGE_VAL : std::max(1.1 * *r_dom, 12.0);
+}
+
 int fill_render_dev(const mk_render_params* p, RenderDev* rp) {
   MK_REQUIRE(p->resolution > 0 && p->max_nsteps >= 1 && p->div != 0.0, "render: bad resolution/max_nsteps/div");
   MK_REQUIRE(p->precision == 0 || p->precision == 1, "render: precision must be 0 (plain FP64) or 1 (mixed)");
@@ -968,70 +926,11 @@ int fill_render_dev(const mk_render_params* p, RenderDev* rp) {
 
 using namespace mk;
 
-// Paired form where the tables fit in LDS next to the rings and the launch
-// has fewer than about 1.75 tiles per SIMD (measured on MI355X: paired is
-// 15-24 % faster up to 1600 tiles on 1024 SIMDs, and 8-24 % slower from 2304
-// tiles, where three classic workgroups per CU keep more waves in flight).
-// Tables in LDS when they fit kMaxTableLds and, with the form's rings, the
-// 160 KB of a CU; the triple form also runs with the tables in global memory.
-template <bool MIXED, bool LDS, int DB_>
-static int launch_tri(const SnapView& sv, const RenderDev& rp, double* d_image, int32_t* d_steps, size_t tab,
-                      hipStream_t st) {
-  long nwg = (rp.ntiles + kPairTiles - 1) / kPairTiles;
-  nwg = (nwg + 7) / 8 * 8;
-  const size_t lds = tab + tri_lds_extra<MIXED, DB_>();
-  // strided tiles for the workgroups resident at once (see k_render_tri)
-  // resident workgroups of the build that runs: the zone build (1) for a
-  // zone; otherwise the zone-free build (0) when the grid is resident at
-  // once with it, else build 2
-  const bool zoned = MIXED && (rp.fp64_r > 0.0 || rp.ring_r > 0.0);
-  int dev = 0, cus = 0, per_cu = 0;
-  hipError_t e = hipGetDevice(&dev);
-  if (e == hipSuccess) e = hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev);
-  if (e == hipSuccess)
-    e = hipOccupancyMaxActiveBlocksPerMultiprocessor(
-        &per_cu, zoned ? k_render_tri<MIXED, LDS, DB_, MIXED ? 1 : 0> : k_render_tri<MIXED, LDS, DB_, 0>,
-        192 * kPairTiles, lds);
-  if (e == hipSuccess && MIXED && !zoned && nwg > (long)per_cu * cus)
-    e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, k_render_tri<MIXED, LDS, DB_, MIXED ? 2 : 0>,
-                                                     192 * kPairTiles, lds);
-  if (e != hipSuccess) {
-    set_error("mk_render: occupancy query failed");
-    return MK_ERR_HIP;
-  }
-  const long R = (long)per_cu * cus;
-  const int nres = nwg <= R ? (int)nwg : (rp.order && nwg <= 2 * R ? (int)R : 0);
-  const int tabd = (int)(tab / sizeof(double));
-  // mixed: the zone build for a zone; without one, the zone-free build where
-  // every workgroup is resident at once (-2 to -3 % at 192^2-256^2) and
-  // build 2 in launches of several workgroup waves (see k_render_tri)
-  const dim3 grid((unsigned)nwg), blk(192 * kPairTiles);
-  if (zoned)
-    k_render_tri<MIXED, LDS, DB_, MIXED ? 1 : 0><<<grid, blk, lds, st>>>(sv, rp, d_image, d_steps, tabd, nres);
-  else if (MIXED && nwg > R) {
-    // build 2 decides FP64 steps per ray: a zone here would break the
-    // tile-wide rule every other form follows
-    MK_REQUIRE(rp.fp64_r <= 0.0 && rp.ring_r <= 0.0, "mk_render: internal: zone sent to the zone-free build");
-    k_render_tri<MIXED, LDS, DB_, MIXED ? 2 : 0><<<grid, blk, lds, st>>>(sv, rp, d_image, d_steps, tabd, nres);
-  }
-  else
-    k_render_tri<MIXED, LDS, DB_, 0><<<grid, blk, lds, st>>>(sv, rp, d_image, d_steps, tabd, nres);
+template <bool MIXED, bool ZONE>
+static int launch_tri(const SnapView& sv, const RenderDev& rp, double* d_image, int32_t* d_steps, hipStream_t st) {
+  k_render_tri<MIXED, ZONE><<<dim3((unsigned)rp.ntiles), dim3(256), 0, st>>>(sv, rp, d_image, d_steps);
   MK_LAUNCH_CHECK();
   return MK_OK;
-}
-
-// The triple form's variant: 0 tables in LDS with 3 ring-B slots (mixed),
-// 1 tables in LDS with 2 slots, 2 tables in global memory (3 slots in mixed,
-// 2 in FP64).
-static int tri_variant(const SnapView& sv, int precision) {
-  const size_t tab = (table_bytes(sv) + 15) / 16 * 16;
-  const bool small = table_bytes(sv) <= kMaxTableLds;
-  if (precision == 1) {
-    if (small && tab + tri_lds_extra<true, 3>() <= 160 * 1024) return 0;
-    if (small && tab + tri_lds_extra<true, 2>() <= 160 * 1024) return 1;
-    return 2;
-  }
-  return small && tab + tri_lds_extra<false, 2>() <= 160 * 1024 ? 1 : 2;
 }
 
 static int choose_form(const SnapView& sv, const RenderDev& rp, int precision, int flags, int* form) {
@@ -1055,7 +954,9 @@ static int choose_form(const SnapView& sv, const RenderDev& rp, int precision, i
   }
   // triple form up to 15.5 tiles per CU in mixed precision (a 496^2 image on
   // 256 CUs) and 11 in FP64 (424^2); the classic form beyond, where every
-  // SIMD holds three waves of whole rays
+  // SIMD holds waves of whole rays.  a = 0.5, i = 30 deg (a = 0.9, i = 60 deg),
+  // triple against classic: mixed 480^2 3.10 (3.15) and 4.72 (7.51) ms, 640^2
+  // 4.9 (4.7) and 4.7 (8.0) ms; plain FP64 416^2 3.45 (3.50) and 4.31 (8.54) ms.
   if (2 * rp.ntiles <= (precision == 1 ? 31L : 22L) * cus) *form = MK_RENDER_TRIPLE;
   return MK_OK;
 }
@@ -1081,6 +982,9 @@ extern "C" int mk_render(const mk_snapshot* snap, const mk_render_params* p, dou
   long nwg = (rp.ntiles + waves_per_wg - 1) / waves_per_wg;
   nwg = (nwg + 7) / 8 * 8;
   const SnapView sv = snap->view();
+  set_domain_radii(sv, d_steps != nullptr, &rp.r_dom, &rp.r_out);
+  // a tile's FP64 zone is decided by its live rays: none may end inside it
+  rp.r_out = std::max(rp.r_out, 1.1 * std::max(rp.fp64_r, rp.ring_r));
   const size_t lds = table_bytes(sv);
   const bool use_lds = lds <= kMaxTableLds;
   const dim3 grid((unsigned)nwg), block(64 * waves_per_wg);
@@ -1091,13 +995,9 @@ extern "C" int mk_render(const mk_snapshot* snap, const mk_render_params* p, dou
   if (rc) return rc;
   if (form != MK_RENDER_PAIRED && !(p->flags & MK_RENDER_ROW_MAJOR)) rp.order = render_tile_order(rp, p, st);
   if (form == MK_RENDER_TRIPLE) {
-    const int v = tri_variant(sv, p->precision);
-    if (p->precision == 0)
-      return v == 1 ? launch_tri<false, true, 2>(sv, rp, d_image, d_steps, tab, st)
-                    : launch_tri<false, false, 2>(sv, rp, d_image, d_steps, 0, st);
-    if (v == 0) return launch_tri<true, true, 3>(sv, rp, d_image, d_steps, tab, st);
-    if (v == 1) return launch_tri<true, true, 2>(sv, rp, d_image, d_steps, tab, st);
-    return launch_tri<true, false, 3>(sv, rp, d_image, d_steps, 0, st);
+    if (p->precision == 0) return launch_tri<false, false>(sv, rp, d_image, d_steps, st);
+    return rp.fp64_r > 0.0 || rp.ring_r > 0.0 ? launch_tri<true, true>(sv, rp, d_image, d_steps, st)
+                                              : launch_tri<true, false>(sv, rp, d_image, d_steps, st);
   }
   if (form == MK_RENDER_PAIRED) {
     long nwg2 = (rp.ntiles + kPairTiles - 1) / kPairTiles;

@@ -40,7 +40,7 @@ def render_params(bhspin, camera_inclination=60, camera_distance=1000, mass_scal
                   ring_drdl=None, form=None):
     """mk_render parameters.  form: None (the library chooses), "classic"
     (one wave per 8x8 tile), "paired" (a geodesic wave and a transfer wave
-    per tile) or "triple" (geodesic, gather and emission waves per tile);
+    per tile) or "triple" (geodesic, two gather and an emission wave per tile);
     all forms give the same image, bit for bit."""
     if precision not in PRECISIONS:
         raise ValueError(f"precision must be one of {sorted(PRECISIONS)}")
