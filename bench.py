@@ -409,13 +409,12 @@ def main():
         form = C.c_int32()
         L.check(L.lib().mk_render_form(snap.handle, par[p], C.byref(form)))
         m = "true" if par[p].precision == 1 else "false"
+        zone = "true" if m == "true" and (par[p].fp64_radius > 0 or par[p].ring_radius > 0) else "false"
         if form.value == images.FORMS["triple"]:
-            zone = "true" if m == "true" and (par[p].fp64_radius > 0 or par[p].ring_radius > 0) else "false"
             return f"k_render_tri<{m}, {zone}>"
         if form.value == images.FORMS["paired"]:
             return f"k_render_pair<{m}>"
-        # classic: tables in LDS; mixed runs three workgroups per CU with in-place samples
-        return f"k_render<{m}, true, {m}>"
+        return f"k_render<{m}, {zone}>"
 
     def launch(p, steps_out=False):
         def fn():

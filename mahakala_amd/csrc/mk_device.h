@@ -660,6 +660,13 @@ struct Corners {
   float4 q[8][2];
 };
 
+// FIRST: all 16 loads are issued before anything that follows waits for one.
+// Scheduled together with the interpolation, the compiler loads and waits in
+// smaller batches to save registers: plain FP64 512^2 image 4.94 ms against
+// 4.01, sampler on 3.4e6 points 133 against 113 us.  The triple form's gather
+// waves do without it: they have 128 registers and would spill (plain 160^2
+// 2.81 against 2.75 ms).
+template <bool FIRST = true>
 __device__ __forceinline__ void fetch(const SnapView& sv, const Stencil& st, Corners& c) {
   if (st.mb < 0) return;
   const long n2 = sv.n2, sj = 2 * n2, sk = 2 * n2 * n2;
@@ -674,6 +681,7 @@ __device__ __forceinline__ void fetch(const SnapView& sv, const Stencil& st, Cor
         c.q[kk * 4 + jj * 2 + ii][0] = e[0];
         c.q[kk * 4 + jj * 2 + ii][1] = e[1];
       }
+  if constexpr (FIRST) __builtin_amdgcn_sched_barrier(0);
 }
 
 // Trilinear interpolant (athenak.py:746-752) as a weighted sum of the 8

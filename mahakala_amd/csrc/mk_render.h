@@ -28,7 +28,7 @@ int fill_render_dev(const mk_render_params* p, RenderDev* rp);
 // tiles out first shortens a launch's tail; only the schedule changes.
 std::vector<int> ring_first_tile_order(int res, double lo, double step, double a, double inc_deg);
 
-// LDS budget for the staged block geometry + lookup grid (bytes)
+// LDS budget for the staged block geometry + lookup grid (bytes; paired form)
 constexpr size_t kMaxTableLds = 64 * 1024;
 size_t table_bytes(const SnapView& sv);
 

@@ -29,121 +29,86 @@
 
 namespace mk {
 
-// One ray: the sample of accepted step k is located (lookup tables in LDS)
-// and its 8 corner records are requested right after the step, then
-// consumed after the next RK4 step has been computed, so the gather latency
-// overlaps the geodesic arithmetic.  Contributions are still added in step
-// order, so the result is the same as sampling in place.
-// CACHE (tables in global memory): the ray keeps its last block record and
-// skips the lookup while its samples stay in that block.  IN_PLACE (mixed
-// precision, tables in LDS, three workgroups per CU): no pipeline; the sample is consumed
-// right after its step, so no corner records are held across the next RK4
-// step and the kernel fits three waves per SIMD (168 VGPRs), which hides the
-// load latency better than the pipeline does at two.
-template <bool MIXED, bool CACHE, bool IN_PLACE>
-__device__ __forceinline__ void trace_ray(const SnapView& sv, const double* meta, const int* grid, const RenderDev& rp,
-                                          double x_img, double y_img, double& I_out, int& steps_out) {
+// One ray.  The sample of an accepted step is located, fetched and added right
+// after the step (in the order of the steps); the ray keeps its last block
+// record and skips the lookup while its samples stay in that block.  ZONE
+// (mixed): FP64 steps while a live ray of the wave is in the zone; a build of
+// its own, since the second RK4 step's code costs every mixed launch (1024^2
+// torus at a = 0.94, i = 17 deg: 9.35 -> 8.44 ms without it).
+template <bool MIXED, bool ZONE>
+__device__ __forceinline__ void trace_ray(const SnapView& sv, const RenderDev& rp, double x_img, double y_img,
+                                          double& I_out, int& steps_out) {
   using T = typename std::conditional<MIXED, float, double>::type;
-  double sx[4], sv4[4], s[8];
+  double sx[4], sv4[4], s[8], nw[8], rn, dtn;
   camera_ray(x_img, y_img, rp.ci, rp.si, rp.dist, sx, sv4);
   nullify(sx, sv4, rp.a, s);
   double r = radius_cal(s[1], s[2], s[3], rp.a);
   double dt = step_rule(r, rp.rEH, rp.div, rp.tol);
   KsHead h{}, hn{};  // FP64: the position terms at s and at the candidate
   if constexpr (!MIXED) h = ks_head(s[1], s[2], s[3], rp.a);
-  double I = 0.0, trans = 1.0, drdl = 1e300;
-  int nacc = 0;
-  bool pend = false;
-  Stencil pst;
-  Corners pc;
-  double ps[8], pdt = 0.0;
-  int cmb = -1;
+  double I = 0.0, trans = 1.0, drdl = 1e300, lim = 1500.0;
+  int nacc = 0, k = 0, cmb = -1;
   double crec[kMeta];
-  // Outside the domain (all primitives zero) and wherever the density is
-  // zero, the reference's j and alpha come out 0 (or NaN, then 0), and the
-  // step adds exactly nothing: those samples skip the emission arithmetic.
-  auto consume = [&]() {
-    if (pst.mb < 0) return;
-    T P[8], j, al;
-    interp<T>(pst, pc, P);
-    if (P[0] == T(0)) return;
-    emission_from_prims<T>(rp.ip, P, ps, rp.a, j, al);
-    const double c = -pdt * rp.ip.L_unit;
-    I += trans * (c * (double)j);
-    trans *= (1.0 - c * (double)al);
-  };
-  // The same sum without branches: lanes with nothing to add evaluate the
-  // emission too and keep I and the transmission by selection.
-  auto consume_flat = [&]() {
-    T P[8], j, al;
-    interp_raw<T>(pst, pc, P);
-    emission_from_prims<T>(rp.ip, P, ps, rp.a, j, al);
-    const bool use = pend && pst.mb >= 0 && P[0] != T(0);
-    const double c = -pdt * rp.ip.L_unit;
-    const double In = I + trans * (c * (double)j);
-    const double tn = trans * (1.0 - c * (double)al);
-    I = use ? In : I;
-    trans = use ? tn : trans;
-  };
-  const bool zone = MIXED && (rp.fp64_r > 0.0 || rp.ring_r > 0.0);
-#pragma unroll
-  for (int q = 0; q < 8; ++q) pc.q[q][0] = pc.q[q][1] = make_float4(0.f, 0.f, 0.f, 0.f);
-  pst.mb = -1;
-  pst.base = 0;
-  pst.fr[0] = pst.fr[1] = pst.fr[2] = 0.0;
-  for (int k = 0; k < rp.N; ++k) {
-    if (dt == 0.0) break;
-    double nw[8];
-    if (!zone && __any(pend && pst.mb >= 0)) {
-      // a sample of the wave is inside the domain: the next RK4 step and
-      // that sample's emission are independent, and one straight block lets
-      // a wave that is alone on its SIMD interleave the two
-      if constexpr (!MIXED) rk4_step64(s, h, dt, rp.a, nw);
-      else rk4_step_mixed(s, dt, (float)rp.a, nw);
-      consume_flat();
-    } else {
-      if constexpr (!MIXED) {
-        rk4_step64(s, h, dt, rp.a, nw);
-      } else {
-        const bool fp64 = zone && __any((r < rp.fp64_r) || (r < rp.ring_r && __builtin_fabs(drdl) < rp.ring_drdl));
-        if (fp64) rk4_step<double>(s, dt, rp.a, nw);
-        else rk4_step_mixed(s, dt, (float)rp.a, nw);
-      }
-      if (pend) consume();
-    }
-    pend = false;
-    double rn, dtn;
+  // RK4 step to the candidate nw, its radius and its step (0 ends the ray)
+  auto step = [&]() {
     if constexpr (!MIXED) {
+      rk4_step64(s, h, dt, rp.a, nw);
       hn = ks_head(nw[1], nw[2], nw[3], rp.a);
       rn = hn.r;
-      dtn = step_rule(rn, rp.rEH, rp.div, rp.tol);
+      dtn = step_rule(rn, rp.rEH, rp.div, rp.tol, lim);
     } else {
+      const bool fp64 = ZONE && __any(dt != 0.0 && ((r < rp.fp64_r) || (r < rp.ring_r && __builtin_fabs(drdl) < rp.ring_drdl)));
+      if (fp64) rk4_step<double>(s, dt, rp.a, nw);
+      else rk4_step_mixed(s, dt, (float)rp.a, nw);
       rn = radius_f32(nw[1], nw[2], nw[3], rp.a);
-      dtn = step_rule_fast(rn, rp.rEH, rp.inv_div, rp.div, rp.tol);
+      dtn = step_rule_fast(rn, rp.rEH, rp.inv_div, rp.div, rp.tol, lim);
     }
-    if (dtn == 0.0) break;
-    ++nacc;
-    if (k + 1 < rp.N) {  // row N is never emitted
-      if constexpr (CACHE) pst = locate_cached(sv, meta, grid, nw[1], nw[2], nw[3], cmb, crec);
-      else pst = locate(sv, meta, grid, nw[1], nw[2], nw[3]);
-      fetch(sv, pst, pc);
-#pragma unroll
-      for (int q = 0; q < 8; ++q) ps[q] = nw[q];
-      pdt = dt;
-      pend = true;
-      if constexpr (IN_PLACE) {
-        consume();
-        pend = false;
-      }
-    }
-    if (zone) drdl = (rn - r) / dt;
+  };
+  auto accept = [&]() {
+    if (ZONE) drdl = (rn - r) / dt;
 #pragma unroll
     for (int q = 0; q < 8; ++q) s[q] = nw[q];
     dt = dtn;
     r = rn;
     h = hn;
+  };
+  // the way in, as in the triple form: no sample until a ray of the wave is
+  // inside the domain's sphere, and the step that takes it there is left to
+  // the loop below
+  while (k < rp.N && __any(dt != 0.0)) {
+    step();
+    dtn = dt != 0.0 ? dtn : 0.0;
+    if (__any(dtn != 0.0 && rn <= rp.r_dom)) break;
+    nacc += dtn != 0.0;
+    accept();
+    ++k;
   }
-  if (pend) consume();
+  // a ray inside the sphere of radius r_out ends when it leaves it again
+  if (r < rp.r_out) lim = __builtin_fmin(1500.0, rp.r_out - rp.rEH);
+  for (; k < rp.N && dt != 0.0; ++k) {
+    step();
+    if (dtn == 0.0) break;
+    ++nacc;
+    if (k + 1 < rp.N) {  // row N is never emitted
+      const Stencil st = locate_cached(sv, sv.meta, sv.grid, nw[1], nw[2], nw[3], cmb, crec);
+      // Outside the domain (all primitives zero) and wherever the density is
+      // zero, the reference's j and alpha come out 0 (or NaN, then 0), and the
+      // step adds exactly nothing: those samples skip the emission arithmetic.
+      if (st.mb >= 0) {
+        Corners c;
+        T P[8], j, al;
+        fetch(sv, st, c);
+        interp<T>(st, c, P);
+        if (P[0] != T(0)) {
+          emission_from_prims<T>(rp.ip, P, nw, rp.a, j, al);
+          const double cc = -dt * rp.ip.L_unit;
+          I += trans * (cc * (double)j);
+          trans *= (1.0 - cc * (double)al);
+        }
+      }
+    }
+    accept();
+  }
   I_out = I;
   steps_out = nacc;
 }
@@ -171,39 +136,35 @@ __device__ __forceinline__ bool pixel_of_lane(const RenderDev& rp, int& i, int& 
   return i < rp.res && j < rp.res;
 }
 
-// Copies the block geometry and the leaf lookup grid into LDS (when they
-// fit), so block lookup and stencil arithmetic never wait on HBM.
-template <bool LDS>
+// Copies the block geometry and the leaf lookup grid into LDS (paired form).
 __device__ __forceinline__ void stage_tables(const SnapView& sv, double* lds, const double*& meta, const int*& grid) {
-  meta = sv.meta;
-  grid = sv.grid;
-  if constexpr (LDS) {
-    const int nm = sv.nmb * kMeta, ng = sv.gx * sv.gy * sv.gz;
-    for (int t = threadIdx.x; t < nm; t += blockDim.x) lds[t] = sv.meta[t];
-    int* g = reinterpret_cast<int*>(lds + nm);
-    for (int t = threadIdx.x; t < ng; t += blockDim.x) g[t] = sv.grid[t];
-    __syncthreads();
-    meta = lds;
-    grid = g;
-  }
+  const int nm = sv.nmb * kMeta, ng = sv.gx * sv.gy * sv.gz;
+  for (int t = threadIdx.x; t < nm; t += blockDim.x) lds[t] = sv.meta[t];
+  int* g = reinterpret_cast<int*>(lds + nm);
+  for (int t = threadIdx.x; t < ng; t += blockDim.x) g[t] = sv.grid[t];
+  __syncthreads();
+  meta = lds;
+  grid = g;
 }
 
-// IN_PLACE (mixed, tables in LDS small enough for three workgroups per CU):
-// samples consumed right after their step, three waves per SIMD.
+// Three waves per SIMD in mixed (168 VGPRs), two in FP64.  The block tables are
+// read from global memory: against one copy of them in LDS per CU (workgroups
+// of 12 or 8 waves) mixed 768^2 at a = 0.9, i = 60 deg 7.05 against 7.88 ms,
+// 1024^2 at a = 0.94, i = 17 deg 8.60 against 8.53 ms, plain FP64 8.3 against
+// 9.1 and 11.7 against 11.9 ms, and a launch needs no staging and no limit on
+// the number of blocks.  (Two waves with the sample pipelined behind the next
+// step, the form before for FP64 and for tables beyond 53 KB: 1024^2 octree
+// 10.5 ms mixed, 13.0 ms FP64 at a = 0.94.)
 //
-// With rp.next_tile the grid holds only the workgroups resident at once: each
-// stages the tables once, and each of its waves takes the next tile (in tile
+// With rp.next_tile the grid holds only the workgroups resident at once, and
+// each of their waves takes the next tile (in tile
 // order) from the counter until none is left, so a wave whose tile ends early
 // starts another instead of idling until its workgroup's longest tile ends.
 // next_tile[1] counts the waves that found none left; the last of them sets
 // both words back to 0, so the next launch on the stream starts from 0.
-template <bool MIXED, bool LDS, bool IN_PLACE>
-__global__ void __launch_bounds__(256, IN_PLACE ? 3 : 2) k_render(SnapView sv, RenderDev rp, double* __restrict__ img,
-                                                                  int32_t* __restrict__ steps) {
-  extern __shared__ double lds[];
-  const double* meta;
-  const int* grid;
-  stage_tables<LDS>(sv, lds, meta, grid);
+template <bool MIXED, bool ZONE>
+__global__ void __launch_bounds__(256, MIXED ? 3 : 2) k_render(SnapView sv, RenderDev rp, double* __restrict__ img,
+                                                               int32_t* __restrict__ steps) {
   if (rp.next_tile) {
     const int lane = threadIdx.x & 63;
     while (true) {
@@ -224,8 +185,7 @@ __global__ void __launch_bounds__(256, IN_PLACE ? 3 : 2) k_render(SnapView sv, R
       if (i < rp.res && j < rp.res) {
         double I;
         int n;
-        trace_ray<MIXED, !LDS, IN_PLACE>(sv, meta, grid, rp, grid_coord(rp.lo, rp.step, i),
-                                         grid_coord(rp.lo, rp.step, j), I, n);
+        trace_ray<MIXED, ZONE>(sv, rp, grid_coord(rp.lo, rp.step, i), grid_coord(rp.lo, rp.step, j), I, n);
         const long p = (long)i * rp.res + j;
         img[p] = I;
         if (steps) steps[p] = n;
@@ -237,8 +197,7 @@ __global__ void __launch_bounds__(256, IN_PLACE ? 3 : 2) k_render(SnapView sv, R
   if (!pixel_of_lane(rp, i, j)) return;
   double I;
   int n;
-  trace_ray<MIXED, !LDS, IN_PLACE>(sv, meta, grid, rp, grid_coord(rp.lo, rp.step, i), grid_coord(rp.lo, rp.step, j),
-                                   I, n);
+  trace_ray<MIXED, ZONE>(sv, rp, grid_coord(rp.lo, rp.step, i), grid_coord(rp.lo, rp.step, j), I, n);
   const long p = (long)i * rp.res + j;
   img[p] = I;
   if (steps) steps[p] = n;
@@ -290,7 +249,7 @@ __global__ void __launch_bounds__(128 * kPairTiles) k_render_pair(SnapView sv, R
   if (threadIdx.x < 4 * kPairTiles) ctr[threadIdx.x] = ((threadIdx.x & 3) == 2) ? -1 : 0;
   const double* meta;
   const int* grid;
-  stage_tables<true>(sv, lds, meta, grid);  // ends with a workgroup barrier
+  stage_tables(sv, lds, meta, grid);  // ends with a workgroup barrier
   const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
   const int pair = wave % kPairTiles;
   const bool geo = wave < kPairTiles;
@@ -671,7 +630,7 @@ __global__ void __launch_bounds__(256, 4) k_render_tri(SnapView sv, RenderDev rp
         const Stencil stc = locate_cached(sv, sv.meta, sv.grid, ps[1], ps[2], ps[3], cmb, crec);
         if (stc.mb >= 0) {
           Corners cr;
-          fetch(sv, stc, cr);
+          fetch<false>(sv, stc, cr);
           interp<T>(stc, cr, P);
         }
         if (stc.mb < 0 || P[0] == T(0)) pdt = 0.0;  // adds exactly nothing
@@ -978,16 +937,11 @@ extern "C" int mk_render(const mk_snapshot* snap, const mk_render_params* p, dou
   RenderDev rp;
   int rc = fill_render_dev(p, &rp);
   if (rc) return rc;
-  const int waves_per_wg = 4;
-  long nwg = (rp.ntiles + waves_per_wg - 1) / waves_per_wg;
-  nwg = (nwg + 7) / 8 * 8;
   const SnapView sv = snap->view();
   set_domain_radii(sv, d_steps != nullptr, &rp.r_dom, &rp.r_out);
   // a tile's FP64 zone is decided by its live rays: none may end inside it
   rp.r_out = std::max(rp.r_out, 1.1 * std::max(rp.fp64_r, rp.ring_r));
   const size_t lds = table_bytes(sv);
-  const bool use_lds = lds <= kMaxTableLds;
-  const dim3 grid((unsigned)nwg), block(64 * waves_per_wg);
   hipStream_t st = as_stream(stream);
   const size_t tab = (lds + 15) / 16 * 16;
   int form = 0;
@@ -1011,27 +965,23 @@ extern "C" int mk_render(const mk_snapshot* snap, const mk_render_params* p, dou
     MK_LAUNCH_CHECK();
     return MK_OK;
   }
-  // the kernel instance and its LDS: three workgroups per CU (mixed) when
-  // their tables fit the CU's 160 KB of LDS
-  void (*kern)(SnapView, RenderDev, double*, int32_t*) = nullptr;
-  size_t kl = use_lds ? lds : 0;
-  if (p->precision == 0) kern = use_lds ? k_render<false, true, false> : k_render<false, false, false>;
-  else if (use_lds && 3 * lds <= 160 * 1024) kern = k_render<true, true, true>;
-  else kern = use_lds ? k_render<true, true, false> : k_render<true, false, false>;
-  dim3 g = grid;
+  const bool zoned = rp.fp64_r > 0.0 || rp.ring_r > 0.0;
+  auto kern = p->precision == 0 ? k_render<false, false> : (zoned ? k_render<true, true> : k_render<true, false>);
+  const int threads = 256, waves = threads / 64;
+  dim3 g((unsigned)(((rp.ntiles + waves - 1) / waves + 7) / 8 * 8));
   if (!(p->flags & MK_RENDER_STATIC_TILES)) {  // tiles from a counter (5-12 % faster at 1024^2)
     int dev = 0, cus = 0, per_cu = 0;
     rp.next_tile = tile_counter(st);
     if (rp.next_tile && hipGetDevice(&dev) == hipSuccess &&
         hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) == hipSuccess &&
-        hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, kern, (int)block.x, kl) == hipSuccess && per_cu > 0) {
+        hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, kern, threads, 0) == hipSuccess && per_cu > 0) {
       const long resident = (long)per_cu * cus;
-      if (resident < nwg) g = dim3((unsigned)resident);
+      if (resident < (long)g.x) g = dim3((unsigned)resident);
     } else {
       rp.next_tile = nullptr;
     }
   }
-  kern<<<g, block, kl, st>>>(sv, rp, d_image, d_steps);
+  kern<<<g, dim3(threads), 0, st>>>(sv, rp, d_image, d_steps);
   MK_LAUNCH_CHECK();
   return MK_OK;
 }

@@ -44,6 +44,7 @@ enum : int { kKindImage = 1, kKindShadow = 2 };
 struct alignas(256) ReqDev {
   int kind, n_items, res, N, iters, tiled;
   double a, ci, si, dist, lo, step, rEH, div, inv_div, tol;
+  double r_dom, r_out;  // image: set_domain_radii
   ImageParams ip;
   SnapView sv;
   double* out;
@@ -222,10 +223,11 @@ __device__ __forceinline__ bool image_pass(const ReqDev& q, bool go, Lane& L, Pe
       rn = radius_f32(nw[1], nw[2], nw[3], q.a);
       dtn = step_rule_fast(rn, q.rEH, q.inv_div, q.div, q.tol);
     }
-    if (dtn == 0.0) {
+    if (dtn == 0.0 || ((rn > q.r_out) & (rn > L.r))) {  // frozen, or outward beyond r_out (set_domain_radii)
       fin = true;
     } else {
-      if (L.k + 1 < q.N) {  // row N is never emitted
+      // row N is never emitted, and a step outside the domain's sphere adds nothing
+      if (L.k + 1 < q.N && rn <= q.r_dom) {
         // FP64 has no registers to spare for the cached record (it would spill)
         if constexpr (MIXED) p.st = locate_cached(q.sv, q.sv.meta, q.sv.grid, nw[1], nw[2], nw[3], L.cmb, L.crec);
         else p.st = locate(q.sv, q.sv.meta, q.sv.grid, nw[1], nw[2], nw[3]);
@@ -879,6 +881,7 @@ void fill_desc(mk_server* s, const mk_server::Pending& p, ReqDev& q, std::vector
     q.rEH = rd.rEH; q.div = rd.div; q.inv_div = rd.inv_div; q.tol = rd.tol;
     q.ip = rd.ip;
     q.sv = s->snaps[r.snapshot]->view();
+    set_domain_radii(q.sv, false, &q.r_dom, &q.r_out);
     return;
   }
   const mk_shadow_request& r = p.sh;
