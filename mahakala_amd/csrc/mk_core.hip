@@ -559,6 +559,157 @@ __global__ void k_attenuated(const double* j, const double* al, const double* dt
   }
 }
 
+// The same two scans for few rays, where one thread per ray leaves most of the
+// chip idle and each thread waits on its own loads (4096 rays are 16 blocks of
+// the kernels above).  A block takes kScanRays rays; its 256 threads load tiles
+// of kScanRows rows into registers, one tile ahead, and hand them over through
+// LDS, where the first kScanRays lanes run the rows in order: each batch of
+// rows is read (two rows a read) while the batch before is computed, so the
+// chain per row is three FP64 instructions (one for the optical depth).  The
+// arithmetic and its order are the kernels' above, bit for bit.  1240 rows,
+// intensity / attenuated emission: 500 rays 106 / 163 -> 32 / 35 us, 4096 rays
+// 106 / 164 -> 32 / 36 us (3.9 / 4.6 TB/s), 16384 rays 176 / 266 -> 97 / 144 us.
+constexpr int kScanRays = 16, kScanRows = 64, kScanThreads = 256;
+constexpr int kScanPer = kScanRays * kScanRows / kScanThreads;  // elements of a tile per thread
+constexpr int kScanStep = kScanThreads / kScanRays;             // rows between them
+constexpr int kScanPitch = kScanRows + 2;  // a lane's 16-byte reads of 16 rays fall in different banks
+// Up to this many rays the tile kernels run (2048 blocks, 8 per CU; from there
+// one thread per ray fills the chip too, and without barriers): 32768 rays at
+// 1240 rows 184 / 292 against 198 / 298 us, at 150 rows 22 / 31 against 22 /
+// 32; 65536 rays 365 / 574 against 312 / 477 us.
+constexpr long kScanMaxRays = 32768;
+
+template <bool DI>
+__global__ void __launch_bounds__(kScanThreads) k_solve_tiles(const double* j, const double* al, const double* dt,
+                                                              long T, long npx, double L, double* I, double* dI) {
+  __shared__ __align__(16) double sj[kScanRays][kScanPitch], sa[kScanRays][kScanPitch], st[kScanRays][kScanPitch];
+  const int ray = threadIdx.x % kScanRays, row0 = threadIdx.x / kScanRays;
+  const long p = (long)blockIdx.x * kScanRays + ray;
+  const bool mine = p < npx;
+  const long rows = T - 1;  // scan row k is sample T - 1 - k
+  double rj[kScanPer], ra[kScanPer], rd[kScanPer];
+  // beyond the rays and rows: zeros, which leave I as it is
+  auto load = [&](long k0) {
+#pragma unroll
+    for (int u = 0; u < kScanPer; ++u) {
+      const long k = k0 + row0 + u * kScanStep, i = T - 1 - k;
+      const bool in = mine && k < rows;
+      rj[u] = in ? j[i * npx + p] : 0.0;
+      ra[u] = in ? al[i * npx + p] : 0.0;
+      rd[u] = in ? dt[(i - 1) * npx + p] : 0.0;
+    }
+  };
+  load(0);
+  double Iv = 0.0;
+  for (long k0 = 0; k0 < rows; k0 += kScanRows) {
+#pragma unroll
+    for (int u = 0; u < kScanPer; ++u) {
+      const int r = row0 + u * kScanStep;
+      sj[ray][r] = rj[u];
+      sa[ray][r] = ra[u];
+      st[ray][r] = -rd[u] * L;
+    }
+    __syncthreads();
+    load(k0 + kScanRows);
+    if (threadIdx.x < kScanRays) {
+      constexpr int B = 4, N = kScanRows / B;  // rows per batch, batches
+      double jj[2][B], aa[2][B], tt[2][B];
+      auto read = [&](int q) {
+#pragma unroll
+        for (int u = 0; u < B; u += 2) {
+          const double2 vj = *reinterpret_cast<const double2*>(&sj[ray][q * B + u]);
+          const double2 va = *reinterpret_cast<const double2*>(&sa[ray][q * B + u]);
+          const double2 vt = *reinterpret_cast<const double2*>(&st[ray][q * B + u]);
+          jj[q & 1][u] = vj.x; jj[q & 1][u + 1] = vj.y;
+          aa[q & 1][u] = va.x; aa[q & 1][u + 1] = va.y;
+          tt[q & 1][u] = vt.x; tt[q & 1][u + 1] = vt.y;
+        }
+      };
+      read(0);
+#pragma unroll
+      for (int q = 0; q < N; ++q) {
+        if (q + 1 < N) read(q + 1);
+#pragma unroll
+        for (int u = 0; u < B; ++u) {
+          const double d = tt[q & 1][u] * (jj[q & 1][u] - (aa[q & 1][u] * Iv));
+          Iv = Iv + d;
+          if (DI) sj[ray][q * B + u] = d;
+        }
+      }
+    }
+    __syncthreads();
+    if (DI) {
+#pragma unroll
+      for (int u = 0; u < kScanPer; ++u) {
+        const int r = row0 + u * kScanStep;
+        if (mine && k0 + r < rows) dI[(k0 + r) * npx + p] = sj[ray][r];
+      }
+      __syncthreads();
+    }
+  }
+  if (threadIdx.x < kScanRays && mine) I[p] = Iv;
+}
+
+__global__ void __launch_bounds__(kScanThreads) k_attenuated_tiles(const double* j, const double* al, const double* dt,
+                                                                   long T, long npx, double L, double* out) {
+  // the optical depths' increments, then the depths
+  __shared__ __align__(16) double stau[2][kScanRays][kScanPitch];
+  const int ray = threadIdx.x % kScanRays, row0 = threadIdx.x / kScanRays;
+  const long p = (long)blockIdx.x * kScanRays + ray;
+  const bool mine = p < npx;
+  const long rows = T - 1;  // output row k is sample k + 1
+  double rj[kScanPer], ra[kScanPer], rd[kScanPer], src[kScanPer];
+  auto load = [&](long k0) {
+#pragma unroll
+    for (int u = 0; u < kScanPer; ++u) {
+      const long k = k0 + row0 + u * kScanStep;
+      const bool in = mine && k < rows;
+      rj[u] = in ? j[(k + 1) * npx + p] : 0.0;
+      ra[u] = in ? al[(k + 1) * npx + p] : 0.0;
+      rd[u] = in ? dt[k * npx + p] : 0.0;
+    }
+  };
+  load(0);
+  double tau = 0.0;
+  int b = 0;
+  for (long k0 = 0; k0 < rows; k0 += kScanRows, b ^= 1) {
+#pragma unroll
+    for (int u = 0; u < kScanPer; ++u) {
+      src[u] = -rj[u] * rd[u] * L;
+      stau[b][ray][row0 + u * kScanStep] = ra[u] * rd[u] * L;
+    }
+    __syncthreads();
+    load(k0 + kScanRows);
+    if (threadIdx.x < kScanRays) {
+      constexpr int B = 8, N = kScanRows / B;
+      double2* row = reinterpret_cast<double2*>(&stau[b][ray][0]);
+      double2 d[2][B / 2];
+      auto read = [&](int q) {
+#pragma unroll
+        for (int u = 0; u < B / 2; ++u) d[q & 1][u] = row[q * (B / 2) + u];
+      };
+      read(0);
+#pragma unroll
+      for (int q = 0; q < N; ++q) {
+        if (q + 1 < N) read(q + 1);
+#pragma unroll
+        for (int u = 0; u < B / 2; ++u) {
+          const double t1 = tau - d[q & 1][u].x;
+          row[q * (B / 2) + u] = make_double2(tau, t1);
+          tau = t1 - d[q & 1][u].y;
+        }
+      }
+    }
+    __syncthreads();
+    // the other buffer takes the next tile, so no barrier is needed after these reads
+#pragma unroll
+    for (int u = 0; u < kScanPer; ++u) {
+      const int r = row0 + u * kScanStep;
+      if (mine && k0 + r < rows) out[(k0 + r) * npx + p] = ::exp(-stau[b][ray][r]) * src[u];
+    }
+  }
+}
+
 __global__ void k_rlow_rhigh(const double* dens, const double* u, const double* beta, long n, double rl, double rh,
                              double ge, double gi, double* out) {
   const long p = (long)blockIdx.x * blockDim.x + threadIdx.x;
@@ -1197,7 +1348,11 @@ int mk_solve_intensity(const double* j, const double* al, const double* dt, long
                        double* dI, void* s) {
   MK_REQUIRE(T >= 0 && npx >= 0 && j && al && dt && I, "mk_solve_intensity: bad arguments");
   if (!npx) return MK_OK;
-  k_solve<<<grid_for(npx, kBlock), kBlock, 0, as_stream(s)>>>(j, al, dt, T, npx, L, I, dI);
+  if (npx <= kScanMaxRays)
+    (dI ? k_solve_tiles<true> : k_solve_tiles<false>)<<<grid_for(npx, kScanRays), kScanThreads, 0, as_stream(s)>>>(
+        j, al, dt, T, npx, L, I, dI);
+  else
+    k_solve<<<grid_for(npx, kBlock), kBlock, 0, as_stream(s)>>>(j, al, dt, T, npx, L, I, dI);
   MK_LAUNCH_CHECK();
   return MK_OK;
 }
@@ -1206,7 +1361,10 @@ int mk_attenuated_emissivity(const double* j, const double* al, const double* dt
                              double* out, void* s) {
   MK_REQUIRE(T >= 0 && npx >= 0 && j && al && dt && out, "mk_attenuated_emissivity: bad arguments");
   if (!npx || T < 2) return MK_OK;
-  k_attenuated<<<grid_for(npx, kBlock), kBlock, 0, as_stream(s)>>>(j, al, dt, T, npx, L, out);
+  if (npx <= kScanMaxRays)
+    k_attenuated_tiles<<<grid_for(npx, kScanRays), kScanThreads, 0, as_stream(s)>>>(j, al, dt, T, npx, L, out);
+  else
+    k_attenuated<<<grid_for(npx, kBlock), kBlock, 0, as_stream(s)>>>(j, al, dt, T, npx, L, out);
   MK_LAUNCH_CHECK();
   return MK_OK;
 }
