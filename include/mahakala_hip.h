@@ -266,10 +266,11 @@ typedef struct mk_server_config {
  * coming; the launch ends once the server has been idle for 20 ms (or, after
  * 1 s, whenever nothing is in flight) and the next request relaunches it.
  * A launch with no bisection to serve runs a kernel without the bisection
- * path, at three waves per SIMD (mixed, default lanes) when it starts with a
- * deep backlog; a launch starting from idle first gathers work for 0.2 ms,
- * and a bisection arriving during an image-only launch waits until that
- * launch has drained.  Work, descriptors and outputs pass through pinned
+ * path: four waves per 8x8 tile or, when it starts with a deep backlog, one
+ * (at three waves per SIMD: mixed, default lanes).  A launch starting from
+ * idle first gathers work for 0.2 ms; a bisection arriving during an
+ * image-only launch, and a deep backlog gathering behind a launch of four
+ * waves per tile, wait until that launch has drained.  Work, descriptors and outputs pass through pinned
  * host memory, and hbm_budget (default 1 GiB here) bounds the pinned output
  * staging.  The results are the same bits as the relaunched form's and
  * mk_render's.  Statistics of this form are updated when a launch ends. */
@@ -283,7 +284,7 @@ typedef struct mk_server_config {
 #define MK_SERVER_SHADOW_IN_LAUNCH 2
 /* mk_server_config.flags: images always run inside the server's launches.
  * Without it, an idle server whose queue holds one image of up to 512^2 and
- * nothing else renders it itself through mk_render (up to 256^2 three waves
+ * nothing else renders it itself through mk_render (up to 256^2 four waves
  * per tile).  The same image, bit for bit.  Above 256^2 that call builds
  * mk_render's tile order for the view, as mk_render's own first call does. */
 #define MK_SERVER_IMAGE_IN_LAUNCH 4

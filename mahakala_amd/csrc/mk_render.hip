@@ -26,6 +26,7 @@
 #include "mk_internal.h"
 #include "mk_render.h"
 #include "mk_snapshot.h"
+#include "mk_triple.h"
 
 namespace mk {
 
@@ -218,10 +219,8 @@ __global__ void __launch_bounds__(256, MIXED ? 3 : 2) k_render(SnapView sv, Rend
 // classic form.
 constexpr int kPairTiles = 4;   // tiles per workgroup (geodesic + transfer wave each)
 constexpr int kPairDepth = 4;   // ring slots per tile
-constexpr int kPairComp = 9;    // state[8], dt
 constexpr size_t kPairRingDoubles = (size_t)kPairTiles * kPairDepth * kPairComp * 64;
 constexpr size_t kPairLdsExtra = kPairRingDoubles * sizeof(double) + kPairTiles * 4 * sizeof(int);
-constexpr int kSpinLimit = 1 << 24;
 
 // Polls *cnt (LDS) until it reaches target; false after `limit` polls.
 __device__ __forceinline__ bool wait_at_least(int* cnt, int target, int limit) {
@@ -232,11 +231,6 @@ __device__ __forceinline__ bool wait_at_least(int* cnt, int target, int limit) {
     __builtin_amdgcn_s_sleep(1);
   }
   return false;
-}
-
-__device__ __forceinline__ void publish(int* cnt, int v) {
-  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
-  if ((threadIdx.x & 63) == 0) __hip_atomic_store(cnt, v, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_WORKGROUP);
 }
 
 template <bool MIXED>
@@ -396,91 +390,12 @@ __global__ void __launch_bounds__(128 * kPairTiles) k_render_pair(SnapView sv, R
   if (valid) img[p] = ok ? I : __builtin_nan("");
 }
 
-// ------------------------------------------------------------- triple form
-// Three stages per tile -- geodesic, gather (lookup, cell loads,
-// interpolation) and emission (fluid scalars, j and alpha, transfer) --
-// chained by two LDS rings with the counters of the paired form.  One tile is
-// one workgroup of four waves: a geodesic wave, two gather waves that take the
-// rounds in turn, and an emission wave.  A lone gather wave's round (ring
-// read, lookup, cell loads, interpolation: one latency after the other) takes
-// about 3300 cycles, a geodesic step 2200, so one gather wave set the pace.
-// The hardware puts a workgroup's four waves on the CU's four SIMDs and
-// rotates the order from workgroup to workgroup, so with four workgroups per
-// CU every SIMD holds one wave of each kind.  The block tables stay in global
-// memory (each gather wave keeps its rays' last block record in registers):
-// with 51 KB of them in LDS only two workgroups fit a CU, and where both fit
-// the times are equal.
-// 256^2, a = 0.9, i = 60 deg (a = 0.5, i = 30 deg): with four tiles and one
-// gather wave each per workgroup, tables in LDS, plain FP64 3.99 (2.08) ms,
-// mixed 3.38 (1.72) ms; with this split 3.48 (2.02) and 3.22 (1.57) ms; with
-// rays ending outside the domain and nothing handed over on their way in 3.14
-// (1.73) and 3.03 (1.46) ms.  160^2 at a = 0.9: plain 3.93 -> 2.70 ms, mixed 3.18 -> 2.65 ms.
-// Ring A carries (state, dt) from the geodesic wave, ring B the eight
-// interpolated primitives and the state in the emission's precision (FP32
-// values are what the FP32 emission would round them to) and dt in FP64 (0:
-// nothing to add).
-template <bool MIXED>
-struct TriRings {
-  using T = typename std::conditional<MIXED, float, double>::type;
-  static constexpr int kDepthA = 4, kDepthB = MIXED ? 4 : 2;  // rounds (35 KB: four workgroups fit 160 KB)
-  static constexpr int kCompB = 15;                           // P[8], s[1..7]
-  double a[kDepthA][kPairComp][64];
-  double bd[kDepthB][64];  // dt
-  T bt[kDepthB][kCompB][64];
-  int producedA, doneA, consumedB;
-  int consumedA[2], producedB[2], doneB[2];  // per gather wave
-};
-
-// Polls *cnt until it reaches target: the value read, or -1 after `limit`
-// polls.
-__device__ __forceinline__ int wait_value(int* cnt, int target, int limit) {
-  for (int spin = 0; spin < limit; ++spin) {
-    const int v = __builtin_amdgcn_readfirstlane(
-        __hip_atomic_load(cnt, __ATOMIC_ACQUIRE, __HIP_MEMORY_SCOPE_WORKGROUP));
-    if (v >= target) return v;
-    __builtin_amdgcn_s_sleep(1);
-  }
-  return -1;
-}
-
-// Waits for round t of a ring: 1 ready (*avail = rounds published), 0 the
-// writer finished after fewer rounds, -1 failure (the writer gave up, or
-// `limit` polls).
-__device__ __forceinline__ int wait_round(int* produced, int* done, int t, int* avail, int limit) {
-  for (int spin = 0; spin < limit; ++spin) {
-    const int pr = __builtin_amdgcn_readfirstlane(
-        __hip_atomic_load(produced, __ATOMIC_ACQUIRE, __HIP_MEMORY_SCOPE_WORKGROUP));
-    if (pr > t) {
-      *avail = pr;
-      return 1;
-    }
-    const int dn = __builtin_amdgcn_readfirstlane(
-        __hip_atomic_load(done, __ATOMIC_ACQUIRE, __HIP_MEMORY_SCOPE_WORKGROUP));
-    if (dn == -2) return -1;
-    if (dn >= 0 && t >= dn) return 0;
-    __builtin_amdgcn_s_sleep(1);
-  }
-  return -1;
-}
-
-// ZONE (mixed): the geodesic wave takes FP64 steps while any of its rays is in
-// the zone (rp.fp64_r, rp.ring_r), as the other forms do; without it the zone
-// code is compiled out.
+// ZONE: see tri_tile.
 template <bool MIXED, bool ZONE>
 __global__ void __launch_bounds__(256, 4) k_render_tri(SnapView sv, RenderDev rp, double* __restrict__ img,
                                                        int32_t* __restrict__ steps) {
-  using T = typename std::conditional<MIXED, float, double>::type;
-  using R = TriRings<MIXED>;
-  constexpr int DA = R::kDepthA, DB = R::kDepthB;
-  __shared__ R ring;
-  if (threadIdx.x == 0) {
-    ring.producedA = ring.consumedB = 0;
-    ring.doneA = -1;
-    for (int g = 0; g < 2; ++g) {
-      ring.consumedA[g] = ring.producedB[g] = 0;
-      ring.doneB[g] = -1;
-    }
-  }
+  __shared__ TriRings<MIXED> ring;
+  if (threadIdx.x == 0) ring.reset();
   __syncthreads();
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   // workgroups start in index order: with a tile order the longest tiles go
@@ -491,189 +406,11 @@ __global__ void __launch_bounds__(256, 4) k_render_tri(SnapView sv, RenderDev rp
   const int pi = (int)(tile / rp.tiles_x) * 8 + (lane >> 3), pj = (int)(tile % rp.tiles_x) * 8 + (lane & 7);
   const bool valid = pi < rp.res && pj < rp.res;
   const long p = (long)pi * rp.res + pj;
-  if (wave == 0) {  // geodesic
-    // A lane is alive while its dt is not 0; dead lanes step along with dt = 0
-    // and are ignored, so the loop has no branches per lane.  All live lanes
-    // have taken the same number of steps, k.
-    double s[8], r = 0.0, dt = 0.0, drdl = 1e300;
-    KsHead h{}, hn{};  // FP64: the position terms at s and at the candidate
-    int k = 0, nacc = 0;
-#pragma unroll
-    for (int q = 0; q < 8; ++q) s[q] = 0.0;
-    if (valid) {
-      double sx[4], sv4[4];
-      camera_ray(grid_coord(rp.lo, rp.step, pi), grid_coord(rp.lo, rp.step, pj), rp.ci, rp.si, rp.dist, sx, sv4);
-      nullify(sx, sv4, rp.a, s);
-      r = radius_cal(s[1], s[2], s[3], rp.a);
-      dt = step_rule(r, rp.rEH, rp.div, rp.tol);
-    }
-    if constexpr (!MIXED) h = ks_head(s[1], s[2], s[3], rp.a);
-    double lim = 1500.0;  // largest |r - r_EH| of a live ray
-    // one RK4 step of every live lane into nw (mixed may step in place: the
-    // step functions write their output only after reading the state)
-    auto step = [&](double nw[8]) {
-      if constexpr (!MIXED) {
-        rk4_step64(s, h, dt, rp.a, nw);
-      } else {
-        const bool fp64 = ZONE && __any(dt != 0.0 && ((r < rp.fp64_r) || (r < rp.ring_r && __builtin_fabs(drdl) < rp.ring_drdl)));
-        if (fp64) rk4_step<double>(s, dt, rp.a, nw);
-        else rk4_step_mixed(s, dt, (float)rp.a, nw);
-      }
-    };
-    // radius and step of the candidate; 0 ends the ray
-    auto rule = [&](const double nw[8], double& rn) {
-      double dtn;
-      if constexpr (!MIXED) {
-        hn = ks_head(nw[1], nw[2], nw[3], rp.a);
-        rn = hn.r;
-        dtn = step_rule(rn, rp.rEH, rp.div, rp.tol, lim);
-      } else {
-        rn = radius_f32(nw[1], nw[2], nw[3], rp.a);
-        dtn = step_rule_fast(rn, rp.rEH, rp.inv_div, rp.div, rp.tol, lim);
-      }
-      return dt != 0.0 ? dtn : 0.0;
-    };
-    // The way in: no ray of the tile is inside the sphere around the domain,
-    // so the steps are taken without handing anything over.  The step that
-    // first takes a ray inside is left to the loop below.
-    double nw_[8];
-    while (k < rp.N && __any(dt != 0.0)) {
-      double rn;
-      step(nw_);
-      const double dtn = rule(nw_, rn);
-      if (__any(dtn != 0.0 && rn <= rp.r_dom)) break;
-      nacc += dtn != 0.0;
-      if (ZONE) drdl = (rn - r) / dt;
-#pragma unroll
-      for (int q = 0; q < 8; ++q) s[q] = nw_[q];
-      dt = dtn;
-      r = rn;
-      h = hn;
-      ++k;
-    }
-    // A ray inside the sphere of radius r_out ends when it leaves it again.
-    if (r < rp.r_out) lim = __builtin_fmin(1500.0, rp.r_out - rp.rEH);
-    bool ok = true;
-    int t = 0;  // the next round
-    for (; k < rp.N && __any(dt != 0.0); ++k, ++t) {
-      // Slot t % DA is free once round t - DA has been read.  That count is
-      // loaded here without waiting and checked after the RK4 step: a wait at
-      // the loop head would also wait on this wave's slot writes of the round
-      // before (-2 to -4 % in FP64, -1 % in mixed).
-      int* readA = &ring.consumedA[t & 1];
-      const int polled = __hip_atomic_load(readA, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
-      double* out = &ring.a[t % DA][0][lane];
-      double* nw = MIXED ? s : nw_;  // mixed in place: -1.3 %; in FP64 the copy is faster
-      step(nw);
-      // release the previous round here: its slot writes were issued a whole
-      // RK4 step ago, so the release fence does not wait on them
-      if (t > 0) publish(&ring.producedA, t);
-      if (__builtin_amdgcn_readfirstlane(polled) > t - DA) {
-        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
-      } else if (wait_value(readA, t - DA + 1, rp.spin_limit) < 0) {
-        ok = false;
-        break;
-      }
-      double rn;
-      const double dtn = rule(nw, rn);
-      nacc += dtn != 0.0;
-#pragma unroll
-      for (int q = 0; q < 8; ++q) out[q * 64] = nw[q];
-      out[8 * 64] = dtn != 0.0 && k + 1 < rp.N ? dt : 0.0;  // row N is never emitted
-      if (ZONE) drdl = (rn - r) / dt;
-      if constexpr (!MIXED) {
-#pragma unroll
-        for (int q = 0; q < 8; ++q) s[q] = nw[q];
-      }
-      dt = dtn;
-      r = rn;
-      h = hn;
-    }
-    if (ok) publish(&ring.producedA, t);
-    publish(&ring.doneA, ok ? t : -2);
-    if (valid && steps) steps[p] = ok ? nacc : -1;
-    return;
-  }
-  if (wave <= 2) {  // gather: lookup, cell loads, interpolation of every other round
-    const int g = wave - 1;
-    bool ok = true;
-    int avail = 0, freed = 0;  // rounds of ring A published, of ring B read (last values seen)
-    int cmb = -1;              // block of the ray's last sample and its record
-    double crec[kMeta];
-    int t = g;
-    for (;; t += 2) {
-      if (t >= avail) {
-        const int st = wait_round(&ring.producedA, &ring.doneA, t, &avail, rp.spin_limit);
-        if (st <= 0) {
-          ok = st == 0;
-          break;
-        }
-      }
-      if (t - DB + 1 > freed) {
-        freed = wait_value(&ring.consumedB, t - DB + 1, rp.spin_limit);
-        if (freed < 0) {
-          ok = false;
-          break;
-        }
-      }
-      const double* in = &ring.a[t % DA][0][lane];
-      double pdt = in[8 * 64];
-      double ps[8];
-#pragma unroll
-      for (int q = 0; q < 8; ++q) ps[q] = in[q * 64];
-      publish(&ring.consumedA[g], t + 1);  // ring A slot is in registers
-      T* ob = &ring.bt[t % DB][0][lane];
-      T P[8];
-#pragma unroll
-      for (int q = 0; q < 8; ++q) P[q] = T(0);
-      if (pdt != 0.0) {
-        const Stencil stc = locate_cached(sv, sv.meta, sv.grid, ps[1], ps[2], ps[3], cmb, crec);
-        if (stc.mb >= 0) {
-          Corners cr;
-          fetch<false>(sv, stc, cr);
-          interp<T>(stc, cr, P);
-        }
-        if (stc.mb < 0 || P[0] == T(0)) pdt = 0.0;  // adds exactly nothing
-      }
-#pragma unroll
-      for (int q = 0; q < 8; ++q) ob[q * 64] = P[q];
-#pragma unroll
-      for (int q = 1; q < 8; ++q) ob[(7 + q) * 64] = (T)ps[q];
-      ring.bd[t % DB][lane] = pdt;
-      publish(&ring.producedB[g], t + 1);
-    }
-    publish(&ring.doneB[g], ok ? t : -2);
-    return;
-  }
-  // emission and transfer, in step order
-  double I = 0.0, trans = 1.0;
-  bool ok = true;
-  for (int t = 0;; ++t) {
-    int avail = 0;
-    const int st = wait_round(&ring.producedB[t & 1], &ring.doneB[t & 1], t, &avail, rp.spin_limit);
-    if (st <= 0) {
-      ok = st == 0;
-      break;
-    }
-    const T* ib = &ring.bt[t % DB][0][lane];
-    const double pdt = ring.bd[t % DB][lane];
-    T P[8];
-    double ps[8];
-#pragma unroll
-    for (int q = 0; q < 8; ++q) P[q] = ib[q * 64];
-    ps[0] = 0.0;
-#pragma unroll
-    for (int q = 1; q < 8; ++q) ps[q] = (double)ib[(7 + q) * 64];
-    publish(&ring.consumedB, t + 1);  // ring B slot is in registers
-    if (pdt != 0.0) {
-      T j, al;
-      emission_from_prims<T>(rp.ip, P, ps, rp.a, j, al);
-      const double cc = -pdt * rp.ip.L_unit;
-      I += trans * (cc * (double)j);
-      trans *= (1.0 - cc * (double)al);
-    }
-  }
-  if (valid) img[p] = ok ? I : __builtin_nan("");
+  TriOut o;
+  tri_tile<MIXED, ZONE>(ring, wave, sv, rp, rp.spin_limit, grid_coord(rp.lo, rp.step, pi),
+                        grid_coord(rp.lo, rp.step, pj), valid, o);
+  if (valid && wave == 0 && steps) steps[p] = o.steps;
+  if (valid && wave == 3) img[p] = o.I;
 }
 
 // Critical curve of a distant camera at inclination theta (Bardeen 1973):

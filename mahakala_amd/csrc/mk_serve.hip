@@ -34,6 +34,7 @@
 #include "mk_internal.h"
 #include "mk_render.h"
 #include "mk_snapshot.h"
+#include "mk_triple.h"
 
 namespace mk {
 
@@ -637,6 +638,87 @@ __global__ void __launch_bounds__(256, (MIXED && !SHADOW) ? 3 : 2)
   }
 }
 
+// The same protocol for a launch of image requests without a deep backlog:
+// each workgroup takes a ticket and runs the tile with its four waves in the
+// render kernel's triple form: a step takes about half the time it takes a
+// wave that does all three stages, and four workgroups per CU hold as many
+// tiles as four such waves would.  A chip with a deep backlog does better with
+// the other kernel (the gather and emission waves of a tile idle while its
+// geodesic wave is the slower), so a launch runs this one only without it.
+// 16 mixed images of 64^2-256^2 submitted together: 12.6 -> 10.0 ms; 1000 mixed images of 64^2-512^2 arriving at 200 per second:
+// p50 7.0 -> 3.7 ms, p99 16.1 -> 10.8 ms; a lone 256^2 image inside the
+// launch 5.4 -> 3.5 ms; 256 queued requests of 512^2 and 4096 angles (the
+// other kernel) unchanged.
+template <bool MIXED>
+__global__ void __launch_bounds__(256, 4) k_serve_tri(const ReqDev* __restrict__ req, PArgs P) {
+  __shared__ TriRings<MIXED> ring;
+  __shared__ int s_state, s_tile, s_rid, s_seq, s_desc;
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  int cursor = 0;
+  while (true) {
+    if (wave == 0) {
+      unsigned long long tk = 0;
+      if (lane == 0) tk = __hip_atomic_fetch_add(P.taken, 1ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      const long long t = bcast64((long long)tk);
+      int state = wait_published(P, t), err = state < 0 ? 3 : 0;
+      PSeg sg{};
+      if (state > 0 && !find_segment(P, t, cursor, sg)) {
+        state = -1;
+        err = 1;
+      }
+      if (lane == 0) {
+        if (err) __hip_atomic_store(&P.ctl->err, err, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+        s_state = state;
+        s_tile = (int)(t - sg.start);
+        s_rid = sg.rid;
+        s_seq = sg.seq;
+        s_desc = sg.desc;
+        ring.reset();
+      }
+    }
+    __syncthreads();
+    if (__builtin_amdgcn_readfirstlane(s_state) <= 0) break;
+    const int tile = __builtin_amdgcn_readfirstlane(s_tile), rid = __builtin_amdgcn_readfirstlane(s_rid);
+    const ReqDev& q = req[__builtin_amdgcn_readfirstlane(s_desc)];
+    const int item = tile * kTile + lane;
+    if (q.kind == kKindImage) {
+      const bool live = item < q.n_items;
+      // the tile order lives in host memory: read once per tile, by the waves that need the pixel
+      const int px = live && (wave == 0 || wave == 3) ? pixel_of_item(q, item) : 0;
+      TriOut o;
+      tri_tile<MIXED, false>(ring, wave, q.sv, q, kSpinLimit, grid_coord(q.lo, q.step, px / q.res),
+                             grid_coord(q.lo, q.step, px % q.res), live, o);
+      if (wave == 0) {
+        unsigned long long w = (unsigned long long)(live && o.steps > 0 ? o.steps : 0);
+        for (int off = 32; off > 0; off >>= 1) w += __shfl_xor(w, off);
+        if (lane == 0) {
+          atomicAdd(P.busy, w);
+          atomicAdd(P.total, 64ull * (unsigned long long)o.rounds);
+        }
+      }
+      if (wave == 3) {
+        if (live) q.out[px] = o.I;
+        if (!o.ok && lane == 0) __hip_atomic_store(&P.ctl->err, 5, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+      }
+    } else if (threadIdx.x == 0) {  // the host publishes no bisection to this launch
+      __hip_atomic_store(&P.ctl->err, 4, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+    }
+    if (wave == 3) {  // as in k_serve_persistent: the outputs, then the count, then the flag
+      __builtin_amdgcn_fence(__ATOMIC_RELEASE, "");
+      if (lane == 0) {
+        const int n = min(kTile, q.n_items - tile * kTile);
+        const int old = __hip_atomic_fetch_add(&P.done[rid], n, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        if (old + n >= q.n_items) {
+          __hip_atomic_store(&P.done[rid], 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+          __builtin_amdgcn_fence(__ATOMIC_RELEASE, "");
+          __hip_atomic_store(&P.fin[rid], s_seq + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+        }
+      }
+    }
+    __syncthreads();  // every wave has left the tile before its rings are reset
+  }
+}
+
 __global__ void k_set_pair(unsigned long long* p, unsigned long long a, unsigned long long b) {
   if (blockIdx.x == 0 && threadIdx.x == 0) {
     p[0] = a;
@@ -723,6 +805,8 @@ struct mk_server {
   bool default_lanes = true;         // lanes not set by the caller: two waves per SIMD
   bool launch_shadow = false;        // the running launch serves bisections too
   bool launch_deep = false;          // the next launch starts with a deep backlog
+  bool launch_tri = false;           // the running (or last) launch runs four waves per tile
+  bool want_deep = false;            // a deep backlog has gathered behind such a launch
   bool want_shadow = false;          // a bisection waits for a launch that serves it
   std::chrono::steady_clock::time_point launch_t0;
   std::map<std::pair<int, double>, std::vector<int>> orders;  // tile orders by (resolution, fov)
@@ -1049,7 +1133,7 @@ bool collect(mk_server* s) {
 // at the head of its queue itself: a bisection of up to 1024 angles in
 // mk_shadow_bisect's band schedule (about one integration chain where the
 // server's launches take one per halving), and, when it is the only request
-// queued, an image of up to 512^2 through mk_render (three waves per 8x8 tile
+// queued, an image of up to 512^2 through mk_render (four waves per 8x8 tile
 // up to 256^2, with row-major tiles, which at one tile per SIMD cost nothing;
 // above, mk_render's ring-first tile order, built once per view and kept).
 // The same results, bit for bit.  (Caller holds mu.)
@@ -1176,8 +1260,24 @@ T load_shared(const T* p) {
 // (caller holds mu).  A request whose tables or descriptor would not fit the
 // launch's fresh memory starts a drain: nothing more is admitted until every
 // request in flight has finished and the launch has ended.
+// A launch of four waves per tile ends, once what it holds is done, when this
+// many times the deep backlog (kDeepTilesPerWave) has gathered.
+constexpr int kDeepRelaunch = 4;
+
+// Work items queued or in flight (caller holds mu).
+long long backlog_items(const mk_server* s) {
+  long long items = 0;
+  for (const auto& kv : s->flight) items += kv.second.n_items;
+  for (const auto& p : s->waiting)
+    items += p.kind == kKindImage ? (long long)p.img.resolution * p.img.resolution : p.sh.n_angles;
+  return items;
+}
+
 void admit_persistent(mk_server* s) {
   if (s->launched && s->stopping) return;  // the waves may be leaving: nothing is published until the launch ends
+  if (s->launched && s->launch_tri && !s->want_deep && !s->waiting.empty())
+    s->want_deep = backlog_items(s) >= (long long)kDeepRelaunch * kDeepTilesPerWave * s->L;
+  if (s->launched && s->want_deep) return;  // the next launch takes the queue
   bool any = false;
   while (!s->draining && !s->waiting.empty() && !s->free_rids.empty()) {
     mk_server::Pending& p = s->waiting.front();
@@ -1293,13 +1393,20 @@ bool launch_persistent(mk_server* s) {
   // per SIMD, for throughput; otherwise two, each wave faster, for latency
   unsigned blocks = (unsigned)((s->L + 255) / 256);
   if (s->cfg.precision == 1 && !shadow && s->default_lanes && s->launch_deep) blocks = blocks * 3 / 2;
+  // images without such a backlog: four waves per tile
+  s->launch_tri = !shadow && !s->launch_deep;
+  s->want_deep = false;
+  if (s->launch_tri) blocks *= 2;  // four waves per SIMD at the default lanes
   // tickets below resume_ticket are done; the previous launch's waves left
   // holding tickets from it on, unpublished then
   k_set_pair<<<1, 64, 0, s->stream>>>(s->d_p, (unsigned long long)s->resume_ticket,
                                       (unsigned long long)s->resume_ticket);
   SRV_HIP_UNLOCKED(hipGetLastError());
   SRV_HIP_UNLOCKED(hipEventRecord(s->ev0, s->stream));
-  if (s->cfg.precision == 0) {
+  if (s->launch_tri) {
+    if (s->cfg.precision == 0) k_serve_tri<false><<<blocks, 256, 0, s->stream>>>(s->p_desc, P);
+    else k_serve_tri<true><<<blocks, 256, 0, s->stream>>>(s->p_desc, P);
+  } else if (s->cfg.precision == 0) {
     if (shadow) k_serve_persistent<false, true><<<blocks, 256, 0, s->stream>>>(s->p_desc, P);
     else k_serve_persistent<false, false><<<blocks, 256, 0, s->stream>>>(s->p_desc, P);
   } else {
@@ -1365,6 +1472,7 @@ void worker_persistent(mk_server* s) {
       s->status = MK_ERR_STATE;
       s->err = ec == 1   ? "persistent launch: a ticket without a published segment"
                : ec == 4 ? "persistent launch: a bisection reached a launch without the bisection path"
+               : ec == 5 ? "persistent launch: a wave waited longer than its limit for the other waves of its tile"
                          : "persistent launch: a wave waited longer than its limit for work";
       break;
     }
@@ -1390,16 +1498,13 @@ void worker_persistent(mk_server* s) {
       last_busy = now;
     }
     if (s->launched && s->flight.empty() &&
-        (s->want_shadow || (s->waiting.empty() && now - last_busy > std::chrono::milliseconds(kPersistIdleMs)) ||
+        (s->want_shadow || s->want_deep ||
+         (s->waiting.empty() && now - last_busy > std::chrono::milliseconds(kPersistIdleMs)) ||
          now - s->launch_t0 > std::chrono::milliseconds(kPersistMaxAgeMs))) {
       stop_persistent(s);  // nothing in flight: the next request relaunches
     }
     if (!s->launched && !s->flight.empty()) {
-      long long items = 0;  // queued or in flight, counted here under mu
-      for (const auto& kv : s->flight) items += kv.second.n_items;
-      for (const auto& p : s->waiting)
-        items += p.kind == kKindImage ? (long long)p.img.resolution * p.img.resolution : p.sh.n_angles;
-      s->launch_deep = items >= (long long)kDeepTilesPerWave * s->L;
+      s->launch_deep = backlog_items(s) >= (long long)kDeepTilesPerWave * s->L;  // under mu
       if (!ready) {
         ready = true;
         ready_since = now;

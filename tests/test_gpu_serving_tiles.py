@@ -1,0 +1,64 @@
+"""Image-only launches of the persistent server: four waves per tile, or one
+wave per tile when the launch starts with a deep backlog (images.py:30-144 of
+the reference).  Both give mk_render's bits, whatever the tile count."""
+import time
+
+import numpy as np
+import pytest
+
+from mahakala_amd import images
+from mahakala_amd.grmhd import synthetic as syn
+from mahakala_amd.grmhd.athenak import AthenakFluidModel
+from mahakala_amd.serving import Server
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def model():
+    return AthenakFluidModel.from_datasets(syn.uniform_torus_snapshot(0.9, seed=0), 0.9, fluid_gamma=13. / 9)
+
+
+def _render(model, view, precision):
+    p = images.render_params(0.9, camera_inclination=view["inclination"], resolution=view["resolution"], fov=20,
+                             observing_frequency=230e9, max_nsteps=view["max_nsteps"], precision=precision)
+    return images.render(model.device_snapshot, p)
+
+
+def _submit(srv, sid, view):
+    return srv.submit_image(sid, bhspin=0.9, observing_frequency=230e9, fov=20, **view)
+
+
+@pytest.mark.parametrize("precision", ["plain64", "mixed"])
+def test_tiles_of_any_count_and_step_limit(model, precision):
+    views = [dict(resolution=r, inclination=i, max_nsteps=n)
+             for r, i, n in [(1, 30.0, 10000), (7, 60.0, 10000), (8, 60.0, 10000), (9, 85.0, 300), (36, 10.0, 1),
+                             (64, 75.0, 10000), (65, 5.0, 90)]]
+    with Server(precision, lanes=1024, image_in_launch=True) as srv:
+        sid = srv.add_snapshot(model)
+        for _ in range(2):  # the second pass reuses the request slots
+            rids = [_submit(srv, sid, v) for v in views]
+            for v, rid in zip(views, rids):
+                np.testing.assert_array_equal(srv.result(rid, timeout=60), _render(model, v, precision), err_msg=str(v))
+
+
+@pytest.mark.parametrize("precision", ["plain64", "mixed"])
+def test_deep_backlog_behind_a_shallow_launch(model, precision):
+    """At 2048 lanes 8192 items make a launch start deep and 32768 end a
+    shallow one: 48^2 starts shallow, 12 images of 64^2 follow it."""
+    first = dict(resolution=48, inclination=60.0, max_nsteps=10000)
+    later = [dict(resolution=64, inclination=5.0 + 6 * k, max_nsteps=10000) for k in range(12)]
+    with Server(precision, lanes=2048, image_in_launch=True) as srv:
+        sid = srv.add_snapshot(model)
+        rids = [_submit(srv, sid, first)]
+        t_wait = time.perf_counter() + 30.0
+        while srv.stats()["iterations"] < 1:
+            assert time.perf_counter() < t_wait, "the first launch did not start"
+            time.sleep(0.0005)
+        rids += [_submit(srv, sid, v) for v in later]
+        got = [srv.result(r, timeout=60) for r in rids]
+        time.sleep(0.1)  # longer than the idle limit: the launch ends
+        st = srv.stats()
+    assert st["completed"] == 13 and st["in_flight"] == 0 and st["iterations"] >= 2
+    for v, img in zip([first] + later, got):
+        np.testing.assert_array_equal(img, _render(model, v, precision), err_msg=str(v))
