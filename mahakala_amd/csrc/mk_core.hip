@@ -118,53 +118,63 @@ struct WalkOut {
   double sel_r;
 };
 
-__device__ __forceinline__ void walk_ray(const double s0[8], int N, double div, double tol, double a, double rEH,
-                                         WalkOut& o) {
-  double s[8], nw[8];
+// Lanes whose ray has ended, and those without one (not live), step along with
+// dt = 0 until the last ray of the wave has ended, and what a ray leaves is
+// saved as it ends.  FP64 with lanes switched off takes longer: with one lane on
+// a step takes 1.0-1.4 us where 64 take 0.965, with a few lanes on in each of 64
+// waves 1.2.  The loop stands there twice, from buffer a to b and back, for
+// want of register copies.
+__device__ __forceinline__ void walk_ray(const double s0[8], bool live, int N, double div, double tol, double a,
+                                         double rEH, WalkOut& o) {
+  double sa[8], sb[8];
 #pragma unroll
-  for (int k = 0; k < 8; ++k) s[k] = s0[k];
-  double r = radius_cal(s[1], s[2], s[3], a);
-  double dt = step_rule(r, rEH, div, tol);
-  KsHead h = ks_head(s[1], s[2], s[3], a), hn = h;
-  double best = -__builtin_inf(), r_prev = __builtin_nan(""), r_at = __builtin_nan("");
-  int besti = -1, K = N;
-  for (int n = 0; n < N; ++n) {
-    bool frozen = (dt == 0.0);
-    double rn = 0.0, dtn = 0.0;
-    if (!frozen) {
-      rk4_step64(s, h, dt, a, nw);
-      hn = ks_head(nw[1], nw[2], nw[3], a);
-      rn = hn.r;
-      dtn = step_rule(rn, rEH, div, tol);
-      frozen = (dtn == 0.0);
+  for (int k = 0; k < 8; ++k) o.last[k] = sa[k] = s0[k];
+  double ra = radius_cal(sa[1], sa[2], sa[3], a), rb = __builtin_nan(""), r_end = ra;
+  double dta = live ? step_rule(ra, rEH, div, tol) : 0.0, dtb = 0.0;
+  KsHead ha = ks_head(sa[1], sa[2], sa[3], a), hb;
+  double best = -__builtin_inf(), r_at = __builtin_nan("");
+  int besti = -1, n = 0;
+  o.K = dta == 0.0 ? 0 : N;
+  // row n at (s, r, dt), the radius of row n - 1 in rn; row n + 1 to (nw, rn, dtn)
+  auto row = [&](const double s[8], const KsHead& h, double r, double dt, double nw[8], KsHead& hn, double& rn,
+                 double& dtn) {
+    const double r_prev = rn;
+    rk4_step64(s, h, dt, a, nw);
+    hn = ks_head(nw[1], nw[2], nw[3], a);
+    rn = hn.r;
+    dtn = step_rule(rn, rEH, div, tol);
+    dtn = dt != 0.0 ? dtn : 0.0;
+    const double row_dt = dtn != 0.0 ? dt : 0.0;
+    const bool up = row_dt > best;
+    best = up ? row_dt : best;
+    besti = up ? n : besti;
+    r_at = up ? r_prev : r_at;
+    if (dt != 0.0 && (dtn == 0.0 || n == N - 1)) {  // the ray's last row
+      if (dtn == 0.0) o.K = n;
+      r_end = r;
+#pragma unroll
+      for (int k = 0; k < 8; ++k) o.last[k] = s[k];
     }
-    const double row_dt = frozen ? 0.0 : dt;
-    if (row_dt > best) { best = row_dt; besti = n; r_at = r_prev; }
-    if (frozen) { K = n; break; }
-    r_prev = r;
-    if (n == N - 1) break;
-#pragma unroll
-    for (int k = 0; k < 8; ++k) s[k] = nw[k];
-    dt = dtn;
-    r = rn;
-    h = hn;
+    ++n;
+  };
+  while (n < N && __any(dta != 0.0)) {
+    row(sa, ha, ra, dta, sb, hb, rb, dtb);
+    if (!(n < N && __any(dtb != 0.0))) break;
+    row(sb, hb, rb, dtb, sa, ha, ra, dta);
   }
-  o.K = K;
-#pragma unroll
-  for (int k = 0; k < 8; ++k) o.last[k] = s[k];
-  o.sel_r = (besti >= 1) ? r_at : r;
+  o.sel_r = (besti >= 1) ? r_at : r_end;
 }
 
 __global__ void __launch_bounds__(256) k_integrate_final(const double* s0, long n, int N, double div, double tol,
                                                          double a, double rEH, int32_t* K, double* last,
                                                          double* sel) {
-  const long p = (long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (p >= n) return;
+  const long p = (long)blockIdx.x * blockDim.x + threadIdx.x, q = p < n ? p : n - 1;
   double st[8];
 #pragma unroll
-  for (int k = 0; k < 8; ++k) st[k] = s0[8 * p + k];
+  for (int k = 0; k < 8; ++k) st[k] = s0[8 * q + k];
   WalkOut o;
-  walk_ray(st, N, div, tol, a, rEH, o);
+  walk_ray(st, p < n, N, div, tol, a, rEH, o);
+  if (p >= n) return;
   if (K) K[p] = o.K;
   if (last)
 #pragma unroll
@@ -182,38 +192,58 @@ __global__ void k_max_K(const int32_t* K, long n, int N, int* out /* [0] max K, 
 
 __global__ void __launch_bounds__(256) k_integrate_history(const double* s0, long n, double div, double tol, double a,
                                                            double rEH, long T, double* S, double* D) {
-  const long p = (long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (p >= n) return;
-  double s[8], nw[8];
+  const long p = (long)blockIdx.x * blockDim.x + threadIdx.x, q = p < n ? p : n - 1;
+  const bool live = p < n;
+  double sa[8], sb[8];
 #pragma unroll
-  for (int k = 0; k < 8; ++k) s[k] = s0[8 * p + k];
-  double dt = step_rule(radius_cal(s[1], s[2], s[3], a), rEH, div, tol);
-  KsHead h = ks_head(s[1], s[2], s[3], a), hn = h;
-  bool frozen = false;
-  for (long row = 0; row < T; ++row) {
-    double edt = 0.0, dtn = 0.0;
-    if (!frozen) {
-      if (dt == 0.0) {
-        frozen = true;
-      } else {
-        rk4_step64(s, h, dt, a, nw);
-        hn = ks_head(nw[1], nw[2], nw[3], a);
-        dtn = step_rule(hn.r, rEH, div, tol);
-        if (dtn == 0.0) frozen = true;
-        else edt = dt;
-      }
+  for (int k = 0; k < 8; ++k) sa[k] = s0[8 * q + k];
+  double dta = step_rule(radius_cal(sa[1], sa[2], sa[3], a), rEH, div, tol), dtb = 0.0;
+  if (!live) dta = 0.0;
+  KsHead ha = ks_head(sa[1], sa[2], sa[3], a), hb;
+  long row = 0;
+  auto put = [&](const double s[8], double edt) {
+    if (live) {
+      double* out = S + 8 * (row * n + p);
+#pragma unroll
+      for (int k = 0; k < 8; ++k) out[k] = s[k];
+      D[row * n + p] = edt;
     }
-    double* out = S + 8 * (row * n + p);
+    ++row;
+  };
+  // writes the row at (s, h, dt) and steps to the next, (nw, hn, dtn)
+  auto step = [&](const double s[8], const KsHead& h, double dt, double nw[8], KsHead& hn, double& dtn) {
+    rk4_step64(s, h, dt, a, nw);
+    hn = ks_head(nw[1], nw[2], nw[3], a);
+    dtn = step_rule(hn.r, rEH, div, tol);
+    dtn = dt != 0.0 ? dtn : 0.0;
+    put(s, dtn != 0.0 ? dt : 0.0);
+    if (dtn == 0.0) {  // the ray has ended: its last row repeats
 #pragma unroll
-    for (int k = 0; k < 8; ++k) out[k] = s[k];
-    D[row * n + p] = edt;
-    if (!frozen) {
-#pragma unroll
-      for (int k = 0; k < 8; ++k) s[k] = nw[k];
-      dt = dtn;
-      h = hn;
+      for (int k = 0; k < 8; ++k) nw[k] = s[k];
     }
+  };
+  while (row < T && __any(dta != 0.0)) {
+    step(sa, ha, dta, sb, hb, dtb);
+    if (!(row < T && __any(dtb != 0.0))) {
+#pragma unroll
+      for (int k = 0; k < 8; ++k) sa[k] = sb[k];
+      break;
+    }
+    step(sb, hb, dtb, sa, ha, dta);
   }
+  while (row < T) put(sa, 0.0);
+}
+
+// The final radius of the ray at image point (x, y); lanes without one pass any
+// point and live = false.
+__device__ __forceinline__ double final_radius(double x, double y, bool live, double ci, double si, double d, int N,
+                                               double a, double rEH) {
+  double sx[4], sv[4], st[8];
+  camera_ray(x, y, ci, si, d, sx, sv);
+  nullify(sx, sv, a, st);
+  WalkOut o;
+  walk_ray(st, live, N, 40.0, 1e-2, a, rEH, o);
+  return o.sel_r;
 }
 
 // select_photons_integrator at (x, y) image points, and the bisection that
@@ -221,33 +251,23 @@ __global__ void __launch_bounds__(256) k_integrate_history(const double* s0, lon
 // each lane runs its own angle for the fixed number of halvings.
 __global__ void __launch_bounds__(256) k_select(double a, double ci, double si, double d, const double* px,
                                                 const double* py, long n, int N, double rEH, double* out) {
-  const long p = (long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (p >= n) return;
-  double sx[4], sv[4], st[8];
-  camera_ray(px[p], py[p], ci, si, d, sx, sv);
-  nullify(sx, sv, a, st);
-  WalkOut o;
-  walk_ray(st, N, 40.0, 1e-2, a, rEH, o);
-  out[p] = o.sel_r;
+  const long p = (long)blockIdx.x * blockDim.x + threadIdx.x, q = p < n ? p : n - 1;
+  const double r = final_radius(px[q], py[q], p < n, ci, si, d, N, a, rEH);
+  if (p < n) out[p] = r;
 }
 
 __global__ void __launch_bounds__(256) k_bisect(double a, double ci, double si, double d, const double* cang,
                                                 const double* sang, long n, int N, int iters, double rEH,
                                                 double* radii) {
-  const long p = (long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (p >= n) return;
+  const long p = (long)blockIdx.x * blockDim.x + threadIdx.x, q = p < n ? p : n - 1;
+  const double ca = cang[q], sa = sang[q];
   double inner = 0.5, outer = 10.0;
   for (int it = 0; it < iters; ++it) {
     const double mid = (outer - inner) / 2 + inner;
-    double sx[4], sv[4], st[8];
-    camera_ray(cang[p] * mid, sang[p] * mid, ci, si, d, sx, sv);
-    nullify(sx, sv, a, st);
-    WalkOut o;
-    walk_ray(st, N, 40.0, 1e-2, a, rEH, o);
-    if (o.sel_r < 100.0) inner = mid;
+    if (final_radius(ca * mid, sa * mid, p < n, ci, si, d, N, a, rEH) < 100.0) inner = mid;
     else outer = mid;
   }
-  radii[p] = inner;
+  if (p < n) radii[p] = inner;
 }
 
 // The same bisection, K halvings per round: each angle's group of 2^K lanes
@@ -273,10 +293,11 @@ __global__ void __launch_bounds__(1024) k_bisect_tree(double a, double ci, doubl
   for (int done = 0; done < iters;) {
     const int kr = min(K, iters - done);
     int c = 0;
-    if (p < n && j < (1 << kr) - 1) {
+    const bool live = p < n && j < (1 << kr) - 1;
+    if (__any(live)) {
       // node j (heap order): the bits of j + 1 below its leading one are the
       // path from the root, 1 = the ray fell in (inner = mid)
-      const int m = j + 1, depth = 31 - __builtin_clz(m);
+      const int m = live ? j + 1 : 1, depth = 31 - __builtin_clz(m);
       double lo = br[2 * g], hi = br[2 * g + 1];
       double mid = (hi - lo) / 2 + lo;
       for (int b = depth - 1; b >= 0; --b) {
@@ -284,12 +305,8 @@ __global__ void __launch_bounds__(1024) k_bisect_tree(double a, double ci, doubl
         else hi = mid;
         mid = (hi - lo) / 2 + lo;
       }
-      double sx[4], sv[4], st[8];
-      camera_ray(cang[p] * mid, sang[p] * mid, ci, si, d, sx, sv);
-      nullify(sx, sv, a, st);
-      WalkOut o;
-      walk_ray(st, N, 40.0, 1e-2, a, rEH, o);
-      c = o.sel_r < 100.0 ? 1 : 0;
+      const long q = p < n ? p : n - 1;
+      c = final_radius(cang[q] * mid, sang[q] * mid, live, ci, si, d, N, a, rEH) < 100.0 ? 1 : 0;
     }
     cls[threadIdx.x] = c;
     __syncthreads();
@@ -326,28 +343,30 @@ __device__ __forceinline__ long long band_range(double rho, double e, int l, lon
     return 0;
   }
   const long long nb = 1ll << l;
-  const double w = 9.5 / (double)nb;
-  b0 = (long long)__builtin_floor((rho - e - 0.5) / w);
-  long long b1 = (long long)__builtin_floor((rho + e - 0.5) / w);
+  const double per_w = (double)nb * (1.0 / 9.5);
+  b0 = (long long)__builtin_floor((rho - e - 0.5) * per_w);
+  long long b1 = (long long)__builtin_floor((rho + e - 0.5) * per_w);
   if (b0 < 0) b0 = 0;
   if (b1 > nb - 1) b1 = nb - 1;
   return b1 >= b0 ? b1 - b0 + 1 : 0;
 }
 constexpr int kBandMaxLevels = 48;
 
-// Midpoints in the band over levels [0, L).
-__device__ __forceinline__ long long band_nodes(double rho, double e, int L) {
+// Midpoints in the band over levels [0, L), B + 1 for more than B.
+template <int B>
+__device__ __forceinline__ int band_nodes(double rho, double e, int L) {
   long long t = 0, b0;
-  for (int l = 0; l < L; ++l) t += band_range(rho, e, l, b0);
-  return t;
+  for (int l = 0; l < L && t <= B; ++l) t += band_range(rho, e, l, b0);
+  return t <= B ? (int)t : B + 1;
 }
 
 // The bisection in fewer rounds, guided by a predicted radius per angle
 // (radii[p] on entry, NaN for none): each angle's B lanes first integrate, in
 // one round, every midpoint whose bracket meets a band about the prediction:
-// the widest band of half-width up to e whose midpoints of every level fit
-// in B lanes with one angle per block (several angles per block: the band
-// of half-width e over as many levels as fit).
+// with `narrow` the widest band of half-width up to e whose midpoints of every
+// level fit in B lanes (one round where the prediction holds), otherwise the
+// band of half-width e over as many levels as fit (two rounds, also where the
+// prediction is off).
 // One lane then replays the halvings from the classifications while the path
 // stays in the band; the halvings left (path out of the band, or levels
 // beyond it) run in tree rounds as in k_bisect_tree.  Every midpoint is
@@ -359,7 +378,7 @@ __device__ __forceinline__ long long band_nodes(double rho, double e, int L) {
 template <int B, int G>
 __global__ void __launch_bounds__(B * G) k_bisect_band(double a, double ci, double si, double d, const double* cang,
                                                        const double* sang, long n, int N, int iters, double rEH,
-                                                       double e, double* radii) {
+                                                       double e, bool narrow, double* radii) {
   constexpr int KB = B >= 255 ? 8 : B >= 127 ? 7 : B >= 63 ? 6 : B >= 31 ? 5 : 4;  // 2^KB - 1 <= B
   __shared__ double br[2 * G];
   __shared__ int cls[B * G], resolved[G];
@@ -368,16 +387,18 @@ __global__ void __launch_bounds__(B * G) k_bisect_band(double a, double ci, doub
   const bool valid = p < n;
   const double rho = valid ? radii[p] : __builtin_nan("");
   const int lmax = iters < kBandMaxLevels ? iters : kBandMaxLevels;
-  // one angle per block: narrow the band until every level fits (several
-  // angles per block keep the band and fewer levels: their lanes are few)
-  if (G == 1 && valid && band_nodes(rho, e, lmax) > B) {
-    double lo = 0.0, hi = e;
-    for (int it = 0; it < 30; ++it) {
-      const double m = 0.5 * (lo + hi);
-      if (band_nodes(rho, m, lmax) <= B) lo = m;
-      else hi = m;
+  if (narrow) {
+    // each of an angle's lanes in the wave tries one width, then one between the
+    // widest that fits and the next (a search by halves in every lane: 160 us)
+    constexpr int W = B < 64 ? B : 64;
+    const int c = threadIdx.x & (W - 1), at = (threadIdx.x & 63) & ~(W - 1);
+    double lo = 0.0, h = e;
+    for (int it = 0; it < 2; ++it) {
+      h *= 1.0 / W;
+      const unsigned long long fits = __ballot(band_nodes<B>(rho, lo + (c + 1) * h, lmax) <= B) >> at;
+      lo += __builtin_popcountll(W < 64 ? fits & ((1ull << (W & 63)) - 1) : fits) * h;
     }
-    e = lo;
+    e = __builtin_fmin(lo, e);
   }
   // this lane's midpoint in the band: level ml, bracket mb
   int L = 0, ml = -1;
@@ -396,22 +417,18 @@ __global__ void __launch_bounds__(B * G) k_bisect_band(double a, double ci, doub
       L = l + 1;
     }
   }
+  const double ca = cang[valid ? p : n - 1], sa = sang[valid ? p : n - 1];
   int c = 0;
-  if (ml >= 0) {
+  if (__any(ml >= 0)) {
     double lo = 0.5, hi = 10.0, mid = (hi - lo) / 2 + lo;
     for (int k = ml - 1; k >= 0; --k) {
       if ((mb >> k) & 1) lo = mid;
       else hi = mid;
       mid = (hi - lo) / 2 + lo;
     }
-    double sx[4], sv[4], st[8];
-    camera_ray(cang[p] * mid, sang[p] * mid, ci, si, d, sx, sv);
-    nullify(sx, sv, a, st);
-    WalkOut o;
-    walk_ray(st, N, 40.0, 1e-2, a, rEH, o);
-    c = o.sel_r < 100.0 ? 1 : 0;
+    c = final_radius(ca * mid, sa * mid, ml >= 0, ci, si, d, N, a, rEH) < 100.0 ? 1 : 0;
   }
-  cls[threadIdx.x] = c;
+  cls[g * B + j] = c;
   __syncthreads();
   if (j == 0) {
     double lo = 0.5, hi = 10.0;
@@ -445,8 +462,9 @@ __global__ void __launch_bounds__(B * G) k_bisect_band(double a, double ci, doub
     const int rounds = (rem + KB - 1) / KB;
     const int kr = rem > 0 ? (rem + rounds - 1) / rounds : 0;
     c = 0;
-    if (j < (1 << kr) - 1) {
-      const int m = j + 1, depth = 31 - __builtin_clz(m);
+    const bool live = j < (1 << kr) - 1;
+    if (__any(live)) {
+      const int m = live ? j + 1 : 1, depth = 31 - __builtin_clz(m);
       double lo = br[2 * g], hi = br[2 * g + 1];
       double mid = (hi - lo) / 2 + lo;
       for (int k = depth - 1; k >= 0; --k) {
@@ -454,14 +472,9 @@ __global__ void __launch_bounds__(B * G) k_bisect_band(double a, double ci, doub
         else hi = mid;
         mid = (hi - lo) / 2 + lo;
       }
-      double sx[4], sv[4], st[8];
-      camera_ray(cang[p] * mid, sang[p] * mid, ci, si, d, sx, sv);
-      nullify(sx, sv, a, st);
-      WalkOut o;
-      walk_ray(st, N, 40.0, 1e-2, a, rEH, o);
-      c = o.sel_r < 100.0 ? 1 : 0;
+      c = final_radius(ca * mid, sa * mid, live, ci, si, d, N, a, rEH) < 100.0 ? 1 : 0;
     }
-    cls[threadIdx.x] = c;
+    cls[g * B + j] = c;
     __syncthreads();
     if (j == 0 && kr > 0) {
       double lo = br[2 * g], hi = br[2 * g + 1];
@@ -1153,17 +1166,19 @@ static void critical_curve_about_origin(double a, double inc_deg, std::vector<do
   }
 }
 
-// Predicted shadow radius along each image direction (angle ang[p], the
-// image x axis at 0): the critical curve's table, interpolated between bin
-// centres; NaN where the table has no value.  Only the bisection's schedule depends on it.  The
-// tables of the last few (spin, inclination) pairs are kept.
+// Predicted shadow radius along each image direction (angle ang[p], cosine
+// cang[p], the image x axis at 0): the critical curve's table, interpolated
+// between bin centres; NaN where the table has no value.  Only the bisection's
+// schedule depends on it.  The tables of the last few (spin, inclination) pairs
+// are kept.
 namespace {
 std::mutex g_curve_mu;
 std::vector<std::pair<std::pair<double, double>, std::vector<double>>> g_curves;  // most recent last
 constexpr size_t kCurvesKept = 8;
 }  // namespace
 
-static void predicted_shadow_radii(double a, double inc_deg, const double* ang, long n, double* rho) {
+static void predicted_shadow_radii(double a, double inc_deg, double dist, const double* ang, const double* cang,
+                                   long n, double* rho) {
   std::vector<double> R;
   {
     std::lock_guard<std::mutex> lk(g_curve_mu);
@@ -1176,13 +1191,16 @@ static void predicted_shadow_radii(double a, double inc_deg, const double* ang, 
     if (g_curves.size() >= kCurvesKept) g_curves.erase(g_curves.begin());
     g_curves.push_back({{a, inc_deg}, R});
   }
+  // at a distance the curve lies 4 a sin(i) / dist towards -x of Bardeen's (the
+  // bisection's deviation from it, fitted at 50-1000 M, to 4 %)
+  const double shift = 4.0 * a * std::sin(inc_deg * M_PI / 180.0) / dist;
   for (long p = 0; p < n; ++p) {
     const double f = ang[p] - 2.0 * M_PI * std::floor((ang[p] + M_PI) / (2.0 * M_PI));  // in [-pi, pi)
     const double u = (f + M_PI) / (2.0 * M_PI) * kPolar - 0.5;
     const double fl = std::floor(u);
     const int k0 = (int)((((long)fl % kPolar) + kPolar) % kPolar), k1 = (k0 + 1) % kPolar;
     const double w = u - fl;
-    rho[p] = (1.0 - w) * R[k0] + w * R[k1];  // NaN when either bin is empty
+    rho[p] = (1.0 - w) * R[k0] + w * R[k1] - shift * cang[p];  // NaN when either bin is empty
   }
 }
 
@@ -1193,28 +1211,33 @@ static hipError_t launch_bisect(double a, double inc, const double* dc, const do
                                 int iters, double dist, double* dr, const double* h_rho, hipStream_t st) {
   double ci, si;
   cam_angles(inc, &ci, &si);
-  // The band form.  The FP64 walk slows with the
-  // waves resident on a CU, so up to 1024 angles each angle is a block of
-  // its own: one wave (the band then fits about 0.012 M about the
-  // prediction, which is within 0.007 M of the result for |a| <= 0.9) or, for
-  // higher spins, where the prediction drifts further (0.02 M at 0.97, more
-  // at high inclination near a = 1), two waves (about 0.03 M).  From 1025
-  // to 4096 angles, 8 angles of 32 lanes per block (2048 angles: 6.9 against
-  // 9.5 ms in tree rounds, 4096 angles 10.1 against 12.8 ms; 16 lanes per
-  // angle: 6.9 and 10.6 ms).
+  // The band form.  A SIMD's FP64 rate is nearly that of its one wave (a step
+  // takes 0.96 us with one wave on each SIMD, 1.85 with two), so the fewest
+  // wave-rounds win: up to 1024 angles one wave per angle, whose narrowed band
+  // is about 0.012 M wide on each side; up to 4096 two angles per wave (about
+  // 0.005 M).  The prediction holds to 0.003 M up to |a| = 0.9; above, rays
+  // near the prograde edge reach max_steps before they fall, and the result
+  // lies up to 0.013 M (0.97) or 0.03 M (0.998) outside it.  So from
+  // |a| = 0.95 two waves per angle up to 1024 angles (0.98, i = 85 deg: 64
+  // angles 2.0 against 3.8 ms, 1024 4.1 against 5.8; 0.95: 1024 angles 2.1 ms
+  // with one wave, 4.0 with two), and from |a| = 0.9 beyond 1024 the wide band
+  // in two rounds (4096 angles, 0.93, 85 deg: 6.0 against 7.7 ms; 0.9, 60 deg:
+  // 5.9 against 3.15 ms; eight angles per block of four waves as the start of
+  // two rounds 6.1, 16 angles per block 4.2 ms).
   const double e = bisect_band();
   if (h_rho && e > 0.0 && iters > 1 && n <= 4096) {
     hipError_t err = hipMemcpyAsync(dr, h_rho, n * sizeof(double), hipMemcpyHostToDevice, st);
     if (err == hipSuccess) err = hipStreamSynchronize(st);  // h_rho may be freed after the return
     if (err != hipSuccess) return err;
     const double rEH = horizon(a);
-    if (n <= 1024 && std::fabs(a) <= 0.9)
-      k_bisect_band<64, 1><<<(unsigned)n, 64, 0, st>>>(a, ci, si, dist, dc, ds, n, max_steps, iters, rEH, e, dr);
+    if (n <= 1024 && std::fabs(a) <= 0.95)
+      k_bisect_band<64, 1><<<(unsigned)n, 64, 0, st>>>(a, ci, si, dist, dc, ds, n, max_steps, iters, rEH, e, true, dr);
     else if (n <= 1024)
-      k_bisect_band<128, 1><<<(unsigned)n, 128, 0, st>>>(a, ci, si, dist, dc, ds, n, max_steps, iters, rEH, e, dr);
+      k_bisect_band<128, 1><<<(unsigned)n, 128, 0, st>>>(a, ci, si, dist, dc, ds, n, max_steps, iters, rEH, e, true,
+                                                         dr);
     else
-      k_bisect_band<32, 8><<<(unsigned)((n + 7) / 8), 256, 0, st>>>(a, ci, si, dist, dc, ds, n, max_steps, iters, rEH,
-                                                               e, dr);
+      k_bisect_band<32, 2><<<(unsigned)((n + 1) / 2), 64, 0, st>>>(a, ci, si, dist, dc, ds, n, max_steps, iters, rEH, e,
+                                                                  std::fabs(a) <= 0.9, dr);
     return hipGetLastError();
   }
   // K halvings per round with 2^K lanes per angle: the fewest rounds with at
@@ -1257,7 +1280,7 @@ hipError_t shadow_bisect_on_stream(double a, double inc, const double* h_angles,
     hc[p] = std::cos(h_angles[p]);
     hs[p] = std::sin(h_angles[p]);
   }
-  predicted_shadow_radii(a, inc, h_angles, n, hr.data());
+  predicted_shadow_radii(a, inc, dist, h_angles, hc.data(), n, hr.data());
   double *dc = d_stage, *ds = d_stage + n, *dr = d_stage + 2 * n;
   hipError_t e = hipMemcpyAsync(dc, hc.data(), n * sizeof(double), hipMemcpyHostToDevice, st);
   if (e == hipSuccess) e = hipMemcpyAsync(ds, hs.data(), n * sizeof(double), hipMemcpyHostToDevice, st);
@@ -1281,7 +1304,7 @@ int mk_shadow_bisect(double a, double inc, const double* h_angles, long n, int m
     hc[p] = std::cos(h_angles[p]);
     hs[p] = std::sin(h_angles[p]);
   }
-  predicted_shadow_radii(a, inc, h_angles, n, hr.data());
+  predicted_shadow_radii(a, inc, dist, h_angles, hc.data(), n, hr.data());
   double *dc = nullptr, *ds = nullptr, *dr = nullptr;
   hipError_t e = hipMalloc(&dc, n * sizeof(double));
   if (e == hipSuccess) e = hipMalloc(&ds, n * sizeof(double));

@@ -645,9 +645,9 @@ __global__ void __launch_bounds__(256, (MIXED && !SHADOW) ? 3 : 2)
 // tiles as four such waves would.  A chip with a deep backlog does better with
 // the other kernel (the gather and emission waves of a tile idle while its
 // geodesic wave is the slower), so a launch runs this one only without it.
-// 16 mixed images of 64^2-256^2 submitted together: 12.6 -> 10.0 ms; 1000 mixed images of 64^2-512^2 arriving at 200 per second:
-// p50 7.0 -> 3.7 ms, p99 16.1 -> 10.8 ms; a lone 256^2 image inside the
-// launch 5.4 -> 3.5 ms; 256 queued requests of 512^2 and 4096 angles (the
+// 16 mixed images of 64^2-256^2 submitted together: 12.6 -> 10.0 ms; 1000
+// mixed images of 64^2-512^2 arriving at 200 per second: p50 7.0 -> 3.7 ms, p99
+// 16.1 -> 10.8 ms; a lone 256^2 image inside the launch 5.4 -> 3.5 ms; 256 queued requests of 512^2 and 4096 angles (the
 // other kernel) unchanged.
 template <bool MIXED>
 __global__ void __launch_bounds__(256, 4) k_serve_tri(const ReqDev* __restrict__ req, PArgs P) {
