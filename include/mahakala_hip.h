@@ -204,7 +204,8 @@ typedef struct mk_render_params {
 } mk_render_params;
 
 /* mk_render_params.flags: kernel form.  By default the library runs a launch
- * of up to 15.5 8x8 tiles per CU (11 in FP64) in the triple form -- a geodesic
+ * of up to 15.5 8x8 tiles per CU (11 in FP64; up to four times as many at
+ * views with |a sin i| > 0.5) in the triple form -- a geodesic
  * wave, two gather waves (block lookup, cell loads, interpolation) and an
  * emission wave per tile -- and a larger one in the classic form (one wave
  * per tile).  The paired form (a geodesic wave and a transfer wave per tile)

@@ -653,7 +653,16 @@ static int choose_form(const SnapView& sv, const RenderDev& rp, int precision, i
   // SIMD holds waves of whole rays.  a = 0.5, i = 30 deg (a = 0.9, i = 60 deg),
   // triple against classic: mixed 480^2 3.10 (3.15) and 4.72 (7.51) ms, 640^2
   // 4.9 (4.7) and 4.7 (8.0) ms; plain FP64 416^2 3.45 (3.50) and 4.31 (8.54) ms.
-  if (2 * rp.ntiles <= (precision == 1 ? 31L : 22L) * cus) *form = MK_RENDER_TRIPLE;
+  // Beyond |a sin i| = 0.5 the rays at the prograde edge take so many steps
+  // that a classic launch lasts as long as their tiles do, at half the triple
+  // form's rate, so the line moves up with them.  Triple against classic, mixed
+  // (FP64): a = 0.7, i = 50 deg, 576^2 4.36 and 4.60 (5.88 and 5.53) ms; a = 0.9,
+  // i = 60 deg, 640^2 5.14 and 6.95 (6.93 and 8.29), 768^2 7.22 and 7.29 (9.7 and
+  // 8.5); a = 0.97, i = 80 deg, 768^2 7.24 and 13.1 (9.7 and 15.6), 1024^2 12.8
+  // and 15.5 (17.1 and 18.5) ms.
+  const double x2 = rp.a * rp.a * rp.si * rp.si;
+  const double scale = x2 > 0.25 ? (x2 < 0.75 ? 1.0 / (1.0 - x2) : 4.0) : 1.0;
+  if ((double)(2 * rp.ntiles) <= scale * (double)((precision == 1 ? 31L : 22L) * cus)) *form = MK_RENDER_TRIPLE;
   return MK_OK;
 }
 
