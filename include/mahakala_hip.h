@@ -105,6 +105,11 @@ int mk_trim_rows(const int32_t* d_K, long n, int N, long* h_T, void* stream);
  * and d_dt (T, n). */
 int mk_integrate_history(const double* d_s0, long n, int N, double div, double tol, double bhspin, long T,
                          double* d_S, double* d_dt, void* stream);
+/* mk_integrate_final, mk_trim_rows and mk_integrate_history in one walk of the
+ * rays: rows 0..T-1 into the first T rows of d_S (N, n, 8) and d_dt (N, n), K
+ * into d_K (n), T into *h_T.  Synchronises the stream. */
+int mk_integrate_rows(const double* d_s0, long n, int N, double div, double tol, double bhspin, double* d_S,
+                      double* d_dt, int32_t* d_K, long* h_T, void* stream);
 
 /* ----------------------------------------------------------------- shadow */
 /* select_photons_integrator  (geodesics.py:354-378): final radius per

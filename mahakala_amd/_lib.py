@@ -103,6 +103,7 @@ _SIGS = {
     "mk_integrate_final": [vp, lng, C.c_int, dbl, dbl, dbl, vp, vp, vp, vp],
     "mk_trim_rows": [vp, lng, C.c_int, C.POINTER(lng), vp],
     "mk_integrate_history": [vp, lng, C.c_int, dbl, dbl, dbl, lng, vp, vp, vp],
+    "mk_integrate_rows": [vp, lng, C.c_int, dbl, dbl, dbl, vp, vp, vp, C.POINTER(lng), vp],
     "mk_select_photons": [dbl, vp, vp, lng, dbl, dbl, C.c_int, vp],
     "mk_shadow_bisect": [dbl, dbl, vp, lng, C.c_int, dbl, C.c_int, dbl, vp],
     "mk_shadow_bisect_noalloc": [dbl, dbl, vp, lng, C.c_int, dbl, C.c_int, dbl, vp],

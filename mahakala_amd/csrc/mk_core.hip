@@ -190,8 +190,11 @@ __global__ void k_max_K(const int32_t* K, long n, int N, int* out /* [0] max K, 
   if (k >= N) atomicOr(&out[1], 1);
 }
 
+// With K (per ray, as walk_ray's) the rows end with the wave's last ray, and
+// k_repeat_rows writes the others once their number is known: one walk where
+// finding T first takes two.
 __global__ void __launch_bounds__(256) k_integrate_history(const double* s0, long n, double div, double tol, double a,
-                                                           double rEH, long T, double* S, double* D) {
+                                                           double rEH, long T, double* S, double* D, int32_t* K) {
   const long p = (long)blockIdx.x * blockDim.x + threadIdx.x, q = p < n ? p : n - 1;
   const bool live = p < n;
   double sa[8], sb[8];
@@ -201,6 +204,7 @@ __global__ void __launch_bounds__(256) k_integrate_history(const double* s0, lon
   if (!live) dta = 0.0;
   KsHead ha = ks_head(sa[1], sa[2], sa[3], a), hb;
   long row = 0;
+  int ended = dta == 0.0 ? 0 : (int)T;
   auto put = [&](const double s[8], double edt) {
     if (live) {
       double* out = S + 8 * (row * n + p);
@@ -216,6 +220,7 @@ __global__ void __launch_bounds__(256) k_integrate_history(const double* s0, lon
     hn = ks_head(nw[1], nw[2], nw[3], a);
     dtn = step_rule(hn.r, rEH, div, tol);
     dtn = dt != 0.0 ? dtn : 0.0;
+    ended = dt != 0.0 && dtn == 0.0 ? (int)row : ended;
     put(s, dtn != 0.0 ? dt : 0.0);
     if (dtn == 0.0) {  // the ray has ended: its last row repeats
 #pragma unroll
@@ -231,7 +236,23 @@ __global__ void __launch_bounds__(256) k_integrate_history(const double* s0, lon
     }
     step(sb, hb, dtb, sa, ha, dta);
   }
+  if (K) {
+    if (row == 0) put(sa, 0.0);
+    if (live) K[p] = ended;
+    return;
+  }
   while (row < T) put(sa, 0.0);
+}
+
+// Rows behind a ray's first frozen row K repeat its state with dt = 0.
+__global__ void k_repeat_rows(const int32_t* K, long n, long T, double* S, double* D) {
+  const long q = (long)blockIdx.x * blockDim.x + threadIdx.x;
+  if (q >= n * T) return;
+  const long row = q / n, p = q % n, k = K[p];
+  if (row <= k) return;
+#pragma unroll
+  for (int c = 0; c < 8; ++c) S[8 * q + c] = S[8 * (k * n + p) + c];
+  D[q] = 0.0;
 }
 
 // The final radius of the ray at image point (x, y); lanes without one pass any
@@ -1013,7 +1034,20 @@ int mk_integrate_history(const double* d_s0, long n, int N, double div, double t
   MK_REQUIRE(n >= 0 && T >= 0 && T <= N && d_s0 && d_S && d_dt, "mk_integrate_history: bad arguments");
   if (!n || !T) return MK_OK;
   k_integrate_history<<<grid_for(n, kChainBlock), kChainBlock, 0, as_stream(s)>>>(d_s0, n, div, tol, a, horizon(a), T, d_S,
-                                                                        d_dt);
+                                                                        d_dt, nullptr);
+  MK_LAUNCH_CHECK();
+  return MK_OK;
+}
+
+int mk_integrate_rows(const double* d_s0, long n, int N, double div, double tol, double a, double* d_S, double* d_dt,
+                      int32_t* d_K, long* h_T, void* s) {
+  MK_REQUIRE(n >= 1 && N >= 1 && d_s0 && div != 0.0 && d_S && d_dt && d_K && h_T,
+             "mk_integrate_rows: bad arguments");
+  k_integrate_history<<<grid_for(n, kChainBlock), kChainBlock, 0, as_stream(s)>>>(d_s0, n, div, tol, a, horizon(a), N,
+                                                                                  d_S, d_dt, d_K);
+  MK_LAUNCH_CHECK();
+  if (int rc = mk_trim_rows(d_K, n, N, h_T, s)) return rc;
+  k_repeat_rows<<<grid_for(n * *h_T, kBlock), kBlock, 0, as_stream(s)>>>(d_K, n, *h_T, d_S, d_dt);
   MK_LAUNCH_CHECK();
   return MK_OK;
 }

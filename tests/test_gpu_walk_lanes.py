@@ -78,3 +78,26 @@ def test_bisection_schedules_give_the_sequential_radii(spin, inc, n, monkeypatch
     few = slice(0, None, max(1, n // 3))
     np.testing.assert_array_equal(got[few], c_oracle.find_shadow_bisection_angles(spin, inc, ang[few], 2000, 1e-3, 40,
                                                                                   distance=1000.0))
+
+
+@pytest.mark.parametrize("n", [1, 63, 65])
+@pytest.mark.parametrize("N", [1, 2, 301, 2500])
+def test_history_in_one_walk_equals_two(n, N):
+    """geodesic_integrator finds T on the way when N rows are small: the rows
+    and T are those of the walk that finds T and the walk that writes."""
+    s0 = _start(n).cpu().numpy()
+    s0[n // 2, 1:4] *= 10.0  # starts beyond 1500 M: frozen from row 0
+    S, D = ma.geodesic_integrator(N, s0, 40, 1e-2, 0.9)
+    S2, D2 = ma.geodesic_integrator(N, s0, 40, 1e-2, 0.9, max_chunk_bytes=1)  # one ray at a time
+    np.testing.assert_array_equal(np.asarray(S), np.asarray(S2))
+    np.testing.assert_array_equal(np.asarray(D), np.asarray(D2))
+
+
+def test_history_in_one_walk_of_rays_that_are_all_frozen():
+    s0 = _start(65).cpu().numpy()
+    s0[:, 1:4] *= 10.0
+    S, D = ma.geodesic_integrator(7, s0, 40, 1e-2, 0.9)
+    S2, D2 = ma.geodesic_integrator(7, s0, 40, 1e-2, 0.9, max_chunk_bytes=1)
+    np.testing.assert_array_equal(np.asarray(S), np.asarray(S2))
+    np.testing.assert_array_equal(np.asarray(D), np.asarray(D2))
+    assert not np.asarray(D).any()
