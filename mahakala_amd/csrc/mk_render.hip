@@ -406,11 +406,18 @@ __global__ void __launch_bounds__(256, 4) k_render_tri(SnapView sv, RenderDev rp
   const int pi = (int)(tile / rp.tiles_x) * 8 + (lane >> 3), pj = (int)(tile % rp.tiles_x) * 8 + (lane & 7);
   const bool valid = pi < rp.res && pj < rp.res;
   const long p = (long)pi * rp.res + pj;
-  TriOut o;
-  tri_tile<MIXED, ZONE>(ring, wave, sv, rp, rp.spin_limit, grid_coord(rp.lo, rp.step, pi),
-                        grid_coord(rp.lo, rp.step, pj), valid, o);
-  if (valid && wave == 0 && steps) steps[p] = o.steps;
-  if (valid && wave == 3) img[p] = o.I;
+  if (wave == 0) {
+    int n;
+    tri_geodesic<MIXED, ZONE>(ring, rp, rp.spin_limit, grid_coord(rp.lo, rp.step, pi), grid_coord(rp.lo, rp.step, pj),
+                              valid, n);
+    if (valid && steps) steps[p] = n;
+  } else if (wave <= 2) {
+    tri_gather<MIXED>(ring, wave - 1, sv, rp.spin_limit);
+  } else {
+    bool ok;
+    const double I = tri_emission<MIXED>(ring, rp, rp.spin_limit, ok);
+    if (valid) img[p] = I;
+  }
 }
 
 // Critical curve of a distant camera at inclination theta (Bardeen 1973):

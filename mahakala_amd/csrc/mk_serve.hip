@@ -21,6 +21,7 @@
 #include <chrono>
 #include <cmath>
 #include <condition_variable>
+#include <cstddef>
 #include <cstring>
 #include <deque>
 #include <map>
@@ -412,7 +413,12 @@ __global__ void __launch_bounds__(256, 2) k_serve(const ReqDev* __restrict__ req
 // trips, and the launch served a twentieth of the relaunched form's rate.)
 // While the launch runs the host issues no copy to or from device memory: it
 // publishes work in pinned, coherent host memory (segments, descriptors, tile
-// orders and angle tables) and the waves read it there; finished pixels and
+// orders and angle tables).  The first waiting wave that sees a new published
+// count copies the new segments, descriptors and tile orders to device memory,
+// where all waves read them: read in host memory by every wave, a tile cost
+// about 13 reads over PCIe, 1.1 us of a link that all tiles share (1024 tiles of
+// one step each 1.27 ms, 0.13 ms from device memory; 16 mixed images of 64^2-256^2
+// queued together 7.9 ms, 5.9 ms).  Finished pixels and
 // radii go straight to pinned host memory, and the wave that completes a
 // request stores the request's sequence number in a pinned completion flag.
 // Every wait is bounded: a waiting wave sleeps between polls and exits when
@@ -439,13 +445,21 @@ struct PCtl {          // pinned host memory; each word on its own 128-byte line
 struct PArgs {
   PCtl* ctl;                    // host
   const PSeg* segs;             // host, seg_cap entries
+  const ReqDev* desc;           // host
+  const char* in;               // host: tile orders and angle tables
+  PSeg* dsegs;                  // device copies of segs, desc and (the first din_bytes of) in
+  ReqDev* ddesc;
+  char* din;
+  size_t din_bytes;
   int* fin;                     // host, per request slot
   unsigned long long* taken;    // device: tickets handed out
-  unsigned long long* seen;     // device: largest published count a wave has read, | kHalt once stopping
+  unsigned long long* seen;     // device: tickets whose segments are in dsegs, | kHalt once stopping
+  int* nseg;                    // device: segments copied to dsegs
+  int* lock;                    // device: held by the wave that copies
   int* done;                    // device: finished items per request slot
   unsigned long long* busy;     // device: lane-steps that advanced a ray
   unsigned long long* total;    // device: 64 x the wave-steps of every tile run
-  int seg_cap, idle_limit;
+  int seg_cap, idle_limit, first_seg;
 };
 
 constexpr unsigned long long kHalt = 1ull << 62;  // in `seen`: the host has set stop
@@ -461,97 +475,156 @@ __device__ __forceinline__ long long bcast64(long long v) {
 // system scope invalidates the L2 of the wave's XCD, and the busy waves of that
 // XCD would fetch their snapshot blocks from HBM again; the relaunched form's
 // loop has no acquire either.  Everything a wave reads that the host or
-// another wave wrote during the launch is read where no cache holds it:
-// segments, published counts, tile orders and angle tables are in pinned
-// coherent host memory, which the L2 does not cache, and are read with
-// system-scope loads; descriptors are read through the scalar cache, which the
-// launch started empty, from slots written before their segment was published
-// and never rewritten during the launch; the device counters are accessed with
-// agent-scope atomics, which are coherent across XCDs.  Program order orders a
-// wave's reads: each read is issued after the value it depends on has returned
-// (the segment after the published count, the descriptor after the segment).
+// another wave wrote during the launch is read where no cache holds an older
+// copy: published counts and angle tables are in pinned coherent host memory,
+// which the L2 does not cache; the counters and segments in device memory are
+// accessed with agent-scope atomics, which are coherent across XCDs;
+// descriptors and tile orders are read through the caches, which the launch
+// started without a copy of them, from memory that is written (through to
+// memory, before `seen` admits a reader) once per launch.  Program order orders
+// a wave's reads: each read is issued after the value it depends on has
+// returned.
 
-// Lane 0 waits until ticket t is published: 1 when it is, 0 when the host
-// has set stop, -1 after `idle_limit` sleeps.  The device word `seen` is read
-// every round; waiters within kFrontTickets of it also read host memory every
-// round (so new work is seen within one round), the others every 64 rounds.
-// A waiter that reads stop in host memory marks `seen` for all the others.
+__device__ __forceinline__ unsigned sys_load(const unsigned* p) {
+  return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+
+// N 32-bit words from host to device memory by the 64 lanes of a wave, C
+// blocks of 64 words in flight.
+template <int C>
+__device__ __forceinline__ void copy_words(const unsigned* src, unsigned* dst, int n) {
+  const int lane = __lane_id();
+  for (int k = 0; k < n; k += 64 * C) {
+    unsigned v[C];
+#pragma unroll
+    for (int c = 0; c < C; ++c) {
+      const int at = k + 64 * c + lane;
+      v[c] = at < n ? sys_load(src + at) : 0;
+    }
+#pragma unroll
+    for (int c = 0; c < C; ++c) {
+      const int at = k + 64 * c + lane;
+      if (at < n) __hip_atomic_store(dst + at, v[c], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    }
+  }
+}
+
+// The segments published since the last copy, with their descriptors and tile
+// orders, to device memory; by one wave at a time (P.lock), with all lanes.
+__device__ __forceinline__ void copy_published(const PArgs& P) {
+  constexpr int kSegWords = sizeof(PSeg) / 4, kDescWords = sizeof(ReqDev) / 4;
+  const int lane = __lane_id();
+  const int n0 = __builtin_amdgcn_readfirstlane(__hip_atomic_load(P.nseg, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT));
+  const int n1 = __builtin_amdgcn_readfirstlane(
+      __hip_atomic_load(&P.ctl->pub_segs, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM));
+  for (int i = n0; i < n1; ++i) {
+    const PSeg* hs = P.segs + i % P.seg_cap;
+    const unsigned w = lane < kSegWords ? sys_load((const unsigned*)hs + lane) : 0;
+    auto word = [&](size_t off) { return __builtin_amdgcn_readlane(w, (int)(off / 4)); };
+    const long long start = (long long)(((unsigned long long)word(offsetof(PSeg, start) + 4) << 32) |
+                                        (unsigned)word(offsetof(PSeg, start)));
+    const int count = word(offsetof(PSeg, count)), slot = word(offsetof(PSeg, desc));
+    const ReqDev* hd = P.desc + slot;
+    const int* ord = (const int*)bcast64(
+        (long long)__hip_atomic_load((const unsigned long long*)&hd->order, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM));
+    copy_words<(kDescWords + 63) / 64>((const unsigned*)hd, (unsigned*)(P.ddesc + slot), kDescWords);
+    const size_t at = (size_t)((const char*)ord - P.din);  // wraps for a null or host pointer
+    if (at < P.din_bytes && 4 * (size_t)count <= P.din_bytes - at)
+      copy_words<16>((const unsigned*)(P.in + at), (unsigned*)(P.din + at), count);
+    if (lane < kSegWords)
+      __hip_atomic_store((unsigned*)(P.dsegs + i % P.seg_cap) + lane, w, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "");  // in memory before the count that admits readers
+    if (lane == 0) __hip_atomic_fetch_max(P.nseg, i + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "");
+    if (lane == 0)
+      __hip_atomic_fetch_max(P.seen, (unsigned long long)(start + count), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  }
+}
+
+// Waits until ticket t is published: 1 when it is, 0 when the host has set
+// stop, -1 after `idle_limit` sleeps; by a whole wave.  The device word `seen`
+// is read every round; waiters within kFrontTickets of it also read host
+// memory every round (so new work is seen within one round), the others every
+// 64 rounds.  A waiter that reads a larger count there copies what was
+// published, or waits for the wave that does; one that reads stop in host
+// memory marks `seen` for all the others.
 __device__ __forceinline__ int wait_published(const PArgs& P, long long t) {
-  int state = 0;
-  if (__lane_id() == 0) {
-    for (int round = 0, slept = 0;; ++round) {
-      const unsigned long long v = __hip_atomic_load(P.seen, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-      long long pub = (long long)(v & ~kHalt);
-      if (t < pub) { state = 1; break; }
-      if (v & kHalt) break;
-      const long long d = t - pub;
-      if (d < kFrontTickets || ((round + (int)t) & 63) == 0) {
-        pub = __hip_atomic_load(&P.ctl->pub_tiles, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
-        __hip_atomic_fetch_max(P.seen, (unsigned long long)pub, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        if (t < pub) { state = 1; break; }
-        if (__hip_atomic_load(&P.ctl->stop, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM)) {
-          __hip_atomic_fetch_or(P.seen, kHalt, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-          break;
+  const bool first = __lane_id() == 0;
+  for (int round = 0, slept = 0; slept < P.idle_limit; ++round) {
+    const unsigned long long v =
+        (unsigned long long)bcast64((long long)__hip_atomic_load(P.seen, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT));
+    const long long pub = (long long)(v & ~kHalt);
+    if (t < pub) return 1;
+    if (v & kHalt) return 0;
+    const long long d = t - pub;
+    if (d < kFrontTickets || ((round + (int)t) & 63) == 0) {
+      const long long host =
+          bcast64(__hip_atomic_load(&P.ctl->pub_tiles, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM));
+      if (host > pub) {
+        int mine = 0;
+        if (first) mine = atomicCAS(P.lock, 0, 1) == 0;
+        if (__builtin_amdgcn_readfirstlane(mine)) {
+          copy_published(P);
+          __builtin_amdgcn_fence(__ATOMIC_RELEASE, "");
+          if (first) __hip_atomic_store(P.lock, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        } else {
+          __builtin_amdgcn_s_sleep(64);
         }
+        ++slept;
+        continue;
       }
-      // about 13 us a round near the published count, 54 us far from it
-      const int naps = d < 512 ? 4 : 16;
-      for (int k = 0; k < naps; ++k) __builtin_amdgcn_s_sleep(127);
-      slept += naps;
-      if (slept >= P.idle_limit) { state = -1; break; }
+      if (__builtin_amdgcn_readfirstlane(
+              __hip_atomic_load(&P.ctl->stop, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM))) {
+        if (first) __hip_atomic_fetch_or(P.seen, kHalt, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        return 0;
+      }
     }
+    // about 13 us a round near the published count, 54 us far from it
+    const int naps = d < 2048 ? 4 : 16;
+    for (int k = 0; k < naps; ++k) __builtin_amdgcn_s_sleep(127);
+    slept += naps;
   }
-  return __builtin_amdgcn_readfirstlane(__shfl(state, 0));
+  return -1;
 }
 
-// Lane 0 finds the published segment holding ticket t (a binary search over
-// the last seg_cap segments, from the wave's cursor); false if none does.
+// Finds the copied segment holding ticket t, 64 of them at a time from the
+// wave's cursor on (most tickets lie in the wave's current segment or the next
+// one); false if none does.  By a whole wave.
 __device__ __forceinline__ bool find_segment(const PArgs& P, long long t, int& cursor, PSeg& out) {
-  int ok = 0;
-  PSeg e{};
-  if (__lane_id() == 0) {
-    const int nseg = __hip_atomic_load(&P.ctl->pub_segs, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
-    int lo = cursor > nseg - P.seg_cap ? cursor : nseg - P.seg_cap, hi = nseg - 1;
-    if (lo < 0) lo = 0;
-    if (lo < hi) {  // most tickets lie in the wave's current segment or the next one
-      const PSeg* m = P.segs + (lo % P.seg_cap);
-      const int sq = __hip_atomic_load(&m->seq, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
-      const long long st = __hip_atomic_load(&m->start, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
-      const int ct = __hip_atomic_load(&m->count, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
-      if (sq == lo && st <= t && t < st + ct) hi = lo;
+  const int lane = __lane_id();
+  const int n = __builtin_amdgcn_readfirstlane(__hip_atomic_load(P.nseg, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT));
+  // an entry overwritten by a newer segment (its seq differs) is older than all in flight
+  for (int base = cursor > n - P.seg_cap ? cursor : n - P.seg_cap; base < n; base += 64) {
+    const int i = base + lane;
+    PSeg e{};
+    bool here = false;
+    if (i >= 0 && i < n) {
+      const PSeg* m = P.dsegs + i % P.seg_cap;
+      e.seq = __hip_atomic_load(&m->seq, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      e.start = __hip_atomic_load(&m->start, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      e.count = __hip_atomic_load(&m->count, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      e.rid = __hip_atomic_load(&m->rid, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      e.desc = __hip_atomic_load(&m->desc, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      here = e.seq == i && e.start <= t && t < e.start + e.count;
     }
-    // entries older than the ones in flight may be overwritten by newer
-    // ones (seq differs); they lie before t's segment
-    for (int guard = 0; guard < 40 && lo < hi; ++guard) {
-      const int mid = lo + (hi - lo + 1) / 2;
-      const PSeg* m = P.segs + (mid % P.seg_cap);
-      const int sq = __hip_atomic_load(&m->seq, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
-      const long long st = __hip_atomic_load(&m->start, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
-      if (sq != mid || st <= t) lo = mid;
-      else hi = mid - 1;
-    }
-    if (lo >= 0 && lo < nseg) {
-      const PSeg* m = P.segs + (lo % P.seg_cap);
-      e.seq = __hip_atomic_load(&m->seq, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
-      e.start = __hip_atomic_load(&m->start, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
-      e.count = __hip_atomic_load(&m->count, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
-      e.rid = __hip_atomic_load(&m->rid, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
-      e.desc = __hip_atomic_load(&m->desc, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
-      ok = (e.seq == lo && e.start <= t && t < e.start + e.count) ? 1 : 0;
-      if (ok) cursor = lo;
+    const unsigned long long found = __ballot(here);
+    if (found) {
+      const int src = __builtin_ctzll(found);
+      out.rid = __builtin_amdgcn_readlane(e.rid, src);
+      out.count = __builtin_amdgcn_readlane(e.count, src);
+      out.seq = __builtin_amdgcn_readlane(e.seq, src);
+      out.desc = __builtin_amdgcn_readlane(e.desc, src);
+      out.start = (long long)(((unsigned long long)(unsigned)__builtin_amdgcn_readlane((int)(e.start >> 32), src) << 32) |
+                              (unsigned)__builtin_amdgcn_readlane((int)e.start, src));
+      cursor = base + src;
+      return true;
     }
   }
-  ok = __builtin_amdgcn_readfirstlane(__shfl(ok, 0));
-  out.start = bcast64(e.start);
-  out.rid = __builtin_amdgcn_readfirstlane(__shfl(e.rid, 0));
-  out.count = __builtin_amdgcn_readfirstlane(__shfl(e.count, 0));
-  out.seq = __builtin_amdgcn_readfirstlane(__shfl(e.seq, 0));
-  out.desc = __builtin_amdgcn_readfirstlane(__shfl(e.desc, 0));
-  return ok != 0;
+  return false;
 }
 
-// `req` is the descriptor slots in pinned host memory, read as the relaunched
-// form reads its table: scalar loads through a read-only pointer.  SHADOW:
+// `req` is the descriptor slots' device copies, read as the relaunched form
+// reads its table: scalar loads through a read-only pointer.  SHADOW:
 // the launch serves bisections too; without them the mixed image path fits
 // three waves per SIMD (168 VGPRs against 236: the bisection's FP64 walk
 // needs the rest), and the host publishes no bisection to such a launch.
@@ -559,7 +632,7 @@ template <bool MIXED, bool SHADOW>
 __global__ void __launch_bounds__(256, (MIXED && !SHADOW) ? 3 : 2)
     k_serve_persistent(const ReqDev* __restrict__ req, PArgs P) {
   const int lane = threadIdx.x & 63;
-  int cursor = 0;
+  int cursor = P.first_seg;
   while (true) {
     unsigned long long tk = 0;
     if (lane == 0) tk = __hip_atomic_fetch_add(P.taken, 1ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
@@ -587,7 +660,7 @@ __global__ void __launch_bounds__(256, (MIXED && !SHADOW) ? 3 : 2)
       live = false;
     }
     if (q.kind == kKindImage) {
-      // the tile order lives in host memory: read it once per tile
+      // the tile order (of a large image in host memory): read it once per tile
       const int px = live ? pixel_of_item(q, item) : 0;
       Pending p;
       bool pend = false;
@@ -645,26 +718,38 @@ __global__ void __launch_bounds__(256, (MIXED && !SHADOW) ? 3 : 2)
 // tiles as four such waves would.  A chip with a deep backlog does better with
 // the other kernel (the gather and emission waves of a tile idle while its
 // geodesic wave is the slower), so a launch runs this one only without it.
-// 16 mixed images of 64^2-256^2 submitted together: 12.6 -> 10.0 ms; 1000
-// mixed images of 64^2-512^2 arriving at 200 per second: p50 7.0 -> 3.7 ms, p99
-// 16.1 -> 10.8 ms; a lone 256^2 image inside the launch 5.4 -> 3.5 ms; 256 queued requests of 512^2 and 4096 angles (the
-// other kernel) unchanged.
+// Against the other kernel, both with the segments read in host memory: 16
+// mixed images of 64^2-256^2 submitted together 12.6 -> 10.0 ms; 1000 mixed
+// images of 64^2-512^2 arriving at 200 per second p50 7.0 -> 3.7 ms.  With the
+// segments in device memory and a loop per role that stream's p50 is 2.5 ms, its
+// p99 7.7 ms, a lone 256^2 image inside the launch 1.7 ms (mixed) and 2.4 ms
+// (FP64; with one loop around the three roles, 252 bytes of spills, 3.5 ms).
 template <bool MIXED>
 __global__ void __launch_bounds__(256, 4) k_serve_tri(const ReqDev* __restrict__ req, PArgs P) {
   __shared__ TriRings<MIXED> ring;
   __shared__ int s_state, s_tile, s_rid, s_seq, s_desc;
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  int cursor = 0;
-  while (true) {
-    if (wave == 0) {
+  auto shared_int = [](const int& v) { return __builtin_amdgcn_readfirstlane(v); };
+  // pixel of the lane's item of the tile, -1 for none
+  auto pixel = [&](const ReqDev& q, int item) { return item < q.n_items ? pixel_of_item(q, item) : -1; };
+  // Each role loops over the tiles; two barriers per tile join them: after the
+  // first the tile is known, after the second no wave is left in it.
+  if (wave == 0) {
+    int cursor = P.first_seg;
+    while (true) {
       unsigned long long tk = 0;
       if (lane == 0) tk = __hip_atomic_fetch_add(P.taken, 1ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
       const long long t = bcast64((long long)tk);
       int state = wait_published(P, t), err = state < 0 ? 3 : 0;
       PSeg sg{};
-      if (state > 0 && !find_segment(P, t, cursor, sg)) {
-        state = -1;
-        err = 1;
+      if (state > 0) {
+        if (!find_segment(P, t, cursor, sg)) {
+          state = -1;
+          err = 1;
+        } else if (req[sg.desc].kind != kKindImage) {  // the host publishes no bisection to this launch
+          state = -1;
+          err = 4;
+        }
       }
       if (lane == 0) {
         if (err) __hip_atomic_store(&P.ctl->err, err, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
@@ -675,35 +760,40 @@ __global__ void __launch_bounds__(256, 4) k_serve_tri(const ReqDev* __restrict__
         s_desc = sg.desc;
         ring.reset();
       }
-    }
-    __syncthreads();
-    if (__builtin_amdgcn_readfirstlane(s_state) <= 0) break;
-    const int tile = __builtin_amdgcn_readfirstlane(s_tile), rid = __builtin_amdgcn_readfirstlane(s_rid);
-    const ReqDev& q = req[__builtin_amdgcn_readfirstlane(s_desc)];
-    const int item = tile * kTile + lane;
-    if (q.kind == kKindImage) {
-      const bool live = item < q.n_items;
-      // the tile order lives in host memory: read once per tile, by the waves that need the pixel
-      const int px = live && (wave == 0 || wave == 3) ? pixel_of_item(q, item) : 0;
-      TriOut o;
-      tri_tile<MIXED, false>(ring, wave, q.sv, q, kSpinLimit, grid_coord(q.lo, q.step, px / q.res),
-                             grid_coord(q.lo, q.step, px % q.res), live, o);
-      if (wave == 0) {
-        unsigned long long w = (unsigned long long)(live && o.steps > 0 ? o.steps : 0);
-        for (int off = 32; off > 0; off >>= 1) w += __shfl_xor(w, off);
-        if (lane == 0) {
-          atomicAdd(P.busy, w);
-          atomicAdd(P.total, 64ull * (unsigned long long)o.rounds);
-        }
+      __syncthreads();
+      if (state <= 0) break;
+      const ReqDev& q = req[sg.desc];
+      const int px = pixel(q, (int)(t - sg.start) * kTile + lane);
+      int n;
+      const int rounds = tri_geodesic<MIXED, false>(ring, q, kSpinLimit, grid_coord(q.lo, q.step, px / q.res),
+                                                    grid_coord(q.lo, q.step, px % q.res), px >= 0, n);
+      unsigned long long w = (unsigned long long)(px >= 0 && n > 0 ? n : 0);
+      for (int off = 32; off > 0; off >>= 1) w += __shfl_xor(w, off);
+      if (lane == 0) {
+        atomicAdd(P.busy, w);
+        atomicAdd(P.total, 64ull * (unsigned long long)rounds);
       }
-      if (wave == 3) {
-        if (live) q.out[px] = o.I;
-        if (!o.ok && lane == 0) __hip_atomic_store(&P.ctl->err, 5, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
-      }
-    } else if (threadIdx.x == 0) {  // the host publishes no bisection to this launch
-      __hip_atomic_store(&P.ctl->err, 4, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+      __syncthreads();
     }
-    if (wave == 3) {  // as in k_serve_persistent: the outputs, then the count, then the flag
+  } else if (wave <= 2) {
+    while (true) {
+      __syncthreads();
+      if (shared_int(s_state) <= 0) break;
+      tri_gather<MIXED>(ring, wave - 1, req[shared_int(s_desc)].sv, kSpinLimit);
+      __syncthreads();
+    }
+  } else {
+    while (true) {
+      __syncthreads();
+      if (shared_int(s_state) <= 0) break;
+      const int tile = shared_int(s_tile), rid = shared_int(s_rid), seq = shared_int(s_seq);
+      const ReqDev& q = req[shared_int(s_desc)];
+      bool ok;
+      const double I = tri_emission<MIXED>(ring, q, kSpinLimit, ok);
+      const int px = pixel(q, tile * kTile + lane);
+      if (px >= 0) q.out[px] = I;
+      if (!ok && lane == 0) __hip_atomic_store(&P.ctl->err, 5, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+      // as in k_serve_persistent: the outputs, then the count, then the flag
       __builtin_amdgcn_fence(__ATOMIC_RELEASE, "");
       if (lane == 0) {
         const int n = min(kTile, q.n_items - tile * kTile);
@@ -711,18 +801,19 @@ __global__ void __launch_bounds__(256, 4) k_serve_tri(const ReqDev* __restrict__
         if (old + n >= q.n_items) {
           __hip_atomic_store(&P.done[rid], 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
           __builtin_amdgcn_fence(__ATOMIC_RELEASE, "");
-          __hip_atomic_store(&P.fin[rid], s_seq + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+          __hip_atomic_store(&P.fin[rid], seq + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
         }
       }
+      __syncthreads();
     }
-    __syncthreads();  // every wave has left the tile before its rings are reset
   }
 }
 
-__global__ void k_set_pair(unsigned long long* p, unsigned long long a, unsigned long long b) {
+__global__ void k_start_launch(unsigned long long* taken, unsigned long long* seen, int* lock,
+                               unsigned long long ticket) {
   if (blockIdx.x == 0 && threadIdx.x == 0) {
-    p[0] = a;
-    p[1] = b;
+    *taken = *seen = ticket;
+    *lock = 0;
   }
 }
 
@@ -794,7 +885,12 @@ struct mk_server {
   char* p_in = nullptr;              // tile orders and angle tables of a launch
   size_t p_in_cap = 0, p_in_off = 0;
   char* p_out = nullptr;             // output staging (the budgeted arena)
-  unsigned long long* d_p = nullptr; // tickets taken, published count seen, busy and total lane-steps
+  // device counters, 128 bytes apart: tickets taken, published count seen, busy
+  // and total lane-steps (together), segments copied, lock of the copy
+  unsigned long long* d_p = nullptr;
+  PSeg* d_psegs = nullptr;           // device copies of p_segs, p_desc and the first kPersistOrderBytes of p_in
+  ReqDev* d_pdesc = nullptr;
+  char* d_pin = nullptr;
   int* d_pdone = nullptr;
   double* d_direct = nullptr;        // staging of bisections the idle worker runs itself
   double* d_direct_img = nullptr;    // and of its images
@@ -1246,6 +1342,8 @@ constexpr int kPersistMaxAgeMs = 1000;
 constexpr int kPersistWaitSleeps = 1 << 23;
 constexpr size_t kPersistInputBytes = (size_t)256 << 20;  // tile orders and angle tables per launch
 constexpr int kPersistDescSlots = 16384;          // descriptor slots per launch
+constexpr size_t kPersistOrderBytes = (size_t)64 << 20;  // of the inputs, the first copied to device memory
+constexpr size_t kPersistOrderTiles = 16384;             // longest tile order copied (1024^2)
 
 template <typename T>
 void store_shared(T* p, T v) {
@@ -1314,7 +1412,9 @@ void admit_persistent(mk_server* s) {
       if (q.tiled) {
         const std::vector<int>& ord = tile_order(s, p.img.resolution, p.img.fov, q.lo, q.step);
         std::memcpy(in, ord.data(), ord.size() * sizeof(int));
-        q.order = (const int*)in;
+        // a long order would hold up the copy: its waves read it in host memory
+        const bool copied = ord.size() <= kPersistOrderTiles && s->p_in_off + in_bytes <= kPersistOrderBytes;
+        q.order = (const int*)(copied ? s->d_pin + s->p_in_off : in);
       }
     } else {
       std::memcpy(in, f.cs.data(), f.cs.size() * sizeof(double));
@@ -1376,10 +1476,18 @@ bool launch_persistent(mk_server* s) {
   P.ctl = s->p_ctl;
   P.segs = s->p_segs;
   P.fin = s->p_fin;
+  P.desc = s->p_desc;
+  P.in = s->p_in;
+  P.dsegs = s->d_psegs;
+  P.ddesc = s->d_pdesc;
+  P.din = s->d_pin;
+  P.din_bytes = kPersistOrderBytes;
   P.taken = s->d_p;
-  P.seen = s->d_p + 1;
-  P.busy = s->d_p + 2;
-  P.total = s->d_p + 3;
+  P.seen = s->d_p + 16;
+  P.busy = s->d_p + 32;
+  P.total = s->d_p + 33;
+  P.nseg = (int*)(s->d_p + 48);
+  P.lock = (int*)(s->d_p + 64);
   P.done = s->d_pdone;
   P.seg_cap = s->seg_cap;
   P.idle_limit = kPersistWaitSleeps;
@@ -1387,7 +1495,11 @@ bool launch_persistent(mk_server* s) {
   s->stopping = false;
   s->want_shadow = false;
   bool shadow = false;
-  for (const auto& kv : s->flight) shadow = shadow || kv.second.shadow;
+  P.first_seg = s->seg_seq;
+  for (const auto& kv : s->flight) {
+    shadow = shadow || kv.second.shadow;
+    P.first_seg = std::min(P.first_seg, kv.second.seq);
+  }
   s->launch_shadow = shadow;
   // mixed without bisections, default lanes and a deep backlog: three waves
   // per SIMD, for throughput; otherwise two, each wave faster, for latency
@@ -1399,19 +1511,18 @@ bool launch_persistent(mk_server* s) {
   if (s->launch_tri) blocks *= 2;  // four waves per SIMD at the default lanes
   // tickets below resume_ticket are done; the previous launch's waves left
   // holding tickets from it on, unpublished then
-  k_set_pair<<<1, 64, 0, s->stream>>>(s->d_p, (unsigned long long)s->resume_ticket,
-                                      (unsigned long long)s->resume_ticket);
+  k_start_launch<<<1, 64, 0, s->stream>>>(P.taken, P.seen, P.lock, (unsigned long long)s->resume_ticket);
   SRV_HIP_UNLOCKED(hipGetLastError());
   SRV_HIP_UNLOCKED(hipEventRecord(s->ev0, s->stream));
   if (s->launch_tri) {
-    if (s->cfg.precision == 0) k_serve_tri<false><<<blocks, 256, 0, s->stream>>>(s->p_desc, P);
-    else k_serve_tri<true><<<blocks, 256, 0, s->stream>>>(s->p_desc, P);
+    if (s->cfg.precision == 0) k_serve_tri<false><<<blocks, 256, 0, s->stream>>>(s->d_pdesc, P);
+    else k_serve_tri<true><<<blocks, 256, 0, s->stream>>>(s->d_pdesc, P);
   } else if (s->cfg.precision == 0) {
-    if (shadow) k_serve_persistent<false, true><<<blocks, 256, 0, s->stream>>>(s->p_desc, P);
-    else k_serve_persistent<false, false><<<blocks, 256, 0, s->stream>>>(s->p_desc, P);
+    if (shadow) k_serve_persistent<false, true><<<blocks, 256, 0, s->stream>>>(s->d_pdesc, P);
+    else k_serve_persistent<false, false><<<blocks, 256, 0, s->stream>>>(s->d_pdesc, P);
   } else {
-    if (shadow) k_serve_persistent<true, true><<<blocks, 256, 0, s->stream>>>(s->p_desc, P);
-    else k_serve_persistent<true, false><<<blocks, 256, 0, s->stream>>>(s->p_desc, P);
+    if (shadow) k_serve_persistent<true, true><<<blocks, 256, 0, s->stream>>>(s->d_pdesc, P);
+    else k_serve_persistent<true, false><<<blocks, 256, 0, s->stream>>>(s->d_pdesc, P);
   }
   SRV_HIP_UNLOCKED(hipGetLastError());
   SRV_HIP_UNLOCKED(hipEventRecord(s->ev1, s->stream));
@@ -1436,7 +1547,7 @@ bool end_persistent(mk_server* s) {
   float ms = 0;
   SRV_HIP_UNLOCKED(hipEventElapsedTime(&ms, s->ev0, s->ev1));
   unsigned long long c[2] = {0, 0};  // busy and total lane-steps, over every launch so far
-  SRV_HIP_UNLOCKED(hipMemcpy(c, s->d_p + 2, sizeof c, hipMemcpyDeviceToHost));
+  SRV_HIP_UNLOCKED(hipMemcpy(c, s->d_p + 32, sizeof c, hipMemcpyDeviceToHost));
   std::lock_guard<std::mutex> lk(s->mu);
   s->st.gpu_ms += ms;
   s->st.lane_steps_busy = (int64_t)c[0];
@@ -1573,7 +1684,10 @@ int mk_server_create(const mk_server_config* cfg, mk_server** out) {
     if (e == hipSuccess) e = hipHostMalloc((void**)&s->p_fin, s->Rmax * sizeof(int), fl);
     if (e == hipSuccess) e = hipHostMalloc((void**)&s->p_in, s->p_in_cap, fl);
     if (e == hipSuccess) e = hipHostMalloc((void**)&s->p_out, s->arena_bytes, fl);
-    if (e == hipSuccess) e = hipMalloc(&s->d_p, 4 * sizeof(unsigned long long));
+    if (e == hipSuccess) e = hipMalloc(&s->d_p, 80 * sizeof(unsigned long long));
+    if (e == hipSuccess) e = hipMalloc(&s->d_psegs, s->seg_cap * sizeof(PSeg));
+    if (e == hipSuccess) e = hipMalloc(&s->d_pdesc, s->desc_cap * sizeof(ReqDev));
+    if (e == hipSuccess) e = hipMalloc(&s->d_pin, kPersistOrderBytes);
     if (e == hipSuccess) e = hipMalloc(&s->d_pdone, s->Rmax * sizeof(int));
     // the launch dereferences these host pointers: they must be its addresses too
     for (void* h : {(void*)s->p_ctl, (void*)s->p_segs, (void*)s->p_desc, (void*)s->p_fin, (void*)s->p_in,
@@ -1586,7 +1700,9 @@ int mk_server_create(const mk_server_config* cfg, mk_server** out) {
       std::memset(s->p_ctl, 0, sizeof(PCtl));
       std::memset(s->p_segs, 0xff, s->seg_cap * sizeof(PSeg));  // seq -1: no segment yet
       std::memset(s->p_fin, 0, s->Rmax * sizeof(int));
-      k_fill_int<<<1, 64, 0, s->stream>>>((int*)s->d_p, 8, 0);
+      k_fill_int<<<1, 256, 0, s->stream>>>((int*)s->d_p, 160, 0);
+      k_fill_int<<<grid_for(s->seg_cap * (sizeof(PSeg) / 4), 256), 256, 0, s->stream>>>((int*)s->d_psegs,
+                                                                                        s->seg_cap * (sizeof(PSeg) / 4), -1);
       k_fill_int<<<grid_for(s->Rmax, 256), 256, 0, s->stream>>>(s->d_pdone, s->Rmax, 0);
       e = hipGetLastError();
     }
@@ -1807,6 +1923,9 @@ int mk_server_destroy(mk_server* s) {
   (void)hipFree(s->d_arena);
   (void)hipFree(s->d_p);
   (void)hipFree(s->d_pdone);
+  (void)hipFree(s->d_psegs);
+  (void)hipFree(s->d_pdesc);
+  (void)hipFree(s->d_pin);
   (void)hipFree(s->d_direct);
   (void)hipFree(s->d_direct_img);
   for (void* h : {(void*)s->p_ctl, (void*)s->p_segs, (void*)s->p_desc, (void*)s->p_fin, (void*)s->p_in,

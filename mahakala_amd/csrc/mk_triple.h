@@ -93,188 +93,190 @@ __device__ __forceinline__ int wait_round(int* produced, int* done, int t, int* 
   return -1;
 }
 
-// What tri_tile leaves: the geodesic wave (0) the accepted steps per lane (-1
-// after a failed wait) and the steps of the longest ray, the emission wave (3)
-// the intensity (NaN after a failed wait, whichever wave's it was, and then ok
-// is false).
-struct TriOut {
-  double I = 0.0;
-  int steps = 0, rounds = 0;
-  bool ok = true;
-};
+// The three roles of a tile's four waves; all four run theirs after
+// ring.reset() and a workgroup barrier.  They are functions of their own, each
+// with the loop over tiles around it where there is one: with one such loop
+// around all three, what the compiler moves out of it is live in every role,
+// and the FP64 gather and emission spill.  rp: a RenderDev or a request
+// descriptor.
 
-// The tile's 64 rays at image points (x_img, y_img), lanes of `valid` only; all
-// four waves of the workgroup call it after ring.reset() and a barrier.  rp: a
-// RenderDev or a request descriptor.  ZONE (mixed): the geodesic wave takes
-// FP64 steps while any of its rays is in the zone (rp.fp64_r, rp.ring_r), as
-// the other forms do; without it the zone code is compiled out.
+// Geodesic wave (0): the tile's 64 rays at image points (x_img, y_img), lanes
+// of `valid` only.  steps: the accepted steps per lane (-1 after a failed wait);
+// returns the steps of the longest ray.  ZONE (mixed): FP64 steps while any of
+// the rays is in the zone (rp.fp64_r, rp.ring_r), as in the other forms; without
+// it the zone code is compiled out.
 template <bool MIXED, bool ZONE, typename Params>
-__device__ __forceinline__ void tri_tile(TriRings<MIXED>& ring, int wave, const SnapView& sv, const Params& rp,
-                                         int spin_limit, double x_img, double y_img, bool valid, TriOut& o) {
-  using T = typename std::conditional<MIXED, float, double>::type;
+__device__ __forceinline__ int tri_geodesic(TriRings<MIXED>& ring, const Params& rp, int spin_limit, double x_img,
+                                            double y_img, bool valid, int& steps) {
+  constexpr int DA = TriRings<MIXED>::kDepthA;
+  const int lane = threadIdx.x & 63;
+  // A lane is alive while its dt is not 0; dead lanes step along with dt = 0
+  // and are ignored, so the loop has no branches per lane.  All live lanes
+  // have taken the same number of steps, k.
+  double s[8], r = 0.0, dt = 0.0, drdl = 1e300;
+  KsHead h{}, hn{};  // FP64: the position terms at s and at the candidate
+  int k = 0, nacc = 0;
+#pragma unroll
+  for (int q = 0; q < 8; ++q) s[q] = 0.0;
+  if (valid) {
+    double sx[4], sv4[4];
+    camera_ray(x_img, y_img, rp.ci, rp.si, rp.dist, sx, sv4);
+    nullify(sx, sv4, rp.a, s);
+    r = radius_cal(s[1], s[2], s[3], rp.a);
+    dt = step_rule(r, rp.rEH, rp.div, rp.tol);
+  }
+  if constexpr (!MIXED) h = ks_head(s[1], s[2], s[3], rp.a);
+  double lim = 1500.0;  // largest |r - r_EH| of a live ray
+  // one RK4 step of every live lane into nw
+  auto step = [&](double nw[8]) {
+    if constexpr (!MIXED) {
+      rk4_step64(s, h, dt, rp.a, nw);
+    } else {
+      bool fp64 = false;
+      if constexpr (ZONE)
+        fp64 = __any(dt != 0.0 && ((r < rp.fp64_r) || (r < rp.ring_r && __builtin_fabs(drdl) < rp.ring_drdl)));
+      if (fp64) rk4_step<double>(s, dt, rp.a, nw);
+      else rk4_step_mixed(s, dt, (float)rp.a, nw);
+    }
+  };
+  // radius and step of the candidate; 0 ends the ray
+  auto rule = [&](const double nw[8], double& rn) {
+    double dtn;
+    if constexpr (!MIXED) {
+      hn = ks_head(nw[1], nw[2], nw[3], rp.a);
+      rn = hn.r;
+      dtn = step_rule(rn, rp.rEH, rp.div, rp.tol, lim);
+    } else {
+      rn = radius_f32(nw[1], nw[2], nw[3], rp.a);
+      dtn = step_rule_fast(rn, rp.rEH, rp.inv_div, rp.div, rp.tol, lim);
+    }
+    return dt != 0.0 ? dtn : 0.0;
+  };
+  // The way in: no ray of the tile is inside the sphere around the domain,
+  // so the steps are taken without handing anything over.  The step that
+  // first takes a ray inside is left to the loop below.
+  double nw[8];
+  while (k < rp.N && __any(dt != 0.0)) {
+    double rn;
+    step(nw);
+    const double dtn = rule(nw, rn);
+    if (__any(dtn != 0.0 && rn <= rp.r_dom)) break;
+    nacc += dtn != 0.0;
+    if (ZONE) drdl = (rn - r) / dt;
+#pragma unroll
+    for (int q = 0; q < 8; ++q) s[q] = nw[q];
+    dt = dtn;
+    r = rn;
+    h = hn;
+    ++k;
+  }
+  // A ray inside the sphere of radius r_out ends when it leaves it again.
+  if (r < rp.r_out) lim = __builtin_fmin(1500.0, rp.r_out - rp.rEH);
+  bool ok = true;
+  int t = 0;  // the next round
+  for (; k < rp.N && __any(dt != 0.0); ++k, ++t) {
+    // Slot t % DA is free once round t - DA has been read.  That count is
+    // loaded here without waiting and checked after the RK4 step: a wait at
+    // the loop head would also wait on this wave's slot writes of the round
+    // before (-2 to -4 % in FP64, -1 % in mixed).
+    int* readA = &ring.consumedA[t & 1];
+    const int polled = __hip_atomic_load(readA, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+    double* out = &ring.a[t % DA][0][lane];
+    step(nw);
+    // release the previous round here: its slot writes were issued a whole
+    // RK4 step ago, so the release fence does not wait on them
+    if (t > 0) publish(&ring.producedA, t);
+    if (__builtin_amdgcn_readfirstlane(polled) > t - DA) {
+      __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
+    } else if (wait_value(readA, t - DA + 1, spin_limit) < 0) {
+      ok = false;
+      break;
+    }
+    double rn;
+    const double dtn = rule(nw, rn);
+    nacc += dtn != 0.0;
+#pragma unroll
+    for (int q = 0; q < 8; ++q) out[q * 64] = nw[q];
+    out[8 * 64] = dtn != 0.0 && k + 1 < rp.N ? dt : 0.0;  // row N is never emitted
+    if (ZONE) drdl = (rn - r) / dt;
+#pragma unroll
+    for (int q = 0; q < 8; ++q) s[q] = nw[q];
+    dt = dtn;
+    r = rn;
+    h = hn;
+  }
+  if (ok) publish(&ring.producedA, t);
+  publish(&ring.doneA, ok ? t : -2);
+  steps = ok ? nacc : -1;
+  return k;
+}
+
+// Gather wave g (0, 1): lookup, cell loads, interpolation of every other round.
+template <bool MIXED>
+__device__ __forceinline__ void tri_gather(TriRings<MIXED>& ring, int g, const SnapView& sv, int spin_limit) {
   using R = TriRings<MIXED>;
+  using T = typename R::T;
   constexpr int DA = R::kDepthA, DB = R::kDepthB;
   const int lane = threadIdx.x & 63;
-  if (wave == 0) {  // geodesic
-    // A lane is alive while its dt is not 0; dead lanes step along with dt = 0
-    // and are ignored, so the loop has no branches per lane.  All live lanes
-    // have taken the same number of steps, k.
-    double s[8], r = 0.0, dt = 0.0, drdl = 1e300;
-    KsHead h{}, hn{};  // FP64: the position terms at s and at the candidate
-    int k = 0, nacc = 0;
-#pragma unroll
-    for (int q = 0; q < 8; ++q) s[q] = 0.0;
-    if (valid) {
-      double sx[4], sv4[4];
-      camera_ray(x_img, y_img, rp.ci, rp.si, rp.dist, sx, sv4);
-      nullify(sx, sv4, rp.a, s);
-      r = radius_cal(s[1], s[2], s[3], rp.a);
-      dt = step_rule(r, rp.rEH, rp.div, rp.tol);
-    }
-    if constexpr (!MIXED) h = ks_head(s[1], s[2], s[3], rp.a);
-    double lim = 1500.0;  // largest |r - r_EH| of a live ray
-    // one RK4 step of every live lane into nw (mixed may step in place: the
-    // step functions write their output only after reading the state)
-    auto step = [&](double nw[8]) {
-      if constexpr (!MIXED) {
-        rk4_step64(s, h, dt, rp.a, nw);
-      } else {
-        bool fp64 = false;
-        if constexpr (ZONE)
-          fp64 = __any(dt != 0.0 && ((r < rp.fp64_r) || (r < rp.ring_r && __builtin_fabs(drdl) < rp.ring_drdl)));
-        if (fp64) rk4_step<double>(s, dt, rp.a, nw);
-        else rk4_step_mixed(s, dt, (float)rp.a, nw);
+  bool ok = true;
+  int avail = 0, freed = 0;  // rounds of ring A published, of ring B read (last values seen)
+  int cmb = -1;              // block of the ray's last sample and its record
+  double crec[kMeta];
+  int t = g;
+  for (;; t += 2) {
+    if (t >= avail) {
+      const int st = wait_round(&ring.producedA, &ring.doneA, t, &avail, spin_limit);
+      if (st <= 0) {
+        ok = st == 0;
+        break;
       }
-    };
-    // radius and step of the candidate; 0 ends the ray
-    auto rule = [&](const double nw[8], double& rn) {
-      double dtn;
-      if constexpr (!MIXED) {
-        hn = ks_head(nw[1], nw[2], nw[3], rp.a);
-        rn = hn.r;
-        dtn = step_rule(rn, rp.rEH, rp.div, rp.tol, lim);
-      } else {
-        rn = radius_f32(nw[1], nw[2], nw[3], rp.a);
-        dtn = step_rule_fast(rn, rp.rEH, rp.inv_div, rp.div, rp.tol, lim);
-      }
-      return dt != 0.0 ? dtn : 0.0;
-    };
-    // The way in: no ray of the tile is inside the sphere around the domain,
-    // so the steps are taken without handing anything over.  The step that
-    // first takes a ray inside is left to the loop below.
-    double nw_[8];
-    while (k < rp.N && __any(dt != 0.0)) {
-      double rn;
-      step(nw_);
-      const double dtn = rule(nw_, rn);
-      if (__any(dtn != 0.0 && rn <= rp.r_dom)) break;
-      nacc += dtn != 0.0;
-      if (ZONE) drdl = (rn - r) / dt;
-#pragma unroll
-      for (int q = 0; q < 8; ++q) s[q] = nw_[q];
-      dt = dtn;
-      r = rn;
-      h = hn;
-      ++k;
     }
-    // A ray inside the sphere of radius r_out ends when it leaves it again.
-    if (r < rp.r_out) lim = __builtin_fmin(1500.0, rp.r_out - rp.rEH);
-    bool ok = true;
-    int t = 0;  // the next round
-    for (; k < rp.N && __any(dt != 0.0); ++k, ++t) {
-      // Slot t % DA is free once round t - DA has been read.  That count is
-      // loaded here without waiting and checked after the RK4 step: a wait at
-      // the loop head would also wait on this wave's slot writes of the round
-      // before (-2 to -4 % in FP64, -1 % in mixed).
-      int* readA = &ring.consumedA[t & 1];
-      const int polled = __hip_atomic_load(readA, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
-      double* out = &ring.a[t % DA][0][lane];
-      double* nw = MIXED ? s : nw_;  // mixed in place: -1.3 %; in FP64 the copy is faster
-      step(nw);
-      // release the previous round here: its slot writes were issued a whole
-      // RK4 step ago, so the release fence does not wait on them
-      if (t > 0) publish(&ring.producedA, t);
-      if (__builtin_amdgcn_readfirstlane(polled) > t - DA) {
-        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
-      } else if (wait_value(readA, t - DA + 1, spin_limit) < 0) {
+    if (t - DB + 1 > freed) {
+      freed = wait_value(&ring.consumedB, t - DB + 1, spin_limit);
+      if (freed < 0) {
         ok = false;
         break;
       }
-      double rn;
-      const double dtn = rule(nw, rn);
-      nacc += dtn != 0.0;
-#pragma unroll
-      for (int q = 0; q < 8; ++q) out[q * 64] = nw[q];
-      out[8 * 64] = dtn != 0.0 && k + 1 < rp.N ? dt : 0.0;  // row N is never emitted
-      if (ZONE) drdl = (rn - r) / dt;
-      if constexpr (!MIXED) {
-#pragma unroll
-        for (int q = 0; q < 8; ++q) s[q] = nw[q];
-      }
-      dt = dtn;
-      r = rn;
-      h = hn;
     }
-    if (ok) publish(&ring.producedA, t);
-    publish(&ring.doneA, ok ? t : -2);
-    o.steps = ok ? nacc : -1;
-    o.rounds = k;
-    return;
-  }
-  if (wave <= 2) {  // gather: lookup, cell loads, interpolation of every other round
-    const int g = wave - 1;
-    bool ok = true;
-    int avail = 0, freed = 0;  // rounds of ring A published, of ring B read (last values seen)
-    int cmb = -1;              // block of the ray's last sample and its record
-    double crec[kMeta];
-    int t = g;
-    for (;; t += 2) {
-      if (t >= avail) {
-        const int st = wait_round(&ring.producedA, &ring.doneA, t, &avail, spin_limit);
-        if (st <= 0) {
-          ok = st == 0;
-          break;
-        }
+    const double* in = &ring.a[t % DA][0][lane];
+    double pdt = in[8 * 64];
+    double ps[8];
+#pragma unroll
+    for (int q = 0; q < 8; ++q) ps[q] = in[q * 64];
+    publish(&ring.consumedA[g], t + 1);  // ring A slot is in registers
+    T* ob = &ring.bt[t % DB][0][lane];
+    T P[8];
+#pragma unroll
+    for (int q = 0; q < 8; ++q) P[q] = T(0);
+    if (pdt != 0.0) {
+      const Stencil stc = locate_cached(sv, sv.meta, sv.grid, ps[1], ps[2], ps[3], cmb, crec);
+      if (stc.mb >= 0) {
+        Corners cr;
+        fetch<false>(sv, stc, cr);
+        interp<T>(stc, cr, P);
       }
-      if (t - DB + 1 > freed) {
-        freed = wait_value(&ring.consumedB, t - DB + 1, spin_limit);
-        if (freed < 0) {
-          ok = false;
-          break;
-        }
-      }
-      const double* in = &ring.a[t % DA][0][lane];
-      double pdt = in[8 * 64];
-      double ps[8];
-#pragma unroll
-      for (int q = 0; q < 8; ++q) ps[q] = in[q * 64];
-      publish(&ring.consumedA[g], t + 1);  // ring A slot is in registers
-      T* ob = &ring.bt[t % DB][0][lane];
-      T P[8];
-#pragma unroll
-      for (int q = 0; q < 8; ++q) P[q] = T(0);
-      if (pdt != 0.0) {
-        const Stencil stc = locate_cached(sv, sv.meta, sv.grid, ps[1], ps[2], ps[3], cmb, crec);
-        if (stc.mb >= 0) {
-          Corners cr;
-          fetch<false>(sv, stc, cr);
-          interp<T>(stc, cr, P);
-        }
-        if (stc.mb < 0 || P[0] == T(0)) pdt = 0.0;  // adds exactly nothing
-      }
-#pragma unroll
-      for (int q = 0; q < 8; ++q) ob[q * 64] = P[q];
-#pragma unroll
-      for (int q = 1; q < 8; ++q) ob[(7 + q) * 64] = (T)ps[q];
-      ring.bd[t % DB][lane] = pdt;
-      publish(&ring.producedB[g], t + 1);
+      if (stc.mb < 0 || P[0] == T(0)) pdt = 0.0;  // adds exactly nothing
     }
-    publish(&ring.doneB[g], ok ? t : -2);
-    return;
+#pragma unroll
+    for (int q = 0; q < 8; ++q) ob[q * 64] = P[q];
+#pragma unroll
+    for (int q = 1; q < 8; ++q) ob[(7 + q) * 64] = (T)ps[q];
+    ring.bd[t % DB][lane] = pdt;
+    publish(&ring.producedB[g], t + 1);
   }
-  // emission and transfer, in step order
+  publish(&ring.doneB[g], ok ? t : -2);
+}
+
+// Emission wave: emission and transfer in step order; the intensity, NaN after
+// a failed wait, whichever wave's it was (then ok is false).
+template <bool MIXED, typename Params>
+__device__ __forceinline__ double tri_emission(TriRings<MIXED>& ring, const Params& rp, int spin_limit, bool& ok) {
+  using R = TriRings<MIXED>;
+  using T = typename R::T;
+  constexpr int DB = R::kDepthB;
+  const int lane = threadIdx.x & 63;
   double I = 0.0, trans = 1.0;
-  bool ok = true;
+  ok = true;
   for (int t = 0;; ++t) {
     int avail = 0;
     const int st = wait_round(&ring.producedB[t & 1], &ring.doneB[t & 1], t, &avail, spin_limit);
@@ -300,8 +302,7 @@ __device__ __forceinline__ void tri_tile(TriRings<MIXED>& ring, int wave, const 
       trans *= (1.0 - cc * (double)al);
     }
   }
-  o.ok = ok;
-  o.I = ok ? I : __builtin_nan("");
+  return ok ? I : __builtin_nan("");
 }
 
 }  // namespace mk
