@@ -153,6 +153,17 @@ __global__ void __launch_bounds__(256) k_sample_prims(SnapView sv, const double*
   for (int c = 0; c < 8; ++c) out[c * n + p] = P[c];
 }
 
+// Per sample 64 bytes in, 40 out and the cells; 100 registers, so four waves
+// per SIMD hide three loads in sequence (lookup record, record, cells) behind
+// 530 instructions.  More waves (launch bounds 5: spills) and a grid of
+// resident blocks that load the next state early are both slower (141 and 140
+// against 125 us at 3.4e6 samples).  STREAM: the outputs bypass the caches'
+// retention, which keeps them from evicting states and cells.  Measured
+// (samples: without, with; in blocks of 64): 4.1e5: 9.5, 7.8 us but followed by a
+// reader of the outputs 18.0, 19.3; 1.6e6: 62, 59 (65); 3.4e6: 125, 112 (107);
+// 6.6e6: 207, 204 (186).
+constexpr long kStreamSamples = 1500000, kSmallBlockSamples = 3000000;
+template <bool STREAM>
 __global__ void __launch_bounds__(256) k_sample_scalars(SnapView sv, const double* S, long n, double a, double fbc,
                                                         double* out) {
   const long p = (long)blockIdx.x * blockDim.x + threadIdx.x;
@@ -165,7 +176,10 @@ __global__ void __launch_bounds__(256) k_sample_scalars(SnapView sv, const doubl
   const Fluid64 F = fluid64(P, q[1], q[2], q[3], q[4], q[5], q[6], q[7], a, fbc);
   const double sc[5] = {P[0], P[1], ::acos(F.cosp), F.kdotu, F.W == 0.0 ? 0.0 : F.sW * F.iu0};
 #pragma unroll
-  for (int c = 0; c < 5; ++c) out[c * n + p] = sc[c];
+  for (int c = 0; c < 5; ++c) {
+    if constexpr (STREAM) __builtin_nontemporal_store(sc[c], out + c * n + p);
+    else out[c * n + p] = sc[c];
+  }
 }
 
 static long pymod(long a, long m) { long r = a % m; return r < 0 ? r + m : r; }
@@ -400,7 +414,9 @@ int mk_sample_scalars(const mk_snapshot* s, const double* d_S, long n, double a,
                       void* st) {
   MK_REQUIRE(s && d_S && d_out && n >= 0, "mk_sample_scalars: bad arguments");
   if (!n) return MK_OK;
-  k_sample_scalars<<<grid_for(n, 256), 256, 0, as_stream(st)>>>(s->view(), d_S, n, a, std::cos(fallback), d_out);
+  const int block = n >= kSmallBlockSamples ? 64 : 256;
+  auto kern = n >= kStreamSamples ? k_sample_scalars<true> : k_sample_scalars<false>;
+  kern<<<grid_for(n, block), block, 0, as_stream(st)>>>(s->view(), d_S, n, a, std::cos(fallback), d_out);
   MK_LAUNCH_CHECK();
   return MK_OK;
 }
