@@ -63,7 +63,6 @@ template <> struct Math<double> {
     g = __builtin_fma(d, h, g);
     return x == 0.0 ? x : g;
   }
-  static __device__ __forceinline__ double sqrt_ieee(double x) { return __builtin_sqrt(x); }
   // sqrt(x) and 1/sqrt(x) from one reciprocal square root: two Goldschmidt
   // steps carry g -> sqrt(x) and h -> 1/(2 sqrt(x)) from the estimate's
   // 2^-24 to about 1.5 ulp, one residual correction rounds g as sqrt()
@@ -104,12 +103,6 @@ template <> struct Math<double> {
     return __builtin_fma(y, __builtin_fma(e, e, e), y);
   }
   static __device__ __forceinline__ double exp(double x) { return ::exp(x); }
-  static __device__ __forceinline__ double pow(double x, double y) { return ::pow(x, y); }
-  static __device__ __forceinline__ double cbrt(double x) { return ::cbrt(x); }
-  static __device__ __forceinline__ double sin(double x) { return ::sin(x); }
-  static __device__ __forceinline__ double acos(double x) { return ::acos(x); }
-  static __device__ __forceinline__ double cos(double x) { return ::cos(x); }
-  static __device__ __forceinline__ double abs(double x) { return __builtin_fabs(x); }
 };
 template <> struct Math<float> {
   static __device__ __forceinline__ float rcp(float x) { return __builtin_amdgcn_rcpf(x); }
@@ -121,23 +114,15 @@ template <> struct Math<float> {
   }
   static __device__ __forceinline__ float div(float a, float b) { return a * __builtin_amdgcn_rcpf(b); }
   static __device__ __forceinline__ float sqrt(float x) { return __builtin_amdgcn_sqrtf(x); }
-  static __device__ __forceinline__ float sqrt_ieee(float x) { return __builtin_amdgcn_sqrtf(x); }
   // sqrt(x) and 1/sqrt(x) from one hardware reciprocal square root
   static __device__ __forceinline__ void sqrt_rcp(float x, float& s, float& is) {
     is = __builtin_amdgcn_rsqf(x);
     s = x * is;
   }
   static __device__ __forceinline__ float exp(float x) { return __builtin_amdgcn_exp2f(x * 1.4426950408889634f); }
-  static __device__ __forceinline__ float pow(float x, float y) {
-    // x >= 0 here; log2(0) = -inf gives 0, log2(inf) = inf gives inf
-    return __builtin_amdgcn_exp2f(y * __builtin_amdgcn_logf(x));
-  }
   static __device__ __forceinline__ float cbrt(float x) {
     return __builtin_amdgcn_exp2f(0.3333333333333333f * __builtin_amdgcn_logf(x));
   }
-  static __device__ __forceinline__ float sin(float x) { return ::__sinf(x); }
-  static __device__ __forceinline__ float acos(float x) { return ::acosf(x); }
-  static __device__ __forceinline__ float cos(float x) { return ::__cosf(x); }
   static __device__ __forceinline__ float abs(float x) { return __builtin_fabsf(x); }
 };
 
