@@ -285,7 +285,7 @@ typedef struct mk_server_config {
  * launches.  Without it, an idle server (no launch running, nothing in
  * flight) runs a bisection of up to 1024 angles at the head of its queue
  * itself, in mk_shadow_bisect's band schedule: about one integration chain
- * instead of one per halving (64 angles: 3.5 against 35 ms); the same radii,
+ * instead of one per halving (64 angles: 2.0 against 23 ms); the same radii,
  * bit for bit.  Requests submitted meanwhile wait until it ends. */
 #define MK_SERVER_SHADOW_IN_LAUNCH 2
 /* mk_server_config.flags: images always run inside the server's launches.

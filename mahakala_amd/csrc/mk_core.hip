@@ -1255,9 +1255,10 @@ static hipError_t launch_bisect(double a, double inc, const double* dc, const do
   // |a| = 0.95 two waves per angle up to 1024 angles (0.98, i = 85 deg: 64
   // angles 2.0 against 3.8 ms, 1024 4.1 against 5.8; 0.95: 1024 angles 2.1 ms
   // with one wave, 4.0 with two), and from |a| = 0.9 beyond 1024 the wide band
-  // in two rounds (4096 angles, 0.93, 85 deg: 6.0 against 7.7 ms; 0.9, 60 deg:
-  // 5.9 against 3.15 ms; eight angles per block of four waves as the start of
-  // two rounds 6.1, 16 angles per block 4.2 ms).
+  // in two rounds (4096 angles, 0.93, 85 deg: 6.0 against 7.7 ms; at 0.9, 60 deg
+  // the narrow one 3.15 against 5.9).  Eight angles per block of four waves take
+  // the same times, 16 per block of eight waves 4.2 ms narrow; 48 lanes per
+  // angle 5.2 ms.
   const double e = bisect_band();
   if (h_rho && e > 0.0 && iters > 1 && n <= 4096) {
     hipError_t err = hipMemcpyAsync(dr, h_rho, n * sizeof(double), hipMemcpyHostToDevice, st);

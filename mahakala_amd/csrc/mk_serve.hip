@@ -417,10 +417,10 @@ __global__ void __launch_bounds__(256, 2) k_serve(const ReqDev* __restrict__ req
 // count copies the new segments, descriptors and tile orders to device memory,
 // where all waves read them: read in host memory by every wave, a tile cost
 // about 13 reads over PCIe, 1.1 us of a link that all tiles share (1024 tiles of
-// one step each 1.27 ms, 0.13 ms from device memory; 16 mixed images of 64^2-256^2
-// queued together 7.9 ms, 5.9 ms).  Finished pixels and
-// radii go straight to pinned host memory, and the wave that completes a
-// request stores the request's sequence number in a pinned completion flag.
+// one step each 1.27 ms, 0.13 ms from device memory; 16 mixed images of
+// 64^2-256^2 queued together 7.9 ms, 5.9 ms).  Finished pixels and radii go
+// straight to pinned host memory, and the wave that completes a request stores
+// the request's sequence number in a pinned completion flag.
 // Every wait is bounded: a waiting wave sleeps between polls and exits when
 // the host sets `stop`, or reports an error after `idle_limit` sleeps.  The
 // host sets `stop` only when every published tile is done, and publishes
