@@ -35,16 +35,22 @@ __device__ __forceinline__ void publish(int* cnt, int v) {
 // rays ending outside the domain and nothing handed over on their way in 3.14
 // (1.73) and 3.03 (1.46) ms.  160^2 at a = 0.9: plain 3.93 -> 2.70 ms, mixed
 // 3.18 -> 2.65 ms.
-// Ring A carries (state, dt) from the geodesic wave, ring B the eight
-// interpolated primitives and the state in the emission's precision (FP32
-// values are what the FP32 emission would round them to) and dt in FP64 (0:
-// nothing to add).
+// Ring A carries the state (in mixed the momentum already as the floats the
+// emission rounds it to) and dt from the geodesic wave, ring B the eight
+// interpolated primitives and the state in the emission's precision and dt in
+// FP64 (0: nothing to add).
 template <bool MIXED>
 struct TriRings {
   using T = typename std::conditional<MIXED, float, double>::type;
-  static constexpr int kDepthA = 4, kDepthB = MIXED ? 4 : 2;  // rounds (35 KB: four workgroups fit 160 KB)
+  static constexpr int kDepthA = 4, kDepthB = MIXED ? 4 : 2;  // rounds (30 and 35 KB: four workgroups fit 160 KB)
   static constexpr int kCompB = 15;                           // P[8], s[1..7]
-  double a[kDepthA][kPairComp][64];
+  // ring A, FP64: the state and dt (without the unused coordinate time the
+  // geodesic loop is scheduled 1-2 % slower); mixed: position, dt and, as the
+  // emission's floats in one 16-byte word, the momentum (a slot write of 8 bytes
+  // costs the geodesic wave about 19 cycles: 256^2 1.422 -> 1.407 ms)
+  static constexpr int kCompA = MIXED ? 4 : kPairComp, kPosA = MIXED ? 0 : 1;
+  double a[kDepthA][kCompA][64];
+  float4 av[MIXED ? kDepthA : 1][64];
   double bd[kDepthB][64];  // dt
   T bt[kDepthB][kCompB][64];
   int producedA, doneA, consumedB;
@@ -108,7 +114,7 @@ __device__ __forceinline__ int wait_round(int* produced, int* done, int t, int* 
 template <bool MIXED, bool ZONE, typename Params>
 __device__ __forceinline__ int tri_geodesic(TriRings<MIXED>& ring, const Params& rp, int spin_limit, double x_img,
                                             double y_img, bool valid, int& steps) {
-  constexpr int DA = TriRings<MIXED>::kDepthA;
+  constexpr int DA = TriRings<MIXED>::kDepthA, CA = TriRings<MIXED>::kCompA;
   const int lane = threadIdx.x & 63;
   // A lane is alive while its dt is not 0; dead lanes step along with dt = 0
   // and are ignored, so the loop has no branches per lane.  All live lanes
@@ -183,6 +189,17 @@ __device__ __forceinline__ int tri_geodesic(TriRings<MIXED>& ring, const Params&
     const int polled = __hip_atomic_load(readA, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
     double* out = &ring.a[t % DA][0][lane];
     step(nw);
+    double rn, dtn;
+    // Mixed: step and rule are kept in front of what follows.  The compiler moves
+    // them behind the wait, which leaves the LDS latency of the poll and of the
+    // slot writes before it uncovered in every round (256^2 1.444 -> 1.422 ms, at
+    // a = 0.9 3.03 -> 2.97; in FP64 2 % slower).
+    if constexpr (MIXED) {
+      dtn = rule(nw, rn);
+#pragma unroll
+      for (int q = 1; q < 8; ++q) asm volatile("" : "+v"(nw[q]));
+      asm volatile("" : "+v"(dtn));
+    }
     // release the previous round here: its slot writes were issued a whole
     // RK4 step ago, so the release fence does not wait on them
     if (t > 0) publish(&ring.producedA, t);
@@ -192,12 +209,17 @@ __device__ __forceinline__ int tri_geodesic(TriRings<MIXED>& ring, const Params&
       ok = false;
       break;
     }
-    double rn;
-    const double dtn = rule(nw, rn);
+    if constexpr (!MIXED) dtn = rule(nw, rn);
     nacc += dtn != 0.0;
+    if constexpr (MIXED) {
 #pragma unroll
-    for (int q = 0; q < 8; ++q) out[q * 64] = nw[q];
-    out[8 * 64] = dtn != 0.0 && k + 1 < rp.N ? dt : 0.0;  // row N is never emitted
+      for (int q = 0; q < 3; ++q) out[q * 64] = nw[1 + q];
+      ring.av[t % DA][lane] = make_float4((float)nw[4], (float)nw[5], (float)nw[6], (float)nw[7]);
+    } else {
+#pragma unroll
+      for (int q = 0; q < 8; ++q) out[q * 64] = nw[q];
+    }
+    out[(CA - 1) * 64] = dtn != 0.0 && k + 1 < rp.N ? dt : 0.0;  // row N is never emitted
     if (ZONE) drdl = (rn - r) / dt;
 #pragma unroll
     for (int q = 0; q < 8; ++q) s[q] = nw[q];
@@ -239,17 +261,26 @@ __device__ __forceinline__ void tri_gather(TriRings<MIXED>& ring, int g, const S
       }
     }
     const double* in = &ring.a[t % DA][0][lane];
-    double pdt = in[8 * 64];
-    double ps[8];
+    double pdt = in[(R::kCompA - 1) * 64];
+    const double px = in[R::kPosA * 64], py = in[(R::kPosA + 1) * 64], pz = in[(R::kPosA + 2) * 64];
+    T mom[4];
+    if constexpr (MIXED) {
+      const float4 m = ring.av[t % DA][lane];
+      mom[0] = m.x;
+      mom[1] = m.y;
+      mom[2] = m.z;
+      mom[3] = m.w;
+    } else {
 #pragma unroll
-    for (int q = 0; q < 8; ++q) ps[q] = in[q * 64];
+      for (int q = 0; q < 4; ++q) mom[q] = in[(4 + q) * 64];
+    }
     publish(&ring.consumedA[g], t + 1);  // ring A slot is in registers
     T* ob = &ring.bt[t % DB][0][lane];
     T P[8];
 #pragma unroll
     for (int q = 0; q < 8; ++q) P[q] = T(0);
     if (pdt != 0.0) {
-      const Stencil stc = locate_cached(sv, sv.meta, sv.grid, ps[1], ps[2], ps[3], cmb, crec);
+      const Stencil stc = locate_cached(sv, sv.meta, sv.grid, px, py, pz, cmb, crec);
       if (stc.mb >= 0) {
         Corners cr;
         fetch<false>(sv, stc, cr);
@@ -259,8 +290,11 @@ __device__ __forceinline__ void tri_gather(TriRings<MIXED>& ring, int g, const S
     }
 #pragma unroll
     for (int q = 0; q < 8; ++q) ob[q * 64] = P[q];
+    ob[8 * 64] = (T)px;
+    ob[9 * 64] = (T)py;
+    ob[10 * 64] = (T)pz;
 #pragma unroll
-    for (int q = 1; q < 8; ++q) ob[(7 + q) * 64] = (T)ps[q];
+    for (int q = 0; q < 4; ++q) ob[(11 + q) * 64] = mom[q];
     ring.bd[t % DB][lane] = pdt;
     publish(&ring.producedB[g], t + 1);
   }
