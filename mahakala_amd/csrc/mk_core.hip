@@ -7,6 +7,7 @@
 #include <algorithm>
 #include <cstring>
 #include <mutex>
+#include <type_traits>
 #include <vector>
 
 #include "mk_device.h"
@@ -622,7 +623,7 @@ __global__ void __launch_bounds__(kScanThreads) k_solve_tiles(const double* j, c
   const bool mine = p < npx;
   const long rows = T - 1;  // scan row k is sample T - 1 - k
   double rj[kScanPer], ra[kScanPer], rd[kScanPer];
-  // beyond the rays and rows: zeros, which leave I as it is
+  // beyond the rays and rows: zeros
   auto load = [&](long k0) {
 #pragma unroll
     for (int u = 0; u < kScanPer; ++u) {
@@ -647,6 +648,9 @@ __global__ void __launch_bounds__(kScanThreads) k_solve_tiles(const double* j, c
     load(k0 + kScanRows);
     if (threadIdx.x < kScanRays) {
       constexpr int B = 4, N = kScanRows / B;  // rows per batch, batches
+      // The last tile stops at its last row: a zero row leaves a finite I as it
+      // is, but turns an infinite one into NaN (0 * inf).
+      const int left = (int)min((long)kScanRows, rows - k0);
       double jj[2][B], aa[2][B], tt[2][B];
       auto read = [&](int q) {
 #pragma unroll
@@ -659,17 +663,22 @@ __global__ void __launch_bounds__(kScanThreads) k_solve_tiles(const double* j, c
           tt[q & 1][u] = vt.x; tt[q & 1][u + 1] = vt.y;
         }
       };
-      read(0);
+      auto scan = [&](auto whole) {
+        read(0);
 #pragma unroll
-      for (int q = 0; q < N; ++q) {
-        if (q + 1 < N) read(q + 1);
+        for (int q = 0; q < N; ++q) {
+          if (!whole && q * B >= left) break;
+          if (q + 1 < N) read(q + 1);
 #pragma unroll
-        for (int u = 0; u < B; ++u) {
-          const double d = tt[q & 1][u] * (jj[q & 1][u] - (aa[q & 1][u] * Iv));
-          Iv = Iv + d;
-          if (DI) sj[ray][q * B + u] = d;
+          for (int u = 0; u < B; ++u) {
+            const double d = tt[q & 1][u] * (jj[q & 1][u] - (aa[q & 1][u] * Iv));
+            Iv = whole || q * B + u < left ? Iv + d : Iv;
+            if (DI) sj[ray][q * B + u] = d;
+          }
         }
-      }
+      };
+      if (left == kScanRows) scan(std::true_type{});
+      else scan(std::false_type{});
     }
     __syncthreads();
     if (DI) {

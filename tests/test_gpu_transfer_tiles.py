@@ -31,3 +31,28 @@ def test_tile_scans_equal_one_thread_per_ray(T):
         for i in range(T - 1, 0, -1):
             ref = ref - dt[i - 1] * 0.5 * (j[i] - al[i] * ref)
     np.testing.assert_allclose(I, ref, rtol=1e-12)
+
+
+@pytest.mark.parametrize("T", [2, 3, 5, 17, 64, 65, 66, 129, 130, 300])
+def test_infinite_intensities_stay_infinite(T):
+    """Intensities that become infinite in the row nearest the camera, with T - 1
+    on and off a multiple of the tile: no row behind the last one is added."""
+    rng = np.random.Generator(np.random.PCG64(T))
+    j, al = rng.exponential(1.0, (2, T, MANY))
+    dt = -rng.exponential(0.1, (T, MANY))
+    j[1, 1], j[1, 2] = np.inf, -np.inf
+    j[1, 3], dt[0, 3] = 1e308, -100.0  # overflows
+    j[1, 4], dt[0, 4] = np.inf, 0.0    # 0 * inf: NaN in the reference too
+    I, dI = transfer.solve_specific_intensity(j, al, dt, 0.5, dIs=True)
+    ref = np.zeros(MANY)
+    with np.errstate(invalid="ignore", over="ignore"):
+        for i in range(T - 1, 0, -1):
+            ref = ref - dt[i - 1] * 0.5 * (j[i] - al[i] * ref)
+    np.testing.assert_array_equal(ref[1:4], [np.inf, -np.inf, np.inf])
+    np.testing.assert_array_equal(I[1:5], ref[1:5])
+    for n in (5, 16, 33):
+        a = [np.ascontiguousarray(v[:, :n]) for v in (j, al, dt)]
+        np.testing.assert_array_equal(transfer.solve_specific_intensity(*a, 0.5), I[:n])
+        In, dIn = transfer.solve_specific_intensity(*a, 0.5, dIs=True)
+        np.testing.assert_array_equal(In, I[:n])
+        np.testing.assert_array_equal(dIn, dI[:, :n])
