@@ -770,7 +770,8 @@ __device__ __forceinline__ void fluid_scalars32(const float P[8], float x, float
 // and cos(pitch) = u^t k.b / (|k.u| sqrt W).  Square roots come with their
 // reciprocals; no division is left.
 struct Fluid64 {
-  double cosp, kdotu, ikdotu;  // cos(pitch), k.u, 1/(k.u)
+  double cosp, kdotu, ikdotu;  // cos(pitch) (the fallback's where k.u = 0), k.u, 1/(k.u)
+  double kb;                   // u^t k.b
   double W, sW, iW;            // (u^t)^2 b.b, its square root and 1/square root (NaN where W = 0)
   double u0, iu0;              // u^t, 1/u^t
 };
@@ -794,8 +795,8 @@ __device__ __forceinline__ Fluid64 fluid64(const double P[8], double x, double y
   o.W = B1 * B1 + B2 * B2 + B3 * B3 + flB * lB + bt * bt;
   M::sqrt_rcp3(o.W, o.sW, o.iW);
   o.ikdotu = M::rcp3(o.kdotu);
-  const double kb = k1 * B1 + k2 * B2 + k3 * B3 + flB * Lk + o.kdotu * bt;
-  double p = kb * o.iW * __builtin_fabs(o.ikdotu);
+  o.kb = k1 * B1 + k2 * B2 + k3 * B3 + flB * Lk + o.kdotu * bt;
+  double p = o.kb * o.iW * __builtin_fabs(o.ikdotu);
   if (is_nan(p)) p = fallback_cos;
   if (__builtin_fabs(p) > 1.0) p = __builtin_copysign(1.0, p);
   o.cosp = p;

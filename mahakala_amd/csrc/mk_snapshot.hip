@@ -174,7 +174,10 @@ __global__ void __launch_bounds__(256) k_sample_scalars(SnapView sv, const doubl
   double P[8];
   trilinear<double>(sv, q[1], q[2], q[3], P);
   const Fluid64 F = fluid64(P, q[1], q[2], q[3], q[4], q[5], q[6], q[7], a, fbc);
-  const double sc[5] = {P[0], P[1], ::acos(F.cosp), F.kdotu, F.W == 0.0 ? 0.0 : F.sW * F.iu0};
+  // k.u = 0 (not of a photon): k.b / (|k.u| |b|) is infinite and clamped; 1/(k.u) came out NaN
+  double cosp = F.cosp;
+  if (F.kdotu == 0.0 && F.W > 0.0 && __builtin_fabs(F.kb) > 0.0) cosp = __builtin_copysign(1.0, F.kb);
+  const double sc[5] = {P[0], P[1], ::acos(cosp), F.kdotu, F.W == 0.0 ? 0.0 : F.sW * F.iu0};
 #pragma unroll
   for (int c = 0; c < 5; ++c) {
     if constexpr (STREAM) __builtin_nontemporal_store(sc[c], out + c * n + p);

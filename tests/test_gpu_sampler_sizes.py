@@ -33,3 +33,26 @@ def test_scalars_do_not_depend_on_the_launch(n):
     idx = torch.arange(n, device="cuda") % base
     got, ref = sample(S[idx].contiguous()), sample(S)[:, idx]
     assert torch.equal(got.view(torch.int64), ref.contiguous().view(torch.int64))
+
+
+def test_pitch_of_momenta_orthogonal_to_the_flow():
+    """k.u = 0 exactly (k^t = 0 in a flow at rest in the normal frame): the cosine
+    k.b / (|k.u| |b|) is infinite and clamped to +-1; the fallback angle is for
+    0/0 only, k.b = 0 or b = 0 (athenak.py:787-793)."""
+    ds = syn.torus_snapshot(0.0, nblocks=2, n=8)
+    ds["uov"][1:4] = 0.0
+    ds["B"][:] = 0.0
+    ds["B"][0] = 1.0
+    ds["B"][:, 0] = 0.0  # no field in the first block
+    m = AthenakFluidModel.from_datasets(ds, 0.0, fluid_gamma=13. / 9)
+    rng = np.random.Generator(np.random.PCG64(2))
+    S = np.zeros((400, 8))
+    S[:, 1:4] = rng.uniform(-30, 30, (400, 3))
+    S[:, 5] = rng.uniform(0.1, 1.0, 400) * np.where(rng.uniform(size=400) < 0.5, -1, 1)
+    S[::5, 5] = 0.0  # k = 0
+    sc = m.get_fluid_scalars_from_geodesics(S[None])
+    assert not np.asarray(sc["kdotu"]).any()
+    b, pitch = np.asarray(sc["b"])[0], np.asarray(sc["pitch_angle"])[0]
+    assert 0 < (b == 0).sum() < 400
+    want = np.where((b == 0) | (S[:, 5] == 0), np.arccos(np.cos(np.pi / 3)), np.where(S[:, 5] > 0, 0.0, np.pi))
+    np.testing.assert_allclose(pitch, want, rtol=0, atol=4e-16)
