@@ -503,14 +503,14 @@ std::vector<int> ring_first_tile_order(int res, double lo, double step, double a
 
 // Device copies of tile orders, one per (device, resolution, fov, spin,
 // inclination), made on first use and kept until the process ends (immutable,
-// so launches in flight never see them change).  Past kOrderCacheBytes, or
-// while the stream is being captured into a graph (no allocation there),
-// launches use row-major tiles.
+// so launches in flight never see them change).  An entry is published only
+// once its copy is in memory: any stream may use it from then on.  Past
+// kOrderCacheBytes, or while the stream is being captured into a graph (no
+// allocation there), launches use row-major tiles.
 namespace {
 std::mutex g_order_mu;
-// device table and the host copy it was filled from (kept, so that the
-// stream-ordered copy never reads freed memory)
-std::map<std::tuple<int, int, double, double, double>, std::pair<int*, std::vector<int>>> g_orders;
+std::map<std::tuple<int, int, double, double, double>, int*> g_orders;
+std::map<int, hipStream_t> g_order_streams;  // per device, for these copies alone
 size_t g_order_bytes = 0;
 constexpr size_t kOrderCacheBytes = (size_t)64 << 20;
 }  // namespace
@@ -545,7 +545,7 @@ static const int* render_tile_order(const RenderDev& rp, const mk_render_params*
   const auto key = std::make_tuple(dev, rp.res, p->fov, p->bhspin, p->inclination);
   std::lock_guard<std::mutex> lk(g_order_mu);
   auto it = g_orders.find(key);
-  if (it != g_orders.end()) return it->second.first;
+  if (it != g_orders.end()) return it->second;
   hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
   if (hipStreamIsCapturing(st, &cap) != hipSuccess || cap != hipStreamCaptureStatusNone) return nullptr;
   const size_t bytes = (size_t)rp.ntiles * sizeof(int);
@@ -553,12 +553,22 @@ static const int* render_tile_order(const RenderDev& rp, const mk_render_params*
   std::vector<int> ord = ring_first_tile_order(rp.res, rp.lo, rp.step, p->bhspin, p->inclination);
   int* d = nullptr;
   if (hipMalloc(&d, bytes) != hipSuccess) return nullptr;
-  // ordered on the caller's stream before the launch that reads it
-  if (hipMemcpyAsync(d, ord.data(), bytes, hipMemcpyHostToDevice, st) != hipSuccess) {
+  // on the caller's stream if it is idle, else on one of its own (made once, 4 ms), so as not to wait for that work
+  hipStream_t copy = st;
+  hipError_t e = hipStreamQuery(st);
+  if (e == hipErrorNotReady) {
+    (void)hipGetLastError();
+    hipStream_t& own = g_order_streams[dev];
+    e = own ? hipSuccess : hipStreamCreateWithFlags(&own, hipStreamNonBlocking);
+    copy = own;
+  }
+  if (e == hipSuccess) e = hipMemcpyAsync(d, ord.data(), bytes, hipMemcpyHostToDevice, copy);
+  if (e == hipSuccess) e = hipStreamSynchronize(copy);
+  if (e != hipSuccess) {
     (void)hipFree(d);
     return nullptr;
   }
-  g_orders.emplace(key, std::make_pair(d, std::move(ord)));
+  g_orders.emplace(key, d);
   g_order_bytes += bytes;
   return d;
 }
