@@ -1058,6 +1058,7 @@ int mk_integrate_rows(const double* d_s0, long n, int N, double div, double tol,
   if (int rc = mk_trim_rows(d_K, n, N, h_T, s)) return rc;
   k_repeat_rows<<<grid_for(n * *h_T, kBlock), kBlock, 0, as_stream(s)>>>(d_K, n, *h_T, d_S, d_dt);
   MK_LAUNCH_CHECK();
+  MK_HIP(hipStreamSynchronize(as_stream(s)));  // the rows are written and d_K is no longer read
   return MK_OK;
 }
 

@@ -6,6 +6,8 @@ others share its wave, and nothing is written past the last one.  The
 bisection's schedule (lanes per angle, width of the band, angles per wave)
 changes no radius.
 """
+import ctypes as C
+
 import numpy as np
 import pytest
 import torch
@@ -101,3 +103,27 @@ def test_history_in_one_walk_of_rays_that_are_all_frozen():
     np.testing.assert_array_equal(np.asarray(S), np.asarray(S2))
     np.testing.assert_array_equal(np.asarray(D), np.asarray(D2))
     assert not np.asarray(D).any()
+
+
+def test_history_in_one_walk_is_complete_on_return():
+    """mk_integrate_rows synchronises its stream: on return the rows behind each
+    ray's last one are written too, also on a stream that no other waits for."""
+    n, N = 50000, 400
+    s0 = _start(144)[torch.arange(n, device="cuda") % 144].contiguous()
+    s0[:, 1:4] *= 10.0  # beyond 1500 M: frozen from row 0, all their rows repeat
+    s0[7] = _start(8)[7]
+    S = torch.full((N, n, 8), GUARD, device="cuda", dtype=torch.float64)
+    D = torch.full((N, n), GUARD, device="cuda", dtype=torch.float64)
+    K = torch.empty(n, device="cuda", dtype=torch.int32)
+    T = C.c_long()
+    torch.cuda.synchronize()
+    st = torch.cuda.Stream()
+    _lib.check(_lib.lib().mk_integrate_rows(s0.data_ptr(), n, N, 40.0, 1e-2, 0.9, S.data_ptr(), D.data_ptr(),
+                                            K.data_ptr(), C.byref(T), st.cuda_stream))
+    done = st.query()
+    with torch.cuda.stream(torch.cuda.Stream()):
+        rest = S[T.value - 1].cpu()
+    assert done
+    st.synchronize()
+    rows = torch.arange(n) != 7
+    assert torch.equal(rest[rows], s0.cpu()[rows]) and not D[:T.value].cpu()[:, rows].any()
