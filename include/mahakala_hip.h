@@ -294,6 +294,10 @@ typedef struct mk_server_config {
  * per tile).  The same image, bit for bit.  Above 256^2 that call builds
  * mk_render's tile order for the view, as mk_render's own first call does. */
 #define MK_SERVER_IMAGE_IN_LAUNCH 4
+/* Testing aid for launches of four waves per tile: every bounded wait between
+ * the waves of a tile gives up after one poll.  The server then reports an
+ * error (MK_ERR_STATE), and the request of such a tile never completes. */
+#define MK_SERVER_WAIT_TEST 8
 
 typedef struct mk_image_request {
   int32_t snapshot;         /* id from mk_server_add_snapshot */

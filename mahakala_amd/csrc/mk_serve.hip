@@ -460,6 +460,7 @@ struct PArgs {
   unsigned long long* busy;     // device: lane-steps that advanced a ray
   unsigned long long* total;    // device: 64 x the wave-steps of every tile run
   int seg_cap, idle_limit, first_seg;
+  int spin_limit;               // polls before a wait between a tile's waves gives up
 };
 
 constexpr unsigned long long kHalt = 1ull << 62;  // in `seen`: the host has set stop
@@ -765,7 +766,7 @@ __global__ void __launch_bounds__(256, 4) k_serve_tri(const ReqDev* __restrict__
       const ReqDev& q = req[sg.desc];
       const int px = pixel(q, (int)(t - sg.start) * kTile + lane);
       int n;
-      const int rounds = tri_geodesic<MIXED, false>(ring, q, kSpinLimit, grid_coord(q.lo, q.step, px / q.res),
+      const int rounds = tri_geodesic<MIXED, false>(ring, q, P.spin_limit, grid_coord(q.lo, q.step, px / q.res),
                                                     grid_coord(q.lo, q.step, px % q.res), px >= 0, n);
       unsigned long long w = (unsigned long long)(px >= 0 && n > 0 ? n : 0);
       for (int off = 32; off > 0; off >>= 1) w += __shfl_xor(w, off);
@@ -779,7 +780,7 @@ __global__ void __launch_bounds__(256, 4) k_serve_tri(const ReqDev* __restrict__
     while (true) {
       __syncthreads();
       if (shared_int(s_state) <= 0) break;
-      tri_gather<MIXED>(ring, wave - 1, req[shared_int(s_desc)].sv, kSpinLimit);
+      tri_gather<MIXED>(ring, wave - 1, req[shared_int(s_desc)].sv, P.spin_limit);
       __syncthreads();
     }
   } else {
@@ -789,13 +790,14 @@ __global__ void __launch_bounds__(256, 4) k_serve_tri(const ReqDev* __restrict__
       const int tile = shared_int(s_tile), rid = shared_int(s_rid), seq = shared_int(s_seq);
       const ReqDev& q = req[shared_int(s_desc)];
       bool ok;
-      const double I = tri_emission<MIXED>(ring, q, kSpinLimit, ok);
+      const double I = tri_emission<MIXED>(ring, q, P.spin_limit, ok);
       const int px = pixel(q, tile * kTile + lane);
       if (px >= 0) q.out[px] = I;
-      if (!ok && lane == 0) __hip_atomic_store(&P.ctl->err, 5, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
       // as in k_serve_persistent: the outputs, then the count, then the flag
       __builtin_amdgcn_fence(__ATOMIC_RELEASE, "");
-      if (lane == 0) {
+      if (!ok) {  // the tile is never counted, so its request never completes
+        if (lane == 0) __hip_atomic_store(&P.ctl->err, 5, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+      } else if (lane == 0) {
         const int n = min(kTile, q.n_items - tile * kTile);
         const int old = __hip_atomic_fetch_add(&P.done[rid], n, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         if (old + n >= q.n_items) {
@@ -1491,6 +1493,7 @@ bool launch_persistent(mk_server* s) {
   P.done = s->d_pdone;
   P.seg_cap = s->seg_cap;
   P.idle_limit = kPersistWaitSleeps;
+  P.spin_limit = (s->cfg.flags & MK_SERVER_WAIT_TEST) ? 1 : kSpinLimit;
   store_shared(&s->p_ctl->stop, 0);
   s->stopping = false;
   s->want_shadow = false;

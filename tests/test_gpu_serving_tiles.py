@@ -1,12 +1,14 @@
 """Image-only launches of the persistent server: four waves per tile, or one
 wave per tile when the launch starts with a deep backlog (images.py:30-144 of
 the reference).  Both give mk_render's bits, whatever the tile count."""
+import ctypes as C
 import time
 
 import numpy as np
 import pytest
 
-from mahakala_amd import images
+from mahakala_amd import _lib, images
+from mahakala_amd.constants import Msun
 from mahakala_amd.grmhd import synthetic as syn
 from mahakala_amd.grmhd.athenak import AthenakFluidModel
 from mahakala_amd.serving import Server
@@ -62,3 +64,32 @@ def test_deep_backlog_behind_a_shallow_launch(model, precision):
     assert st["completed"] == 13 and st["in_flight"] == 0 and st["iterations"] >= 2
     for v, img in zip([first] + later, got):
         np.testing.assert_array_equal(img, _render(model, v, precision), err_msg=str(v))
+
+
+@pytest.mark.parametrize("precision", [0, 1])
+def test_a_tile_whose_waves_gave_up_does_not_complete_its_request(model, precision):
+    """With a limit of one poll the waves of a tile give up on each other: the
+    server reports it, and no request is handed out as completed with the NaN of
+    such a tile."""
+    lib, n = _lib.lib(), 64
+    cfg = _lib.mk_server_config(precision, 0, 0, 0, 0, 0, 1 | 4 | 8)  # PERSISTENT, IMAGE_IN_LAUNCH, WAIT_TEST
+    h, sid, rid = _lib.vp(), C.c_int32(), C.c_int64()
+    _lib.check(lib.mk_server_create(C.byref(cfg), C.byref(h)))
+    try:
+        _lib.check(lib.mk_server_add_snapshot(h, model.device_snapshot.handle, C.byref(sid)))
+        out = np.full((n, 16, 16), -7.0)
+        ids = []
+        for k in range(n):
+            req = _lib.mk_image_request(sid.value, 16, 10000, 0, 0.9, 30.0 + k / 4, 1000.0, 10.0, 230e9, 1e26, 6.2e9 * Msun,
+                                        40.0, 13. / 9)
+            if lib.mk_server_submit_image(h, C.byref(req), out[k].ctypes.data, C.byref(rid)):
+                break  # the error is out already
+            ids.append(rid.value)
+        assert ids
+        assert {lib.mk_server_wait(h, i, 30.0) for i in ids + [-1]} == {-5}  # MK_ERR_STATE
+        assert b"waited longer than its limit" in lib.mk_last_error()
+        st = _lib.mk_server_stats()
+        assert lib.mk_server_get_stats(h, C.byref(st)) == -5  # filled in all the same
+        assert st.completed == 0 and (out == -7.0).all()
+    finally:
+        _lib.check(lib.mk_server_destroy(h))
