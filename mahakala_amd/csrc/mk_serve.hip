@@ -909,6 +909,7 @@ struct mk_server {
   std::chrono::steady_clock::time_point launch_t0;
   std::map<std::pair<int, double>, std::vector<int>> orders;  // tile orders by (resolution, fov)
   std::deque<Pending> waiting;         // by priority, then submit order
+  long long backlog = 0;               // work items of the requests waiting and in flight
   Pending running{};                   // the request the idle worker runs itself
   int64_t running_id = 0;              // its id while it runs, else 0
   std::set<int64_t> cancelled;         // ids removed from the queue (the newest kCancelledKept)
@@ -936,9 +937,15 @@ constexpr int kDirectShadowAngles = 1024;         // bisections an idle server r
 constexpr int kDirectImageRes = 512;              // and images, when one is all it has
 constexpr size_t kCancelledKept = size_t(1) << 16; // cancelled ids remembered for mk_server_wait
 
+// Work items of a request: pixels or angles.
+long long items_of(const mk_server::Pending& p) {
+  return p.kind == kKindImage ? (long long)p.img.resolution * p.img.resolution : p.sh.n_angles;
+}
+
 // Queues a request behind every queued one of the same or a higher priority
 // (caller holds mu).
 void enqueue(mk_server* s, mk_server::Pending&& p) {
+  s->backlog += items_of(p);
   auto it = s->waiting.end();
   while (it != s->waiting.begin() && std::prev(it)->priority < p.priority) --it;
   s->waiting.insert(it, std::move(p));
@@ -1222,6 +1229,7 @@ bool collect(mk_server* s) {
     s->unpolled.emplace_back(id, ms);
     ++s->st.completed;
     s->st.items_done += n_items;
+    s->backlog -= n_items;
   }
   if (!fin.empty()) s->cv_done.notify_all();
   return true;
@@ -1253,6 +1261,7 @@ bool serve_direct(mk_server* s) {
     std::lock_guard<std::mutex> lk(s->mu);
     s->running = std::move(s->waiting.front());
     s->waiting.pop_front();
+    s->backlog -= items_of(s->running);
     s->running_id = s->running.id;
     if (s->running.kind == kKindImage) snap = s->snaps[s->running.img.snapshot];
   }
@@ -1364,19 +1373,10 @@ T load_shared(const T* p) {
 // many times the deep backlog (kDeepTilesPerWave) has gathered.
 constexpr int kDeepRelaunch = 4;
 
-// Work items queued or in flight (caller holds mu).
-long long backlog_items(const mk_server* s) {
-  long long items = 0;
-  for (const auto& kv : s->flight) items += kv.second.n_items;
-  for (const auto& p : s->waiting)
-    items += p.kind == kKindImage ? (long long)p.img.resolution * p.img.resolution : p.sh.n_angles;
-  return items;
-}
-
 void admit_persistent(mk_server* s) {
   if (s->launched && s->stopping) return;  // the waves may be leaving: nothing is published until the launch ends
   if (s->launched && s->launch_tri && !s->want_deep && !s->waiting.empty())
-    s->want_deep = backlog_items(s) >= (long long)kDeepRelaunch * kDeepTilesPerWave * s->L;
+    s->want_deep = s->backlog >= (long long)kDeepRelaunch * kDeepTilesPerWave * s->L;
   if (s->launched && s->want_deep) return;  // the next launch takes the queue
   bool any = false;
   while (!s->draining && !s->waiting.empty() && !s->free_rids.empty()) {
@@ -1469,6 +1469,7 @@ void collect_persistent(mk_server* s) {
     s->unpolled.emplace_back(id, ms);
     ++s->st.completed;
     s->st.items_done += n_items;
+    s->backlog -= n_items;
   }
   if (!fin.empty()) s->cv_done.notify_all();
 }
@@ -1618,7 +1619,7 @@ void worker_persistent(mk_server* s) {
       stop_persistent(s);  // nothing in flight: the next request relaunches
     }
     if (!s->launched && !s->flight.empty()) {
-      s->launch_deep = backlog_items(s) >= (long long)kDeepTilesPerWave * s->L;  // under mu
+      s->launch_deep = s->backlog >= (long long)kDeepTilesPerWave * s->L;  // under mu
       if (!ready) {
         ready = true;
         ready_since = now;
@@ -1837,6 +1838,7 @@ int mk_server_cancel(mk_server* s, int64_t id, int32_t* h_cancelled) {
   *h_cancelled = 0;
   for (auto it = s->waiting.begin(); it != s->waiting.end(); ++it) {
     if (it->id != id) continue;
+    s->backlog -= items_of(*it);
     s->waiting.erase(it);
     if (s->cancelled_order.size() >= kCancelledKept) {
       s->cancelled.erase(s->cancelled_order.front());
