@@ -7,6 +7,7 @@ import time
 import numpy as np
 import pytest
 
+import mahakala_amd as ma
 from mahakala_amd import _lib, images
 from mahakala_amd.constants import Msun
 from mahakala_amd.grmhd import synthetic as syn
@@ -93,3 +94,30 @@ def test_a_tile_whose_waves_gave_up_does_not_complete_its_request(model, precisi
         assert st.completed == 0 and (out == -7.0).all()
     finally:
         _lib.check(lib.mk_server_destroy(h))
+
+
+@pytest.mark.parametrize("shadows", [False, True])
+def test_many_requests_published_together(model, shadows):
+    """Requests of one published batch share a copy to device memory: small and
+    large tile orders, images without one (size not a multiple of 8), one too long
+    to be copied, and bisections between them, behind an image that keeps the
+    launch busy while they gather."""
+    sizes = [256] + [8, 16, 8, 33, 64, 8, 8, 7, 24, 8, 8, 8, 8, 8, 8, 8, 8, 8, 8, 128, 160, 9, 16, 8, 1032, 8, 48] * 2 + [8] * 70
+    views = [dict(resolution=r, inclination=5.0 + (7 * k) % 80, max_nsteps=10000 if r < 1000 else 340)
+             for k, r in enumerate(sizes)]
+    ang = np.arange(5.0)
+    with Server("mixed", image_in_launch=True, shadow_in_launch=True) as srv:
+        sid = srv.add_snapshot(model)
+        for _ in range(2):
+            rids = []
+            for k, v in enumerate(views):
+                rids.append(_submit(srv, sid, v))
+                if shadows and k % 11 == 0:
+                    rids.append(srv.submit_shadow(0.9, 60.0, ang + k, max_steps=50))
+            got = [srv.result(r, timeout=60) for r in rids]
+    images_got = [g for g in got if g.ndim == 2]
+    for v, img in zip(views, images_got):
+        np.testing.assert_array_equal(img, _render(model, v, "mixed"), err_msg=str(v))
+    if shadows:
+        want = [ma.find_shadow_bisection_angles(0.9, 60.0, ang + k, max_steps=50) for k in range(0, len(views), 11)]
+        np.testing.assert_array_equal([g for g in got if g.ndim == 1], want)
