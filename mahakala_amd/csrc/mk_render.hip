@@ -677,8 +677,17 @@ static int choose_form(const SnapView& sv, const RenderDev& rp, int precision, i
   // i = 60 deg, 640^2 5.14 and 6.95 (6.93 and 8.29), 768^2 7.22 and 7.29 (9.7 and
   // 8.5); a = 0.97, i = 80 deg, 768^2 7.24 and 13.1 (9.7 and 15.6), 1024^2 12.8
   // and 15.5 (17.1 and 18.5) ms.
-  const double x2 = rp.a * rp.a * rp.si * rp.si;
-  const double scale = x2 > 0.25 ? (x2 < 0.75 ? 1.0 / (1.0 - x2) : 4.0) : 1.0;
+  // The line moves with the field of view f (in M) too: the wider, the smaller the
+  // share of tiles with long rays, and the more such a launch waits for them.
+  // Times where the forms are level, in tiles per CU, |a sin i| <= 0.25, mixed (FP64):
+  // f = 5 M 5 (3), 8 M 10 (6), 12 M 11 (8), 20 M 16 (12), 36 M 20 (17), 60 M 28 (22),
+  // 100 M 36 (32), 300 M 36 (34).  The factor f / (0.355 f + 12.9) is 1 at 20 M and
+  // 0.34, 0.70, 1.75 and 2.5 at 5, 12, 60 and 300 M.  Octree of 512 blocks, mixed,
+  // a = 0, f = 60 M, 512^2: triple 2.06, classic 3.14 ms; a = 0.9, i = 60 deg, f = 12 M,
+  // 768^2 9.1 and 7.7 ms.  At most 8 in all: 1408^2 is the largest image measured.
+  const double x2 = rp.a * rp.a * rp.si * rp.si, f = std::fabs(2.0 * rp.lo);
+  const double edge = x2 > 0.25 ? (x2 < 0.75 ? 1.0 / (1.0 - x2) : 4.0) : 1.0;
+  const double scale = std::min(edge * f / (0.355 * f + 12.9), 8.0);
   if ((double)(2 * rp.ntiles) <= scale * (double)((precision == 1 ? 31L : 22L) * cus)) *form = MK_RENDER_TRIPLE;
   return MK_OK;
 }
