@@ -211,9 +211,9 @@ typedef struct mk_render_params {
 /* mk_render_params.flags: kernel form.  By default the library runs a launch
  * of up to 15.5 8x8 tiles per CU (11 in FP64; up to four times as many at
  * views with |a sin i| > 0.5; fewer below and up to 2.8 times as many above a
- * field of view of 20 M) in the triple form -- a geodesic wave, two gather waves (block lookup, cell loads, interpolation) and an
- * emission wave per tile -- and a larger one in the classic form (one wave
- * per tile).  The paired form (a geodesic wave and a transfer wave per tile)
+ * field of view of 20 M) in the triple form -- a geodesic wave, two gather
+ * waves (block lookup, cell loads, interpolation) and an emission wave per
+ * tile -- and a larger one in the classic form (one wave per tile).  The paired form (a geodesic wave and a transfer wave per tile)
  * runs only when forced and its tables fit in LDS (else the classic form).
  * The bits force one form; all give the same image, bit for bit. */
 #define MK_RENDER_CLASSIC 1

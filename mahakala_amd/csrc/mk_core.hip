@@ -3,6 +3,7 @@
 #include <hip/hip_runtime.h>
 
 #include <cmath>
+#include <cstdint>
 #include <cstdlib>
 #include <algorithm>
 #include <cstring>
@@ -613,6 +614,24 @@ constexpr int kScanPitch = kScanRows + 2;  // a lane's 16-byte reads of 16 rays 
 // 1240 rows 184 / 292 against 198 / 298 us, at 150 rows 22 / 31 against 22 /
 // 32; 65536 rays 365 / 574 against 312 / 477 us.
 constexpr long kScanMaxRays = 32768;
+// And from half a tile of rows, or a whole one beyond 16384 rays: fewer rows are
+// read in one go by a thread per ray too, while a tile costs its loads and
+// barriers.  Intensities with the increments / attenuated emission, tiles against
+// one thread per ray: 16384 rays of 17 rows 5.3 / 5.4 against 4.5 / 4.4 us, of 33
+// 6.6 / 6.0 against 6.5 / 6.4; 32768 rays of 33 rows 9.8 / 9.0 against 7.1 / 7.1,
+// of 65 14.2 / 13.4 against 15.1 / 13.8; 4096 rays of 33 rows 4.3 / 4.1 against
+// 6.1 / 6.1.
+// Where a block's 16 rays are not one 128-byte line of a row (a number of rays that
+// is no multiple of 16), two blocks, mostly of two XCDs, fetch each line, and the
+// tiles pay up to 12288 rays only: intensities of 300 rows 12001 rays 27.5 against
+// 29.9 us (12000: 18.2 against 29.6), 16383 38.4 against 30.4, 32767 67.2 against
+// 38.4.
+constexpr long kScanMaxSplitRays = 12288;
+
+static bool scan_tiles(const double* j, const double* al, const double* dt, long T, long npx) {
+  const bool lines = npx % kScanRays == 0 && ((uintptr_t)j | (uintptr_t)al | (uintptr_t)dt) % 128 == 0;
+  return npx <= (lines ? kScanMaxRays : kScanMaxSplitRays) && T - 1 >= (npx <= 16384 ? kScanRows / 2 : kScanRows);
+}
 
 template <bool DI>
 __global__ void __launch_bounds__(kScanThreads) k_solve_tiles(const double* j, const double* al, const double* dt,
@@ -1416,7 +1435,7 @@ int mk_solve_intensity(const double* j, const double* al, const double* dt, long
                        double* dI, void* s) {
   MK_REQUIRE(T >= 0 && npx >= 0 && j && al && dt && I, "mk_solve_intensity: bad arguments");
   if (!npx) return MK_OK;
-  if (npx <= kScanMaxRays)
+  if (scan_tiles(j, al, dt, T, npx))
     (dI ? k_solve_tiles<true> : k_solve_tiles<false>)<<<grid_for(npx, kScanRays), kScanThreads, 0, as_stream(s)>>>(
         j, al, dt, T, npx, L, I, dI);
   else
@@ -1429,7 +1448,7 @@ int mk_attenuated_emissivity(const double* j, const double* al, const double* dt
                              double* out, void* s) {
   MK_REQUIRE(T >= 0 && npx >= 0 && j && al && dt && out, "mk_attenuated_emissivity: bad arguments");
   if (!npx || T < 2) return MK_OK;
-  if (npx <= kScanMaxRays)
+  if (scan_tiles(j, al, dt, T, npx))
     k_attenuated_tiles<<<grid_for(npx, kScanRays), kScanThreads, 0, as_stream(s)>>>(j, al, dt, T, npx, L, out);
   else
     k_attenuated<<<grid_for(npx, kBlock), kBlock, 0, as_stream(s)>>>(j, al, dt, T, npx, L, out);

@@ -3,8 +3,9 @@
 edges of the 64-row tiles and 16-ray blocks."""
 import numpy as np
 import pytest
+import torch
 
-from mahakala_amd import transfer
+from mahakala_amd import _lib, transfer
 
 pytestmark = pytest.mark.gpu
 MANY = 32768 + 17  # beyond the tile kernels' range
@@ -56,3 +57,35 @@ def test_infinite_intensities_stay_infinite(T):
         In, dIn = transfer.solve_specific_intensity(*a, 0.5, dIs=True)
         np.testing.assert_array_equal(In, I[:n])
         np.testing.assert_array_equal(dIn, dI[:, :n])
+
+
+@pytest.mark.parametrize("T", [32, 33, 64, 65])
+def test_every_choice_of_kernel_gives_the_same_bits(T):
+    """By rows, rays and whether a block's rays are one line of a row: numbers of
+    rays on both sides of each limit, and arrays that start off a line."""
+    n = 40000
+    g = torch.Generator(device="cuda").manual_seed(T)
+    j, al, dt = (torch.empty(T, n, device="cuda", dtype=torch.float64).exponential_(1.0, generator=g) for _ in range(3))
+    dt *= -0.1
+
+    def scan(v, shift=0):
+        k = v[0].shape[1]
+        p = []
+        for x in v:  # copies at a byte offset of 8 * shift
+            buf = torch.empty(T * k + shift, device="cuda", dtype=torch.float64)
+            buf[shift:] = x.reshape(-1)
+            p.append(buf[shift:])
+        I = torch.empty(k, device="cuda", dtype=torch.float64)
+        dI, att = torch.empty((2, T - 1, k), device="cuda", dtype=torch.float64)
+        a = [x.data_ptr() for x in p]
+        _lib.check(_lib.lib().mk_solve_intensity(*a, T, k, 0.5, I.data_ptr(), dI.data_ptr(), None))
+        _lib.check(_lib.lib().mk_attenuated_emissivity(*a, T, k, 0.5, att.data_ptr(), None))
+        torch.cuda.synchronize()
+        return I, dI, att
+
+    ref = scan([j, al, dt])
+    for k, shift in [(16, 0), (17, 0), (12287, 0), (12288, 0), (12288, 1), (12289, 0), (12304, 0), (12304, 3), (16384, 0), (16385, 0),
+                     (16400, 0), (32752, 0), (32768, 0), (32784, 0)]:
+        got = scan([x[:, :k].contiguous() for x in (j, al, dt)], shift)
+        for a, b in zip(got, ref):
+            assert torch.equal(a, b[..., :k]), (k, shift)
