@@ -157,12 +157,14 @@ __global__ void __launch_bounds__(256) k_sample_prims(SnapView sv, const double*
 // per SIMD hide three loads in sequence (lookup record, record, cells) behind
 // 530 instructions.  More waves (launch bounds 5: spills) and a grid of
 // resident blocks that load the next state early are both slower (141 and 140
-// against 125 us at 3.4e6 samples).  STREAM: the outputs bypass the caches'
-// retention, which keeps them from evicting states and cells.  Measured
-// (samples: without, with; in blocks of 64): 4.1e5: 9.5, 7.8 us but followed by a
-// reader of the outputs 18.0, 19.3; 1.6e6: 62, 59 (65); 3.4e6: 125, 112 (107);
-// 6.6e6: 207, 204 (186).
-constexpr long kStreamSamples = 1500000, kSmallBlockSamples = 3000000;
+// against 125 us at 3.4e6 samples).  Large launches run in blocks of 64: 1.6e6 samples
+// 74 us (blocks of 256: 72), 2.5e6 101 (101), 3.4e6 116 (122), 6.6e6 184 (200).
+// STREAM: the outputs bypass the caches' retention.  Alone the sampler takes the same
+// time with and without, from 1.6e6 to 2.7e7 samples; followed by the synchrotron
+// kernel, which reads all five outputs, 1.6e6 samples take 93 us with and 91 without,
+// 3.4e6 146.0 and 145.1, 6.6e6 242 and 245, 8.4e6 293 and 298, 1.3e7 502 and 517: the
+// stores stream once the outputs fill the 256 MB Infinity Cache by themselves.
+constexpr long kStreamSamples = 6000000, kSmallBlockSamples = 3000000;
 template <bool STREAM>
 __global__ void __launch_bounds__(256) k_sample_scalars(SnapView sv, const double* S, long n, double a, double fbc,
                                                         double* out) {

@@ -56,3 +56,8 @@ def test_pitch_of_momenta_orthogonal_to_the_flow():
     assert 0 < (b == 0).sum() < 400
     want = np.where((b == 0) | (S[:, 5] == 0), np.arccos(np.cos(np.pi / 3)), np.where(S[:, 5] > 0, 0.0, np.pi))
     np.testing.assert_allclose(pitch, want, rtol=0, atol=4e-16)
+
+
+@pytest.mark.parametrize("n", [5999999, 6000000 + 65])
+def test_scalars_around_the_streamed_stores(n):
+    test_scalars_do_not_depend_on_the_launch(n)
