@@ -1280,10 +1280,10 @@ static hipError_t launch_bisect(double a, double inc, const double* dc, const do
   // is about 0.012 M wide on each side; up to 4096 two angles per wave (about
   // 0.005 M).  The prediction holds to 0.003 M up to |a| = 0.9; above, rays
   // near the prograde edge reach max_steps before they fall, and the result
-  // lies up to 0.013 M (0.97) or 0.03 M (0.998) outside it.  So from
+  // lies up to 0.013 M (0.97) or 0.03 M (0.998) outside it.  So above
   // |a| = 0.95 two waves per angle up to 1024 angles (0.98, i = 85 deg: 64
   // angles 2.0 against 3.8 ms, 1024 4.1 against 5.8; 0.95: 1024 angles 2.1 ms
-  // with one wave, 4.0 with two), and from |a| = 0.9 beyond 1024 the wide band
+  // with one wave, 4.0 with two), and above |a| = 0.9 beyond 1024 the wide band
   // in two rounds (4096 angles, 0.93, 85 deg: 6.0 against 7.7 ms; at 0.9, 60 deg
   // the narrow one 3.15 against 5.9).  Eight angles per block of four waves take
   // the same times, 16 per block of eight waves 4.2 ms narrow; 48 lanes per
@@ -1294,14 +1294,20 @@ static hipError_t launch_bisect(double a, double inc, const double* dc, const do
     if (err == hipSuccess) err = hipStreamSynchronize(st);  // h_rho may be freed after the return
     if (err != hipSuccess) return err;
     const double rEH = horizon(a);
+    const bool narrow = std::fabs(a) <= 0.9;
+    // The narrowed band's search starts at a width whose last level alone has more
+    // than B midpoints.  (From e itself, at 24 halvings, where 1e-5 M fits, its steps
+    // were too wide to find any: a = 0, i = 10 deg, 64 angles 4.3 ms, 1.6 from here.)
+    auto widest = [&](int B) { return std::min(e, 2.0 * B * 9.5 / std::ldexp(1.0, std::min(iters, kBandMaxLevels))); };
     if (n <= 1024 && std::fabs(a) <= 0.95)
-      k_bisect_band<64, 1><<<(unsigned)n, 64, 0, st>>>(a, ci, si, dist, dc, ds, n, max_steps, iters, rEH, e, true, dr);
+      k_bisect_band<64, 1><<<(unsigned)n, 64, 0, st>>>(a, ci, si, dist, dc, ds, n, max_steps, iters, rEH, widest(64),
+                                                       true, dr);
     else if (n <= 1024)
-      k_bisect_band<128, 1><<<(unsigned)n, 128, 0, st>>>(a, ci, si, dist, dc, ds, n, max_steps, iters, rEH, e, true,
-                                                         dr);
+      k_bisect_band<128, 1><<<(unsigned)n, 128, 0, st>>>(a, ci, si, dist, dc, ds, n, max_steps, iters, rEH,
+                                                         widest(128), true, dr);
     else
-      k_bisect_band<32, 2><<<(unsigned)((n + 1) / 2), 64, 0, st>>>(a, ci, si, dist, dc, ds, n, max_steps, iters, rEH, e,
-                                                                  std::fabs(a) <= 0.9, dr);
+      k_bisect_band<32, 2><<<(unsigned)((n + 1) / 2), 64, 0, st>>>(a, ci, si, dist, dc, ds, n, max_steps, iters, rEH,
+                                                                  narrow ? widest(32) : e, narrow, dr);
     return hipGetLastError();
   }
   // K halvings per round with 2^K lanes per angle: the fewest rounds with at

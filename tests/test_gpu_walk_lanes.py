@@ -127,3 +127,15 @@ def test_history_in_one_walk_is_complete_on_return():
     st.synchronize()
     rows = torch.arange(n) != 7
     assert torch.equal(rest[rows], s0.cpu()[rows]) and not D[:T.value].cpu()[:, rows].any()
+
+
+@pytest.mark.parametrize("spin,inc", [(0.0, 10.0), (0.5, 30.0), (0.97, 80.0)])
+@pytest.mark.parametrize("n", [1, 65, 1025])
+def test_bisection_to_small_errors(spin, inc, n, monkeypatch):
+    """More halvings than the band's width is first searched for."""
+    ang = np.arange(n) / n * 2 * np.pi + 0.1
+    for err, it in ((1e-6, 40), (1e-9, 40), (0.0, 20)):
+        got = ma.find_shadow_bisection_angles(spin, inc, ang, error_allowed=err, max_it=it)
+        with monkeypatch.context() as mp:
+            mp.setenv("MK_BISECT_BAND", "0")  # tree rounds
+            np.testing.assert_array_equal(got, ma.find_shadow_bisection_angles(spin, inc, ang, error_allowed=err, max_it=it))
