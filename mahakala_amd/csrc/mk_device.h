@@ -30,7 +30,9 @@ constexpr double kPI = 3.141592653589793;
 // FP64: division and square root on the geodesic right-hand side use the
 // hardware reciprocal / reciprocal square root refined by Newton and
 // Goldschmidt steps (within 2 ulp of IEEE; positive normal arguments only
-// there); the step rule, radius and camera keep IEEE operations.  FP32: hardware reciprocal,
+// there).  The step rule's quotient is the IEEE one (step_rule); its radius comes
+// from the same refined roots (ks_head), and the camera, the null normalisation and
+// a ray's first radius keep IEEE or library operations.  FP32: hardware reciprocal,
 // square root, exp2 and log2 (about 1 ulp).
 template <typename T> struct Math;
 template <> struct Math<double> {

@@ -390,7 +390,7 @@ __global__ void __launch_bounds__(128 * kPairTiles) k_render_pair(SnapView sv, R
   if (valid) img[p] = ok ? I : __builtin_nan("");
 }
 
-// ZONE: see tri_tile.
+// ZONE: see tri_geodesic.
 template <bool MIXED, bool ZONE>
 __global__ void __launch_bounds__(256, 4) k_render_tri(SnapView sv, RenderDev rp, double* __restrict__ img,
                                                        int32_t* __restrict__ steps) {
